@@ -421,28 +421,23 @@ int mdn_set_params(mdn_ctx* ctx, const double* kstr, const double* eql, const do
 /* ---- batched minimization ------------------------------------------------------------- */
 
 /* CGMethod::minimize (CGMethod.hpp:1746-1759) of n independent systems in one persistent kernel:
- * each workgroup pulls a system from a device queue and minimizes it to completion (same
- * semantics as mdn_minimize per system; only the rounding order of the block reductions
- * differs), then pulls the next. ctxs[i] must have its system uploaded and its neighbor lists
- * built, all on one device; ctxs[0] is the lead context (its stream runs the batch and it keeps
- * the tuned schedule). coords[i] (3 * n_beads of system i) is the start and receives the result
- * (coords[i] NULL: the start is the context's device coordinates, which receive the result, with
- * no coordinate transfer over the host link);
+ * every large system by a team of up to 32 workgroups of one XCD, the others by single workgroups
+ * that pull them from a device queue, largest first (same semantics as mdn_minimize per system;
+ * only the rounding order of the reductions differs, and it does not depend on the schedule).
+ * ctxs[i] must have its system uploaded and its neighbor lists built, all on one device; ctxs[0]
+ * is the lead context (its stream runs the batch). coords[i] (3 * n_beads of system i) is the
+ * start and receives the result (coords[i] NULL: the start is the context's device coordinates,
+ * which receive the result, with no coordinate transfer over the host link);
  * forces_out may be null, or forces_out[i] may be null; results[i] is filled for every system.
- * The schedule (workgroup size 128, 256, 512 or 1024 threads, given or largest-first order) is chosen on
- * the first call for a given (n, precision, total beads) by timing a complete run of each candidate
- * from the given coordinates.
  * Returns MDN_OK when every system succeeded, else the status of the first failing system (its
  * context's mdn_last_error and the lead's carry the message). No reference counterpart for the
  * batching itself: the reference minimizes one system per call. */
 int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* params,
                          double* const* coords, double* const* forces_out, mdn_min_result* results);
 
-/* The schedule of the last batched minimization on a lead context: out3 = [workgroup size,
- * largest-first order (1) or given order (0), tuned in that call (1) or reused (0)]; tune_ms (may
- * be null, MDN_BATCH_CANDIDATES values) = the tuning times in ms of the candidates 128 given,
- * 128 largest first, 256 given, 256 largest first, 512 given, 512 largest first, 1024 given,
- * 1024 largest first. */
+/* The schedule of batched minimizations: out3 = [workgroup size, largest-first order (1), tuned in
+ * that call (0)]. It is fixed by the systems' sizes, with nothing timed: tune_ms (may be null,
+ * MDN_BATCH_CANDIDATES values) is set to zero. */
 #define MDN_BATCH_CANDIDATES 8
 int mdn_last_batch_schedule(mdn_ctx* ctx, int32_t* out3, double* tune_ms);
 

@@ -6,7 +6,7 @@
 // slots hold R.
 //
 // Layout in HBM (all device buffers owned by the context):
-//   x[2][3*n_beads] (current / next coordinates), F, F_prev, d[2] (search direction, current
+//   x[2][3*n_beads] (current / next coordinates), F[2] (current / next), d[2] (search direction, current
 //   / next), x_min[2] (minimum-energy backup, committed / candidate): the reference's flat AoS
 //   coord vectors (DofSerializer.hpp:64-187), double.
 //   Term tables: structure of arrays per force field (bead indices int32, parameters double).
@@ -681,14 +681,13 @@ __global__ void __launch_bounds__(BLOCK) k_dof_gather(int n, const int* __restri
 }
 
 // Slots of every interaction at x (ForceFieldManager::computeForces before the gather).
-// Excluded-volume pairs needing the numerical fallback are listed in bad_list.
+// Excluded-volume pairs needing the numerical fallback are listed in bad_list (null: counted only).
 // Grid: the interaction blocks. The mixed instantiation is held to 4 waves per SIMD (126 VGPRs,
 // no spills; measured 1-2 % faster per evaluation at 42,000 and 420,000 beads), the FP64 one
 // keeps 3 (at 4 it spills and was slower at 42,000 beads).
 template <typename R>
-__global__ void __launch_bounds__(BLOCK, sizeof(R) == 4 ? 4 : 1) k_forces_terms(DevSys s, const double* __restrict__ x,
-                                                        R* __restrict__ slots, int* bad_count, int* bad_list,
-                                                        int bead0, int bmask, const double* __restrict__ base) {
+__device__ inline void terms_block(const DevSys& s, const double* __restrict__ x, R* __restrict__ slots, int* bad_count,
+                                   int* bad_list, int bead0, int bmask, const double* __restrict__ base) {
     // blocks from bead0 on (when bead0 >= 0) are bead blocks: the bonded sums (bead_bonded_sum)
     if (bead0 >= 0 && (int)blockIdx.x >= bead0) {
         bead_bonded_sum<R>(s, x, blockIdx.x - bead0, bmask, base);
@@ -703,8 +702,14 @@ __global__ void __launch_bounds__(BLOCK, sizeof(R) == 4 ? 4 : 1) k_forces_terms(
     (void)term_ef<R>(s, ff, t, p, slots, -1, &fbad, &bad_t);   // forces only: the energy half is dead code
     if (fbad) {
         const int k = atomicAdd(bad_count, 1);
-        bad_list[k] = bad_t;
+        if (bad_list) bad_list[k] = bad_t;
     }
+}
+template <typename R>
+__global__ void __launch_bounds__(BLOCK, sizeof(R) == 4 ? 4 : 1) k_forces_terms(DevSys s, const double* __restrict__ x,
+                                                        R* __restrict__ slots, int* bad_count, int* bad_list,
+                                                        int bead0, int bmask, const double* __restrict__ base) {
+    terms_block<R>(s, x, slots, bad_count, bad_list, bead0, bmask, base);
 }
 
 // force[b] = base[b] + the bonded pieces selected by bmask + b's slots with id in [lo, hi)
@@ -749,9 +754,10 @@ __global__ void __launch_bounds__(BLOCK) k_gather_tangents(DevSys s, const doubl
 // Returns the number of deferred pairs (DEFER_CAP exceeded when larger). The count is read and
 // reset with atomics: in the batched minimizer the pairs were pushed by other waves of the same
 // workgroup within the kernel.
-// run_defers_n: the same with the count n already read (by every thread).
+// run_defers_eval: the energies alone (into each entry's U); defer_sums: the sums by one thread;
+// run_defers_n: both and the reset, with the count n already read (by every thread).
 template <int NTH = BLOCK>
-__device__ inline int run_defers_n(const DevSys& s, int n, double* lds, double* sum, int* badc, int ncode) {
+__device__ inline void run_defers_eval(const DevSys& s, int n, double* lds) {
     const int m = min(n, DEFER_CAP);
     const int op1[1] = {0};
     for (int k = 0; k < m; k++) {
@@ -762,23 +768,30 @@ __device__ inline int run_defers_n(const DevSys& s, int n, double* lds, double* 
         block_reduce_n<1, NTH>(&r, op1, lds);
         if (threadIdx.x == 0) e.U = exvol_energyN_finish(c1, c2, c3, c4, e.ks, r);
     }
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < ncode; c++) {
-            sum[c] = 0.0;
-            badc[c] = 0;
-            int last_t = -1;
-            for (;;) {
-                int best = -1;
-                for (int k = 0; k < m; k++)
-                    if (s.defer[k].code == c && s.defer[k].t > last_t && (best < 0 || s.defer[k].t < s.defer[best].t))
-                        best = k;
-                if (best < 0) break;
-                const double U = s.defer[best].U;
-                if (energy_bad(U)) badc[c] = 1;
-                else sum[c] += U;
-                last_t = s.defer[best].t;
-            }
+}
+__device__ inline void defer_sums(const DevSys& s, int m, double* sum, int* badc, int ncode) {
+    for (int c = 0; c < ncode; c++) {
+        sum[c] = 0.0;
+        badc[c] = 0;
+        int last_t = -1;
+        for (;;) {
+            int best = -1;
+            for (int k = 0; k < m; k++)
+                if (s.defer[k].code == c && s.defer[k].t > last_t && (best < 0 || s.defer[k].t < s.defer[best].t))
+                    best = k;
+            if (best < 0) break;
+            const double U = s.defer[best].U;
+            if (energy_bad(U)) badc[c] = 1;
+            else sum[c] += U;
+            last_t = s.defer[best].t;
         }
+    }
+}
+template <int NTH = BLOCK>
+__device__ inline int run_defers_n(const DevSys& s, int n, double* lds, double* sum, int* badc, int ncode) {
+    run_defers_eval<NTH>(s, n, lds);
+    if (threadIdx.x == 0) {
+        defer_sums(s, min(n, DEFER_CAP), sum, badc, ncode);
         __hip_atomic_store(s.defer_n, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     return n;
@@ -856,9 +869,8 @@ __global__ void __launch_bounds__(BLOCK) k_vec_stats_fin(const double* __restric
 
 // Per-FF energies at x, block partials. Grid: interaction blocks only.
 template <typename R>
-__global__ void __launch_bounds__(BLOCK) k_energy_report(DevSys s, const double* __restrict__ x,
-                                                         double* __restrict__ partial) {
-    __shared__ double lds[BLOCK / 64];
+__device__ inline void energy_block(const DevSys& s, const double* __restrict__ x, double* __restrict__ partial,
+                                    double* lds) {
     const int ff = ff_of_block(s, blockIdx.x);
     double v = 0.0;
     if (ff < NFF) {
@@ -871,13 +883,18 @@ __global__ void __launch_bounds__(BLOCK) k_energy_report(DevSys s, const double*
     block_reduce_n<1>(&v, op1, lds);
     if (threadIdx.x == 0) partial[PSTRIDE * blockIdx.x] = v;
 }
+template <typename R>
+__global__ void __launch_bounds__(BLOCK) k_energy_report(DevSys s, const double* __restrict__ x,
+                                                         double* __restrict__ partial) {
+    __shared__ double lds[BLOCK / 64];
+    energy_block<R>(s, x, partial, lds);
+}
 
 // out[0..5] per force field (excluded volume = -1 on the sentinel), out[6] =
 // computeIndividualEnergies total (plain sum), out[7] = computeEnergy total (+inf on a sentinel),
 // out[8] = deferred Simpson pairs beyond capacity. One block.
-__global__ void __launch_bounds__(BLOCK) k_energy_report_fin(DevSys s, const double* __restrict__ partial,
-                                                             double* __restrict__ out) {
-    __shared__ double lds[NFF * (BLOCK / 64)];
+__device__ inline void energy_fin(const DevSys& s, const double* __restrict__ partial, double* __restrict__ out,
+                                  double* lds) {
     double acc[NFF];
     int opn[NFF];
 #pragma unroll
@@ -908,6 +925,11 @@ __global__ void __launch_bounds__(BLOCK) k_energy_report_fin(DevSys s, const dou
         out[7] = failed ? INFINITY : tot_s;
         out[8] = n > DEFER_CAP ? (double)n : 0.0;
     }
+}
+__global__ void __launch_bounds__(BLOCK) k_energy_report_fin(DevSys s, const double* __restrict__ partial,
+                                                             double* __restrict__ out) {
+    __shared__ double lds[NFF * (BLOCK / 64)];
+    energy_fin(s, partial, out, lds);
 }
 
 // Numerical excluded-volume force fallback (forceN, CylinderExclVolRepulsion.cpp:984-1254)
@@ -1032,7 +1054,6 @@ struct CgBufs {
     double* d[2];       // current / next search direction (dpar)
     double* xmin[2];    // committed / candidate minimum-energy backup (bkpar)
     double* f[2];       // current / next force (fpar)
-    double* fp;         // previous force (the batched minimizer's; here F_prev is f[fpar])
     double* xh;         // x + (lambda / 2) d, the second trial of a launch after a rejection
     void* slots;        // 3 values of the evaluation's arithmetic type per slot
     double* partial;    // line-search partials, value-major: [value][interaction blocks + bead blocks]

@@ -18,7 +18,7 @@
 
 #include "../../include/mdn_mech.h"
 #include "mdn_kernels.h"
-#include "mdn_batched.h"
+#include "mdn_team.h"
 
 using namespace mdn;
 
@@ -70,6 +70,11 @@ struct DBuf {
         n = 0;
     }
 };
+
+// The CG state and, from TEAM_CTL_OFF on, the persistent minimizer's barrier: uploaded together.
+constexpr size_t TEAM_CTL_OFF = 1024, CG_BYTES = TEAM_CTL_OFF + sizeof(TeamCtl);
+static_assert(sizeof(CgState) <= TEAM_CTL_OFF, "the barrier follows the state");
+TeamCtl* team_ctl(CgState* cg) { return reinterpret_cast<TeamCtl*>(reinterpret_cast<char*>(cg) + TEAM_CTL_OFF); }
 
 struct HipErr {
     hipError_t e;
@@ -135,7 +140,7 @@ struct mdn_ctx {
     std::vector<int> bnd_nneighbors;
 
     // state vectors
-    DBuf<double> x[2], f, f2, fp, xh, d[2], xmin[2], scratch_f, ext;   // f, f2: the CG force pair
+    DBuf<double> x[2], f, f2, xh, d[2], xmin[2], scratch_f, ext;   // f, f2: the CG force pair
     DBuf<double> slots;   // 3 values per slot; the mixed path uses the first half as float
     DBuf<double> partial;
     DBuf<int> bad_count, bad_list;
@@ -154,15 +159,18 @@ struct mdn_ctx {
     DevSys sys{};
     int cur = 0;   // which x buffer holds the current coordinates
 
+    DBuf<double> team_part;   // wavefront partials of the persistent minimizer
+    int team_size = -1;       // workgroups of the persistent minimizer: -1 by size, 0 never (MDN_CG_TEAM)
     // batched minimizer (the lead context of a batch owns these)
+    DBuf<TeamSlot> batch_slot;
+    DBuf<TeamInfo> batch_team;
+    DBuf<TeamCtl> batch_ctl;
     DBuf<BatchItem> batch_items;
     DBuf<CgState> batch_states;   // the batch's final states and reports, gathered for one read-back
     DBuf<double> batch_reports;
     DBuf<int> batch_order, batch_queue;
     DBuf<BatchCopy> batch_copy;   // [start copies | start backups | restores], one per system each
-    long batch_key = -1;          // (systems, precision, beads) of the tuned schedule
-    int batch_nt = 256, batch_sorted = 1, batch_tuned = 0;
-    double batch_tune_ms[MDN_BATCH_CANDIDATES] = {};
+    int batch_nt = TEAM_NT;
 
     bool use_graph = true;   // replay the CG slots as a captured hipGraph (MDN_CG_GRAPH=0: launch them directly)
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};   // per precision (MDN_PREC_*)
@@ -317,6 +325,9 @@ int ensure_eval_buffers(mdn_ctx* ctx) {
     // blocks; this also covers the evaluation partials), then the CG gather's
     const long nls = (long)s.lsp;
     HIPCHK(ctx->partial.ensure((size_t)(nls + gather_blocks(ctx) + 1) * PSTRIDE));
+    // the persistent minimizer's partials, for a network minimized alone or in a batch
+    if (ctx->n_beads < GB_LARGE_BEADS)
+        HIPCHK(ctx->team_part.ensure((size_t)std::max(team_wpart_doubles(s, SUM_SLOTS), team_wpart_doubles(s, SUM_STRIDED))));
     HIPCHK(ctx->pos.ensure((size_t)std::max(1L, s.slot0[NFF])));
     HIPCHK(ctx->sorted_id.ensure((size_t)std::max(1L, s.slot0[NFF])));
     HIPCHK(ctx->bad_list.ensure((size_t)std::max(1, s.n[FF_EXVOL])));
@@ -496,6 +507,10 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     // instead of replaying a captured graph (the same kernels and decisions; for tools that do
     // not follow graph launches)
     if (const char* env = getenv("MDN_CG_GRAPH")) ctx->use_graph = atoi(env) != 0;
+    // MDN_CG_TEAM at context creation: 0 = always the four-kernel slots, n = a team of n
+    // workgroups of one XCD for every network; unset: by the network's size (team_workgroups)
+    // (the result does not depend on it)
+    if (const char* env = getenv("MDN_CG_TEAM")) ctx->team_size = std::max(0, std::min(TEAM_MAX, atoi(env)));
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
         return MDN_ERR_HIP;
@@ -505,7 +520,7 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
         delete ctx;
         return MDN_ERR_HIP;
     }
-    if (hipHostMalloc(&ctx->h_cg, sizeof(CgState)) != hipSuccess ||
+    if (hipHostMalloc(&ctx->h_cg, CG_BYTES) != hipSuccess ||
         hipHostMalloc(&ctx->h_eout, sizeof(double) * 32) != hipSuccess ||
         hipHostMalloc(&ctx->h_int, sizeof(int) * 16) != hipSuccess) {
         delete ctx;
@@ -513,7 +528,7 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     }
     if (ctx->ticket.ensure(8) != hipSuccess || ctx->eout.ensure(32) != hipSuccess ||
         ctx->vstat.ensure(2 * VSTAT_BLOCKS) != hipSuccess ||
-        ctx->bad_count.ensure(1) != hipSuccess || ctx->cg.ensure(1) != hipSuccess ||
+        ctx->bad_count.ensure(1) != hipSuccess || ctx->cg.ensure(CG_BYTES / sizeof(CgState) + 1) != hipSuccess ||
         ctx->nl_err.ensure(1) != hipSuccess || ctx->defer.ensure(DEFER_CAP) != hipSuccess ||
         ctx->defer_n.ensure(1) != hipSuccess) {
         delete ctx;
@@ -556,7 +571,7 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
                           &ctx->lnk_p1, &ctx->lnk_p2, &ctx->lnk_sf, &ctx->mot_k, &ctx->mot_eql, &ctx->mot_p1,
                           &ctx->mot_p2, &ctx->mot_sf, &ctx->ev_ks, &ctx->bnd_krep, &ctx->bnd_slen,
                           &ctx->d_cyl_kexvol, &ctx->d_cyl_eql, &ctx->d_krep_e, &ctx->d_slen_e, &ctx->mid,
-                          &ctx->x[0], &ctx->x[1], &ctx->f, &ctx->f2, &ctx->fp, &ctx->xh, &ctx->d[0], &ctx->d[1],
+                          &ctx->x[0], &ctx->x[1], &ctx->f, &ctx->f2, &ctx->xh, &ctx->d[0], &ctx->d[1],
                           &ctx->xmin[0], &ctx->xmin[1], &ctx->scratch_f, &ctx->ext, &ctx->partial, &ctx->eout,
                           &ctx->vstat, &ctx->fallback_partial, &ctx->dof_next, &ctx->dof_new};
     for (auto* b : db) b->release();
@@ -581,6 +596,10 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
     ctx->ticket.release();
     ctx->defer.release();
     ctx->defer_n.release();
+    ctx->team_part.release();
+    ctx->batch_slot.release();
+    ctx->batch_team.release();
+    ctx->batch_ctl.release();
     ctx->batch_items.release();
     ctx->batch_states.release();
     ctx->batch_reports.release();
@@ -855,7 +874,7 @@ int mdn_system_upload(mdn_ctx* ctx, const mdn_system_desc* d, const double* coor
     }
     // state vectors
     size_t nv = 3 * (size_t)ctx->n_beads;
-    for (auto* b : {&ctx->x[0], &ctx->x[1], &ctx->f, &ctx->f2, &ctx->fp, &ctx->xh, &ctx->d[0], &ctx->d[1],
+    for (auto* b : {&ctx->x[0], &ctx->x[1], &ctx->f, &ctx->f2, &ctx->xh, &ctx->d[0], &ctx->d[1],
                     &ctx->xmin[0], &ctx->xmin[1], &ctx->scratch_f, &ctx->ext})
         HIPCHK(b->ensure(nv));
     ctx->cur = 0;
@@ -1714,7 +1733,7 @@ static CgBufs cg_bufs(mdn_ctx* ctx) {
     B.x[0] = ctx->x[0].p; B.x[1] = ctx->x[1].p;
     B.d[0] = ctx->d[0].p; B.d[1] = ctx->d[1].p;
     B.xmin[0] = ctx->xmin[0].p; B.xmin[1] = ctx->xmin[1].p;
-    B.f[0] = ctx->f.p; B.f[1] = ctx->f2.p; B.fp = ctx->fp.p; B.xh = ctx->xh.p;
+    B.f[0] = ctx->f.p; B.f[1] = ctx->f2.p; B.xh = ctx->xh.p;
     B.slots = (void*)ctx->slots.p; B.partial = ctx->partial.p; B.bad_count = ctx->bad_count.p;
     B.gpartial = ctx->partial.p + (long)PSTRIDE * ls_blocks(ctx);   // after the line-search partials
     return B;
@@ -1777,6 +1796,52 @@ static int cg_graph(mdn_ctx* ctx, int prec) {
     return MDN_OK;
 }
 
+// The work of a network in the persistent minimizer, in beads: an excluded-volume pair costs what
+// about eight beads do.
+static long team_cost(const DevSys& s) {
+    return s.n_beads + s.n[FF_LINKER] + s.n[FF_MOTOR] + 8L * s.n[FF_EXVOL] + s.n[FF_BOUNDARY];
+}
+// Work per workgroup below which another workgroup does not pay: batches of 8, 16 and 48 networks
+// of up to 12,000 beads take 2.3, 2.6 and 4.4 ms with 256, 2.8, 3.0 and 4.7 ms with 1024, 3.5, 3.8
+// and 5.7 ms with 2048.
+static const long TEAM_SHARE = 256;
+// A single network's team: 16 workgroups at most (32 are 5 to 10 % slower below TEAM_WIDE, where
+// their dearer barriers count more than the work they share: 1,300 beads in a cube 1.74 against
+// 1.92 ms per 80 iterations), 32 from there to TEAM_COST_MAX (8,400 beads in a sphere, work 36,000:
+// 2.10 against 2.34 ms), and from there on the four-kernel slots over the whole chip (10,500 beads
+// in a sphere, work 43,000: 2.30 ms against 2.38 ms with 32 workgroups; 3,100 in a cube, work
+// 40,000: 2.35 against 2.27 ms; 550 beads: 2.14 against 1.55 ms).
+static const long TEAM_WIDE = 33000, TEAM_COST_MAX = 41000;
+// Workgroups of the persistent minimizer for a single network; 0: the four-kernel slots.
+static int team_workgroups(const mdn_ctx* ctx) {
+    if (!cg_bonded_sums(ctx, 0) || ctx->n_beads >= GB_LARGE_BEADS) return 0;
+    if (ctx->team_size >= 0) return ctx->team_size;
+    const long c = team_cost(ctx->sys);
+    return c > TEAM_COST_MAX ? 0 : c > TEAM_WIDE ? TEAM_MAX : (int)std::min<long>(16, (c + TEAM_SHARE - 1) / TEAM_SHARE);
+}
+
+// The persistent minimizer on one system from its device state until that is done. The barrier's
+// words at team_ctl(cg) are zero.
+static int launch_team(mdn_ctx* ctx, int prec, int size) {
+    DevSys s = cg_sys(ctx, prec);
+    CgBufs B = cg_bufs(ctx);
+    CgState* st = ctx->cg.p;
+    TeamCtl* ctl = team_ctl(st);
+    double* wp = ctx->team_part.p;
+    int stride = size > 1 ? 8 : 1;
+    void* args[] = {&s, &B, &st, &ctl, &wp, &size, &stride};
+    const dim3 g(stride * (size - 1) + 1), b(TEAM_NT);
+    auto launch = [&](auto k) {
+        // the workgroups of a team wait for each other: a cooperative launch has them all resident
+        if (size > 1) return hipLaunchCooperativeKernel(k, g, b, args, 0, ctx->stream);
+        hipLaunchKernelGGL(k, g, b, 0, ctx->stream, s, B, st, ctl, wp, size, stride);
+        return hipGetLastError();
+    };
+    if (prec == MDN_PREC_MIXED) HIPCHK(launch(k_cg_team_one<float, TEAM_NT>));
+    else HIPCHK(launch(k_cg_team_one<double, TEAM_NT>));
+    return MDN_OK;
+}
+
 int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* force_out, mdn_min_result* res) {
     int st = need_system(ctx, true);
     if (st) return st;
@@ -1818,7 +1883,7 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     HIPCHK(hipStreamSynchronize(ctx->stream));
     const double ff = ctx->h_eout[16], mx = ctx->h_eout[17];
     CgState& S = *ctx->h_cg;
-    memset(&S, 0, sizeof(S));
+    memset((void*)ctx->h_cg, 0, CG_BYTES);
     S.method = p->method;
     S.ls_algo = p->line_search;
     S.try_recover = p->try_recover;
@@ -1850,12 +1915,13 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     const bool limit0 = (S.force_call_limit != 0 && S.num_force_call > S.force_call_limit);
     S.done = (S.grad_inf_norm < S.grad_tol || S.energy_rel_change < S.energy_rel_tol || limit0) ? 1 : 0;
     HIPCHK(hipMemsetAsync(ctx->d[0].p, 0, sizeof(double) * nv, ctx->stream));   // searchDir.assign(numDof, 0)
-    HIPCHK(hipMemcpyAsync(ctx->cg.p, &S, sizeof(CgState), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->cg.p, &S, CG_BYTES, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
+    const int team = team_workgroups(ctx);
     // The slots are captured into a graph once a layout is minimized a second time: a graph made
     // for one minimization (a layout that the next neighbor-list rebuild replaces) costs more to
     // instantiate than its replays save over launching the same kernels directly.
-    const bool graph = ctx->use_graph && (ctx->graph_gen[prec] == ctx->sys_gen || ctx->min_gen[prec] == ctx->sys_gen);
+    const bool graph = !team && ctx->use_graph && (ctx->graph_gen[prec] == ctx->sys_gen || ctx->min_gen[prec] == ctx->sys_gen);
     ctx->min_gen[prec] = ctx->sys_gen;
     if (graph && (st = cg_graph(ctx, prec))) return st;
     const DevSys slot_sys = cg_sys(ctx, prec);
@@ -1875,6 +1941,11 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
         h_done[0] = h_done[1] = 0;
         int k = 0;
         long here = 0;
+        if (team && !done) {
+            if (n_forcen) HIPCHK(hipMemsetAsync(team_ctl(ctx->cg.p), 0, sizeof(TeamCtl), ctx->stream));
+            if ((st = launch_team(ctx, prec, team))) return st;
+            done = true;
+        }
         while (!done && launched < max_batches) {
             if (graph) {
                 HIPCHK(hipGraphLaunch(ctx->graph_exec[prec], ctx->stream));
@@ -1895,7 +1966,8 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
             }
             k ^= 1;
         }
-        HIPCHK(d2h(ctx, &S, ctx->cg.p, sizeof(CgState)));
+        HIPCHK(d2h(ctx, ctx->h_cg, ctx->cg.p, CG_BYTES));
+        if (team_ctl(ctx->h_cg)->failed) return fail(ctx, MDN_ERR_STATE, "a workgroup of the minimizer gave up waiting for the others");
         if (!(S.done && S.status == ST_NEED_FORCEN)) break;
         // The step's forces need the numerical excluded-volume fallback (forceN,
         // CylinderExclVolRepulsion.cpp:984-1254): recompute them at the new coordinates with it
@@ -1989,36 +2061,77 @@ static void fill_result(const CgState& S, const double* rep_before, const double
     res->restored_min_energy = S.reserved[0];
 }
 
-template <typename R, int NT>
-static int launch_batched(mdn_ctx* L, int n, const BatchParams& P) {
-    auto kern = k_cg_batched<R, NT>;
-    int per_cu = 0, n_cu = 0;
-    HIPCHK_CTX(L, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, NT, 0));
-    HIPCHK_CTX(L, hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, L->device));
-    int grid = std::max(1, std::min(n, std::max(1, per_cu) * std::max(1, n_cu)));
-    // MDN_BATCH_MAX_WORKGROUPS caps the persistent grid, so that every workgroup pulls several
-    // systems from the queue (the schedule a batch larger than the resident workgroups runs)
-    if (const char* env = getenv("MDN_BATCH_MAX_WORKGROUPS"))
-        if (atoi(env) > 0) grid = std::min(grid, atoi(env));
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, L->stream, L->batch_queue.p, 0);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, L->stream, (const BatchItem*)L->batch_items.p,
-                       (const int*)L->batch_order.p, n, L->batch_queue.p, P);
-    HIPCHK_CTX(L, hipGetLastError());
-    return MDN_OK;
-}
-
-template <typename R>
-static int run_batched_t(mdn_ctx* L, int n, const BatchParams& P, int nt) {
-    switch (nt) {
-    case 128: return launch_batched<R, 128>(L, n, P);
-    case 512: return launch_batched<R, 512>(L, n, P);
-    case 1024: return launch_batched<R, 1024>(L, n, P);
-    default: return launch_batched<R, 256>(L, n, P);
+// A batch's workgroups: which team each is in, and which system each team has. Large systems get
+// teams of their own, sized to their share of the work; the others are pulled from a queue,
+// largest first, by single workgroups. A workgroup b runs on XCD b % 8, and a team's workgroups
+// are taken from one XCD.
+struct TeamPlan {
+    std::vector<TeamSlot> slot;
+    std::vector<TeamInfo> team;
+    std::vector<int> order;   // the queue
+    bool wait = false;        // some team has more than one workgroup
+};
+static TeamPlan plan_teams(const std::vector<long>& cost, int groups) {
+    const int n = (int)cost.size(), NX = 8;
+    TeamPlan P;
+    std::vector<int> room(NX, 0);
+    for (int b = 0; b < groups; b++) room[b % NX]++;
+    long total = 0;
+    for (long c : cost) total += c;
+    std::vector<int> k(n, 1), by(n);
+    for (int i = 0; i < n; i++) by[i] = i;
+    std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    // the share of work per workgroup, raised until the teams and the queue's workgroups fit
+    for (double share = std::max<double>(TEAM_SHARE, (double)total / groups);; share *= 1.1) {
+        int used = 0, small = 0;
+        double rest = 0;
+        for (int i = 0; i < n; i++) {
+            k[i] = (int)std::max(1.0, std::min<double>(std::min(TEAM_MAX, room[0]), std::ceil(cost[i] / share)));
+            if (k[i] > 1) used += k[i];
+            else { small++; rest += cost[i]; }
+        }
+        if (used + std::min<double>(small, std::ceil(rest / share)) <= groups) break;
     }
+    P.slot.assign(groups, TeamSlot{-1, 0});
+    std::vector<int> taken(NX, 0);
+    auto place = [&](int want, int sys) {   // a team of `want` workgroups on the XCD with the most room
+        int x = 0;
+        for (int q = 1; q < NX; q++)
+            if (room[q] - taken[q] > room[x] - taken[x]) x = q;
+        const int size = std::min(want, room[x] - taken[x]);
+        if (size <= 0) return false;
+        for (int m = 0; m < size; m++) P.slot[x + NX * (taken[x] + m)] = TeamSlot{(int)P.team.size(), m};
+        taken[x] += size;
+        P.team.push_back(TeamInfo{size, sys});
+        P.wait = P.wait || size > 1;
+        return true;
+    };
+    for (int i : by)
+        if (k[i] == 1 || !place(k[i], i)) P.order.push_back(i);
+    for (size_t j = 0; j < P.order.size(); j++)
+        if (!place(1, -1)) break;
+    return P;
 }
 
-static int run_batched(mdn_ctx* L, int n, const BatchParams& P, int prec, int nt) {
-    return prec == MDN_PREC_MIXED ? run_batched_t<float>(L, n, P, nt) : run_batched_t<double>(L, n, P, nt);
+// The persistent kernel of a planned batch.
+static int launch_batch(mdn_ctx* L, const TeamPlan& P, int prec) {
+    const BatchItem* items = L->batch_items.p;
+    const TeamSlot* slot = L->batch_slot.p;
+    const TeamInfo* team = L->batch_team.p;
+    TeamCtl* ctl = L->batch_ctl.p;
+    const int* order = L->batch_order.p;
+    int n = (int)P.order.size();
+    int* queue = L->batch_queue.p;
+    void* args[] = {&items, &slot, &team, &ctl, &order, &n, &queue};
+    const dim3 g(P.slot.size()), b(TEAM_NT);
+    auto launch = [&](auto k) {
+        if (P.wait) return hipLaunchCooperativeKernel(k, g, b, args, 0, L->stream);
+        hipLaunchKernelGGL(k, g, b, 0, L->stream, items, slot, team, ctl, order, n, queue);
+        return hipGetLastError();
+    };
+    if (prec == MDN_PREC_MIXED) HIPCHK_CTX(L, launch(k_cg_team<float, TEAM_NT>));
+    else HIPCHK_CTX(L, launch(k_cg_team<double, TEAM_NT>));
+    return MDN_OK;
 }
 
 extern "C" {
@@ -2048,30 +2161,34 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     // every context's own work is complete before the lead stream reads its buffers
     for (int i = 1; i < n; i++) HIPCHK_CTX(L, hipStreamSynchronize(ctxs[i]->stream));
     std::vector<BatchItem> items(n);
-    std::vector<long> size(n);
-    // device-to-device copies in three sets of n (a zero count copies nothing), each set one launch:
-    // the systems that start from their device coordinates (x[cur] -> x[0]), the start's backup for
-    // the schedule tuning runs (x[0] -> ext) and its restore before each of them (ext -> x[0])
-    std::vector<BatchCopy> copies(3 * (size_t)n);
+    std::vector<long> cost(n);
+    // the systems that start from their device coordinates: x[cur] -> x[0], all in one launch (a
+    // zero count copies nothing)
+    std::vector<BatchCopy> copies((size_t)n);
     long max_nv = 1;
+    int max_blk = 1, max_nbb = 1, max_terms = 1;
     for (int i = 0; i < n; i++) {
         mdn_ctx* c = ctxs[i];
         const long nv = 3L * c->n_beads;
-        const size_t bytes = sizeof(double) * nv;
         max_nv = std::max(max_nv, nv);
         if (coords[i])
-            HIPCHK_CTX(L, hipMemcpyAsync(c->x[0].p, coords[i], bytes, hipMemcpyHostToDevice, L->stream));
+            HIPCHK_CTX(L, hipMemcpyAsync(c->x[0].p, coords[i], sizeof(double) * nv, hipMemcpyHostToDevice, L->stream));
         else if (c->cur != 0)   // the context's device coordinates
             copies[i] = BatchCopy{c->x[c->cur].p, c->x[0].p, nv};
         c->cur = 0;
-        copies[n + i] = BatchCopy{c->x[0].p, c->ext.p, nv};
-        copies[2L * n + i] = BatchCopy{c->ext.p, c->x[0].p, nv};
-        items[i].s = c->sys;
-        items[i].B = cg_bufs(c);
-        items[i].st = c->cg.p;
-        items[i].report = c->eout.p;
-        size[i] = c->n_beads;
-        for (int ff = 0; ff < NFF; ff++) size[i] += c->sys.n[ff];
+        BatchItem& it = items[i];
+        it.s = c->sys;
+        it.s.bonded_gather = 1;
+        it.s.bead_energy = 1;   // the filament terms' energies with their forces, by the bead blocks
+        it.B = cg_bufs(c);
+        it.st = c->cg.p;
+        it.report = c->eout.p;
+        HIPCHK_CTX(L, c->team_part.ensure((size_t)team_wpart_doubles(it.s, SUM_STRIDED)));   // large systems
+        it.wpart = c->team_part.p;
+        cost[i] = team_cost(it.s);
+        max_blk = std::max(max_blk, it.s.blk[NFF]);
+        max_nbb = std::max(max_nbb, it.s.nbb);
+        max_terms = std::max(max_terms, it.s.blk_nb + it.s.nbb);
     }
     BatchParams P{};
     P.method = p->method;
@@ -2080,74 +2197,74 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     P.force_call_limit = p->force_call_limit;
     P.energy_call_limit = p->energy_call_limit;
     P.report_on_call_limit = p->report_on_call_limit;
-    P.limit_override = 0;
     P.max_dist = p->max_dist;
     P.lambda_max = p->lambda_max;
     P.grad_tol = p->grad_tol;
     P.energy_rel_tol = p->energy_rel_tol;
+    // one workgroup per CU (12 wavefronts at 168 VGPRs fill it); MDN_BATCH_MAX_WORKGROUPS caps
+    // them, so that every workgroup pulls several systems (what a batch larger than the chip does)
+    int n_cu = 0;
+    HIPCHK_CTX(L, hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, L->device));
+    int groups = std::max(1, n_cu);
+    if (const char* env = getenv("MDN_BATCH_MAX_WORKGROUPS"))
+        if (atoi(env) > 0) groups = std::min(groups, atoi(env));
+    const TeamPlan plan = plan_teams(cost, groups);
+    const size_t nq = std::max<size_t>(1, plan.order.size());
     HIPCHK_CTX(L, L->batch_items.ensure(n));
-    HIPCHK_CTX(L, L->batch_order.ensure(n));
+    HIPCHK_CTX(L, L->batch_order.ensure(nq));
     HIPCHK_CTX(L, L->batch_queue.ensure(1));
-    HIPCHK_CTX(L, L->batch_copy.ensure(3 * (size_t)n));
+    HIPCHK_CTX(L, L->batch_copy.ensure((size_t)n));
+    HIPCHK_CTX(L, L->batch_slot.ensure(plan.slot.size()));
+    HIPCHK_CTX(L, L->batch_team.ensure(plan.team.size()));
+    HIPCHK_CTX(L, L->batch_ctl.ensure(plan.team.size()));
     HIPCHK_CTX(L, hipMemcpyAsync(L->batch_items.p, items.data(), sizeof(BatchItem) * n, hipMemcpyHostToDevice,
                                  L->stream));
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * 3 * n, hipMemcpyHostToDevice,
+    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * n, hipMemcpyHostToDevice,
                                  L->stream));
+    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_slot.p, plan.slot.data(), sizeof(TeamSlot) * plan.slot.size(),
+                                 hipMemcpyHostToDevice, L->stream));
+    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_team.p, plan.team.data(), sizeof(TeamInfo) * plan.team.size(),
+                                 hipMemcpyHostToDevice, L->stream));
+    if (!plan.order.empty())
+        HIPCHK_CTX(L, hipMemcpyAsync(L->batch_order.p, plan.order.data(), sizeof(int) * plan.order.size(),
+                                     hipMemcpyHostToDevice, L->stream));
+    HIPCHK_CTX(L, hipMemsetAsync(L->batch_ctl.p, 0, sizeof(TeamCtl) * plan.team.size(), L->stream));
+    HIPCHK_CTX(L, hipMemsetAsync(L->batch_queue.p, 0, sizeof(int), L->stream));
+    const BatchItem* di = L->batch_items.p;
     const dim3 cgrid((unsigned)std::min(64L, std::max(1L, (long)ceil_div(max_nv, 256L))), (unsigned)std::min(n, 4096));
-    auto copy_set = [&](int set) {   // set 0: start copies, 1: backups, 2: restores
-        hipLaunchKernelGGL(k_batch_copy, cgrid, dim3(256), 0, L->stream,
-                           (const BatchCopy*)(L->batch_copy.p + (size_t)set * n), n);
-        return hipGetLastError();
-    };
-    HIPCHK_CTX(L, copy_set(0));
-    std::vector<int> order_given(n), order_sorted(n);
-    for (int i = 0; i < n; i++) order_given[i] = order_sorted[i] = i;
-    std::stable_sort(order_sorted.begin(), order_sorted.end(), [&](int a, int b) { return size[a] > size[b]; });
     int st;
-    // schedule: workgroup size (128, 256, 512, 1024) x system order (given, largest first), chosen once
-    // per (systems, precision, beads) by timing each candidate on this batch, run to completion
-    // from the caller's coordinates: the batch time is set by its slowest systems, whose iteration
-    // counts only a complete run shows (a short run measures the start-up instead)
-    const long key = ((long)n * 2 + p->precision) * 1000003L + beads;
-    if (L->batch_key != key) {
-        const BatchParams T = P;
-        hipEvent_t e0, e1;
-        HIPCHK_CTX(L, hipEventCreate(&e0));
-        HIPCHK_CTX(L, hipEventCreate(&e1));
-        float best = 1e30f;
-        const int nts[4] = {128, 256, 512, 1024};
-        HIPCHK_CTX(L, copy_set(1));   // the start, kept for the tuning runs
-        for (int c = 0; c < MDN_BATCH_CANDIDATES; c++) {
-            const int nt = nts[c >> 1], sorted = c & 1;
-            HIPCHK_CTX(L, copy_set(2));   // every candidate starts from the given coordinates
-            HIPCHK_CTX(L, hipMemcpyAsync(L->batch_order.p, sorted ? order_sorted.data() : order_given.data(),
-                                         sizeof(int) * n, hipMemcpyHostToDevice, L->stream));
-            HIPCHK_CTX(L, hipEventRecord(e0, L->stream));
-            if ((st = run_batched(L, n, T, p->precision, nt))) return st;
-            HIPCHK_CTX(L, hipEventRecord(e1, L->stream));
-            HIPCHK_CTX(L, hipEventSynchronize(e1));
-            float ms = 0;
-            HIPCHK_CTX(L, hipEventElapsedTime(&ms, e0, e1));
-            L->batch_tune_ms[c] = ms;
-            if (ms < best) {
-                best = ms;
-                L->batch_nt = nt;
-                L->batch_sorted = sorted;
-            }
+    hipLaunchKernelGGL(k_batch_copy, cgrid, dim3(256), 0, L->stream, (const BatchCopy*)L->batch_copy.p, n);
+    // a grid's second dimension holds at most 65535 systems: the launches below go in parts
+    for (int i0 = 0; i0 < n; i0 += 32768) {
+        const unsigned m = (unsigned)std::min(n - i0, 32768);
+        const bool mixed = p->precision == MDN_PREC_MIXED;
+        const dim3 vg((unsigned)std::min(64, max_nbb), m), b(BLOCK);
+        const BatchItem* d = di + i0;
+        hipLaunchKernelGGL(k_batch_zero, vg, b, 0, L->stream, d);
+        hipLaunchKernelGGL(k_batch_energy<double>, dim3(max_blk, m), b, 0, L->stream, d, 0);
+        hipLaunchKernelGGL(k_batch_energy_fin, dim3(m), b, 0, L->stream, d, 0, 0);
+        if (mixed) {   // the minimizer's own start energy
+            hipLaunchKernelGGL(k_batch_energy<float>, dim3(max_blk, m), b, 0, L->stream, d, 0);
+            hipLaunchKernelGGL(k_batch_energy_fin, dim3(m), b, 0, L->stream, d, 0, 18);
+            hipLaunchKernelGGL(k_batch_terms<float>, dim3(max_terms, m), b, 0, L->stream, d);
+            hipLaunchKernelGGL(k_batch_gather<float>, dim3(max_nbb, m), b, 0, L->stream, d);
+        } else {
+            hipLaunchKernelGGL(k_batch_terms<double>, dim3(max_terms, m), b, 0, L->stream, d);
+            hipLaunchKernelGGL(k_batch_gather<double>, dim3(max_nbb, m), b, 0, L->stream, d);
         }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        L->batch_key = key;
-        L->batch_tuned = 1;
-        // the tuning runs moved the coordinates: start again from the given ones
-        HIPCHK_CTX(L, copy_set(2));
-    } else {
-        L->batch_tuned = 0;
+        hipLaunchKernelGGL(k_batch_init, dim3(m), dim3(SUM_NT), 0, L->stream, d, P, mixed ? 18 : 0);
+        HIPCHK_CTX(L, hipGetLastError());
     }
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_order.p, L->batch_sorted ? order_sorted.data() : order_given.data(),
-                                 sizeof(int) * n, hipMemcpyHostToDevice, L->stream));
-    if ((st = run_batched(L, n, P, p->precision, L->batch_nt))) return st;
-    HIPCHK_CTX(L, hipStreamSynchronize(L->stream));
+    if ((st = launch_batch(L, plan, p->precision))) return st;
+    for (int i0 = 0; i0 < n; i0 += 32768) {
+        const unsigned m = (unsigned)std::min(n - i0, 32768);
+        const BatchItem* d = di + i0;
+        hipLaunchKernelGGL(k_batch_restore, dim3((unsigned)std::min(64, max_nbb), m), dim3(BLOCK), 0, L->stream, d,
+                           P.report_on_call_limit);
+        hipLaunchKernelGGL(k_batch_energy<double>, dim3(max_blk, m), dim3(BLOCK), 0, L->stream, d, 1);
+        hipLaunchKernelGGL(k_batch_energy_fin, dim3(m), dim3(BLOCK), 0, L->stream, d, 1, 9);
+    }
+    HIPCHK_CTX(L, hipGetLastError());
     // results: every system's state and report gathered on the device and read back at once, then
     // the coordinates (and forces) of every system queued with one synchronization
     HIPCHK_CTX(L, L->batch_states.ensure((size_t)n));
@@ -2157,9 +2274,14 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     HIPCHK_CTX(L, hipGetLastError());
     std::vector<CgState> states(n);
     std::vector<double> reports(27 * (size_t)n);
+    std::vector<TeamCtl> ctl(plan.team.size());
     HIPCHK_CTX(L, hipMemcpyAsync(states.data(), L->batch_states.p, sizeof(CgState) * n, hipMemcpyDeviceToHost,
                                  L->stream));
+    HIPCHK_CTX(L, hipMemcpyAsync(ctl.data(), L->batch_ctl.p, sizeof(TeamCtl) * ctl.size(), hipMemcpyDeviceToHost,
+                                 L->stream));
     HIPCHK_CTX(L, d2h(L, reports.data(), L->batch_reports.p, sizeof(double) * 27 * n));
+    for (const TeamCtl& c : ctl)
+        if (c.failed) return fail(L, MDN_ERR_STATE, "a workgroup of the minimizer gave up waiting for the others");
     for (int i = 0; i < n; i++) {
         mdn_ctx* c = ctxs[i];
         const CgState& S = states[i];
@@ -2209,10 +2331,10 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
 int mdn_last_batch_schedule(mdn_ctx* ctx, int32_t* out3, double* tune_ms) {
     if (!ctx || !out3) return MDN_ERR_ARG;
     out3[0] = ctx->batch_nt;
-    out3[1] = ctx->batch_sorted;
-    out3[2] = ctx->batch_tuned;
+    out3[1] = 1;
+    out3[2] = 0;
     if (tune_ms)
-        for (int c = 0; c < MDN_BATCH_CANDIDATES; c++) tune_ms[c] = ctx->batch_tune_ms[c];
+        for (int c = 0; c < MDN_BATCH_CANDIDATES; c++) tune_ms[c] = 0.0;
     return MDN_OK;
 }
 

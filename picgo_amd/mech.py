@@ -390,7 +390,7 @@ def minimize_batched(systems, params, coords, want_forces=True):
 
 
 def last_batch_schedule(lead):
-    """(workgroup size, largest-first order, tuned in the last call, tuning times in ms)."""
+    """(workgroup size, largest-first order, tuned in the last call (0), times in ms (zeros))."""
     out = (C.c_int32 * 3)()
     ms = (C.c_double * abi.MDN_BATCH_CANDIDATES)()
     st = lib().mdn_last_batch_schedule(lead._h, out, ms)
