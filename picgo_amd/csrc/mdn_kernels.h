@@ -715,16 +715,21 @@ __global__ void __launch_bounds__(BLOCK, sizeof(R) == 4 ? 4 : 1) k_forces_terms(
 // force[b] = base[b] + the bonded pieces selected by bmask + b's slots with id in [lo, hi)
 // (base may be null: zero-fill). BG: the first two terms come as the bonded sums of the terms
 // kernel's bead blocks (which took base and bmask); else from base and the piece arrays. Grid:
-// gather blocks (GB beads each).
+// gather blocks (GB beads each). bad (may be null): the terms kernel's count of pairs that need
+// the numerical fallback; it goes to *bad_host (pinned host memory), so the host learns it with
+// the forces in one wait, and unless it is zero no force is written.
 template <typename R, int GB, bool BG>
 __global__ void __launch_bounds__(BLOCK) k_gather_plain(DevSys s, int bmask, const R* __restrict__ slots, long lo,
-                                                        long hi, const double* __restrict__ base, double* __restrict__ f) {
+                                                        long hi, const double* __restrict__ base, double* __restrict__ f,
+                                                        const int* __restrict__ bad, int* bad_host) {
     __shared__ double L[GCHUNK_BYTES / sizeof(double)];
+    const int n_bad = bad ? *bad : 0;
+    if (bad && blockIdx.x == 0 && threadIdx.x == 0) *bad_host = n_bad;
     const int b = blockIdx.x * GB + threadIdx.x;
     const bool mine = threadIdx.x < GB && b < s.n_beads;
     D3 acc = (!BG && base && mine) ? D3{base[3 * b], base[3 * b + 1], base[3 * b + 2]} : D3{0.0, 0.0, 0.0};
     acc = gather_block<R, GB, BG>(s, bmask, slots, lo, hi, lo == 0 && hi == s.slot0[NFF], acc, L);
-    if (!mine) return;
+    if (!mine || n_bad) return;
     f[3 * b] = acc.x; f[3 * b + 1] = acc.y; f[3 * b + 2] = acc.z;
 }
 

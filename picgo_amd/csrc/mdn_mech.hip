@@ -268,17 +268,22 @@ int gather_blocks(mdn_ctx* ctx) { return std::max(1, ceil_div(ctx->n_beads, gath
 // the gather kernels at the context's beads-per-block
 template <typename R>
 void launch_gather_plain(mdn_ctx* ctx, const DevSys& s, int bmask, const R* slots, long lo, long hi, const double* base,
-                         double* out, bool bg) {
+                         double* out, bool bg, const int* bad = nullptr) {
+    int* host = ctx->h_int;
     const dim3 g(gather_blocks(ctx)), b(BLOCK);
     const bool l = gather_size(ctx) == 128;
     if (bg && l)
-        hipLaunchKernelGGL((k_gather_plain<R, 128, true>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out);
+        hipLaunchKernelGGL((k_gather_plain<R, 128, true>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out, bad,
+                           host);
     else if (bg)
-        hipLaunchKernelGGL((k_gather_plain<R, 64, true>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out);
+        hipLaunchKernelGGL((k_gather_plain<R, 64, true>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out, bad,
+                           host);
     else if (l)
-        hipLaunchKernelGGL((k_gather_plain<R, 128, false>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out);
+        hipLaunchKernelGGL((k_gather_plain<R, 128, false>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out, bad,
+                           host);
     else
-        hipLaunchKernelGGL((k_gather_plain<R, 64, false>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out);
+        hipLaunchKernelGGL((k_gather_plain<R, 64, false>), g, b, 0, ctx->stream, s, bmask, slots, lo, hi, base, out, bad,
+                           host);
 }
 // The terms kernel's grid: every interaction block (pieces: the filament terms write their
 // pieces), or the other force fields' blocks followed by the bead blocks of the bonded sums.
@@ -393,39 +398,38 @@ int set_coords_dev(mdn_ctx* ctx, const double* coord) {
     return MDN_OK;
 }
 
-// Term forces + numerical fallback for non-finite excluded-volume pairs, into ctx->slots (in
-// the arithmetic type R), at device coordinates x.
+// The term kernel at device coordinates x into slots (in the arithmetic type R); the pairs whose
+// closed-form forces are non-finite are counted and listed. pieces: the filament terms' pieces for
+// a gather that reads them; else the bonded sums of the pieces selected by bmask on top of base
+// (null: zero) for a gather that starts from them.
 template <typename R>
-int eval_slots_t(mdn_ctx* ctx, const double* x, bool pieces, int bmask, const double* base) {
-    const DevSys& s = ctx->sys;
-    R* slots = reinterpret_cast<R*>(ctx->slots.p);
-    HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
+void launch_terms(mdn_ctx* ctx, const DevSys& s, const double* x, R* slots, bool pieces, int bmask, const double* base,
+                  int* bad_count, int* bad_list) {
     if (force_blocks(s, pieces) > 0)
         hipLaunchKernelGGL(k_forces_terms<R>, dim3(force_blocks(s, pieces)), dim3(BLOCK), 0, ctx->stream, s, x, slots,
-                           ctx->bad_count.p, ctx->bad_list.p, bead_block0(s, pieces), bmask, base);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(ctx->h_int, ctx->bad_count.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    int nbad = ctx->h_int[0];
-    if (nbad == 0) return MDN_OK;
-    std::vector<int> bad(nbad);
-    HIPCHK(d2h(ctx, bad.data(), ctx->bad_list.p, sizeof(int) * nbad));
-    std::sort(bad.begin(), bad.end());
-    const int G = 240;
-    HIPCHK(ctx->fallback_partial.ensure(6 * G));
-    HIPCHK(ctx->fallback_ok.ensure(1));
-    for (int t : bad) {
-        // forceN (FP64 in both paths), retried once with beads 1 and 2 moved out of plane
-        // (CylinderExclVolRepulsion.cpp:1198-1204)
+                           bad_count, bad_list, bead_block0(s, pieces), bmask, base);
+}
+
+constexpr int FORCEN_BLOCKS = 240;
+
+// forceN (FP64 in both paths) for the nbad listed pairs, into their slots: retried once with beads
+// 1 and 2 moved out of plane (CylinderExclVolRepulsion.cpp:1198-1204). Each pair writes only its
+// own slots, so the order does not matter.
+template <typename R>
+int settle_pairs(mdn_ctx* ctx, const DevSys& s, const double* x, R* slots, const int* bad_list, int nbad,
+                 double* partial, int* ok_dev) {
+    for (int i = 0; i < nbad; i++) {
+        HIPCHK(d2h(ctx, ctx->h_int + 1, bad_list + i, sizeof(int)));
+        const int t = ctx->h_int[1];
         int ok = 0;
         for (int mv = 0; mv < 2 && !ok; mv++) {
-            hipLaunchKernelGGL(k_exvol_forceN_rows, dim3(G), dim3(BLOCK), 0, ctx->stream, s, x, t, mv,
-                               ctx->fallback_partial.p);
-            hipLaunchKernelGGL(k_exvol_forceN_finish<R>, dim3(1), dim3(64), 0, ctx->stream, s, x, t, mv, G,
-                               (const double*)ctx->fallback_partial.p, slots, ctx->fallback_ok.p);
-            HIPCHK(hipMemcpyAsync(ctx->h_int, ctx->fallback_ok.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(hipStreamSynchronize(ctx->stream));
-            ok = ctx->h_int[0];
+            hipLaunchKernelGGL(k_exvol_forceN_rows, dim3(FORCEN_BLOCKS), dim3(BLOCK), 0, ctx->stream, s, x, t, mv,
+                               partial);
+            hipLaunchKernelGGL(k_exvol_forceN_finish<R>, dim3(1), dim3(64), 0, ctx->stream, s, x, t, mv,
+                               FORCEN_BLOCKS, (const double*)partial, slots, ok_dev);
+            HIPCHK(hipGetLastError());
+            HIPCHK(d2h(ctx, ctx->h_int + 2, ok_dev, sizeof(int)));
+            ok = ctx->h_int[2];
         }
         if (!ok)
             return fail(ctx, MDN_ERR_NONFINITE,
@@ -433,46 +437,96 @@ int eval_slots_t(mdn_ctx* ctx, const double* x, bool pieces, int bmask, const do
     }
     return MDN_OK;
 }
-// pieces: the filament terms' pieces for a gather that reads them; else the bonded sums of
-// the pieces selected by bmask on top of base (null: zero) for a gather that starts from them
-int eval_slots(mdn_ctx* ctx, const double* x, int prec, bool pieces, int bmask = 3, const double* base = nullptr) {
-    return prec == MDN_PREC_MIXED ? eval_slots_t<float>(ctx, x, pieces, bmask, base)
-                                  : eval_slots_t<double>(ctx, x, pieces, bmask, base);
+int settle_pairs(mdn_ctx* ctx, const double* x, int prec, int nbad) {
+    HIPCHK(ctx->fallback_partial.ensure(6 * FORCEN_BLOCKS));
+    HIPCHK(ctx->fallback_ok.ensure(1));
+    const DevSys& s = ctx->sys;
+    return prec == MDN_PREC_MIXED
+               ? settle_pairs<float>(ctx, s, x, (float*)ctx->slots.p, ctx->bad_list.p, nbad, ctx->fallback_partial.p,
+                                     ctx->fallback_ok.p)
+               : settle_pairs<double>(ctx, s, x, ctx->slots.p, ctx->bad_list.p, nbad, ctx->fallback_partial.p,
+                                      ctx->fallback_ok.p);
 }
 
-// force = base + the bonded pieces selected by bmask (bit 0 stretching, bit 1 bending) + the
-// slots with id in [lo, hi). bg: the first two terms come as the bonded sums the terms kernel's
-// bead blocks wrote (eval_slots without pieces, with the same bmask and base).
-int gather(mdn_ctx* ctx, int bmask, long lo, long hi, const double* base, double* out, int prec, bool bg) {
+// Term forces at x with the fallback settled, into ctx->slots (synchronous).
+int eval_slots(mdn_ctx* ctx, const double* x, int prec, bool pieces) {
+    HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
     if (prec == MDN_PREC_MIXED)
-        launch_gather_plain<float>(ctx, ctx->sys, bmask, (const float*)ctx->slots.p, lo, hi, base, out, bg);
+        launch_terms<float>(ctx, ctx->sys, x, (float*)ctx->slots.p, pieces, 3, nullptr, ctx->bad_count.p, ctx->bad_list.p);
     else
-        launch_gather_plain<double>(ctx, ctx->sys, bmask, (const double*)ctx->slots.p, lo, hi, base, out, bg);
+        launch_terms<double>(ctx, ctx->sys, x, ctx->slots.p, pieces, 3, nullptr, ctx->bad_count.p, ctx->bad_list.p);
     HIPCHK(hipGetLastError());
-    return MDN_OK;
+    HIPCHK(d2h(ctx, ctx->h_int, ctx->bad_count.p, sizeof(int)));
+    return ctx->h_int[0] ? settle_pairs(ctx, x, prec, ctx->h_int[0]) : MDN_OK;
 }
 
-void launch_energy(mdn_ctx* ctx, const double* x, int prec) {
+// One force evaluation at device coordinates x into out: base + the bonded pieces selected by
+// bmask (bit 0 stretching, bit 1 bending) + the slots with id in [lo, hi). start() queues the terms
+// and the gather, before the host knows whether a pair needs the numerical fallback (rare: the
+// gather then writes nothing); after the caller's wait finish() settles those pairs and queues
+// the gather again. So an evaluation costs one wait.
+struct ForceEval {
+    mdn_ctx* ctx;
+    const double* x;
+    int prec, bmask;
+    long lo, hi;
+    const double* base;
+    double* out;
+
+    void gather(const int* bad) {
+        const bool bg = ctx->bg_eval != 0;
+        if (prec == MDN_PREC_MIXED)
+            launch_gather_plain<float>(ctx, ctx->sys, bmask, (const float*)ctx->slots.p, lo, hi, base, out, bg, bad);
+        else
+            launch_gather_plain<double>(ctx, ctx->sys, bmask, (const double*)ctx->slots.p, lo, hi, base, out, bg, bad);
+    }
+    int start() {
+        const bool pieces = ctx->bg_eval == 0;
+        HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
+        if (prec == MDN_PREC_MIXED)
+            launch_terms<float>(ctx, ctx->sys, x, (float*)ctx->slots.p, pieces, bmask, base, ctx->bad_count.p,
+                                ctx->bad_list.p);
+        else
+            launch_terms<double>(ctx, ctx->sys, x, ctx->slots.p, pieces, bmask, base, ctx->bad_count.p, ctx->bad_list.p);
+        gather(ctx->bad_count.p);
+        HIPCHK(hipGetLastError());
+        return MDN_OK;
+    }
+    // after a synchronization of the stream: *redone when the forces were gathered again (queued)
+    int finish(bool* redone) {
+        *redone = ctx->h_int[0] != 0;
+        if (!*redone) return MDN_OK;
+        const int st = settle_pairs(ctx, x, prec, ctx->h_int[0]);
+        if (st) return st;
+        gather(nullptr);
+        HIPCHK(hipGetLastError());
+        return MDN_OK;
+    }
+};
+
+// Per-FF energies at device coordinates x into out[0..8] (pinned host memory), queued.
+void launch_energy(mdn_ctx* ctx, const double* x, int prec, double* out) {
     const DevSys& s = ctx->sys;
     int grid = std::max(1, s.blk[NFF]);
     if (prec == MDN_PREC_MIXED)
         hipLaunchKernelGGL(k_energy_report<float>, dim3(grid), dim3(BLOCK), 0, ctx->stream, s, x, ctx->partial.p);
     else
         hipLaunchKernelGGL(k_energy_report<double>, dim3(grid), dim3(BLOCK), 0, ctx->stream, s, x, ctx->partial.p);
-    hipLaunchKernelGGL(k_energy_report_fin, dim3(1), dim3(BLOCK), 0, ctx->stream, s, (const double*)ctx->partial.p,
-                       ctx->eout.p);
+    hipLaunchKernelGGL(k_energy_report_fin, dim3(1), dim3(BLOCK), 0, ctx->stream, s, (const double*)ctx->partial.p, out);
+}
+int check_energy(mdn_ctx* ctx, const double* e) {
+    if (e[8] != 0.0)
+        return fail(ctx, MDN_ERR_UNSUPPORTED, "%.0f excluded-volume pairs need the Simpson energy (capacity %d)", e[8],
+                    DEFER_CAP);
+    return MDN_OK;
 }
 
-// Per-FF energies at device coordinates x into ctx->h_eout[0..7] (synchronous).
+// Per-FF energies at device coordinates x into ctx->h_eout[0..8] (synchronous).
 int energy_report(mdn_ctx* ctx, const double* x, int prec) {
-    launch_energy(ctx, x, prec);
+    launch_energy(ctx, x, prec, ctx->h_eout);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(ctx->h_eout, ctx->eout.p, sizeof(double) * 9, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (ctx->h_eout[8] != 0.0)
-        return fail(ctx, MDN_ERR_UNSUPPORTED, "%.0f excluded-volume pairs need the Simpson energy (capacity %d)",
-                    ctx->h_eout[8], DEFER_CAP);
-    return MDN_OK;
+    return check_energy(ctx, ctx->h_eout);
 }
 
 void fill_report(const double* e, mdn_energy_report* out) {
@@ -1366,9 +1420,11 @@ static int forces_impl(mdn_ctx* ctx, int ff, const double* coord, double* force,
         base = ctx->scratch_f.p;
     }
     const int bmask = ff < 0 ? 3 : ff == FF_STRETCH ? 1 : ff == FF_BEND ? 2 : 0;
-    const bool bg = ctx->bg_eval != 0;
-    if ((st = eval_slots(ctx, x, prec, !bg, bmask, base))) return st;
-    if ((st = gather(ctx, bmask, lo, hi, base, ctx->f.p, prec, bg))) return st;
+    ForceEval ev{ctx, x, prec, bmask, lo, hi, base, ctx->f.p};
+    if ((st = ev.start())) return st;
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    bool redone;
+    if ((st = ev.finish(&redone))) return st;
     HIPCHK(hipMemcpyAsync(force, ctx->f.p, sizeof(double) * n_var, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return MDN_OK;
@@ -1641,7 +1697,6 @@ namespace {
 struct ScratchLayout {
     size_t bad_count, ok, partial, bad_list, bsum, slots, total;
 };
-constexpr int FORCEN_BLOCKS = 240;
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 ScratchLayout scratch_layout(const DevSys& s, int n_beads, size_t rsize) {
     ScratchLayout L;
@@ -1665,33 +1720,18 @@ int forces_noalloc_t(mdn_ctx* ctx, unsigned char* scr, const double* x, double* 
     int* bad_list = reinterpret_cast<int*>(scr + L.bad_list);
     s.bsum = reinterpret_cast<double*>(scr + L.bsum);
     R* slots = reinterpret_cast<R*>(scr + L.slots);
-    // the previous call's count stays in the array: clear it (a kernel, not a memset node)
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, bad_count, 0);
-    hipLaunchKernelGGL(k_forces_terms<R>, dim3(force_blocks(s, false)), dim3(BLOCK), 0, ctx->stream, s, x, slots,
-                       bad_count, bad_list, bead_block0(s, false), 3, (const double*)nullptr);
+    // the terms, then the gather before the host knows whether a pair needs the numerical fallback
+    // and writes nothing if one does. Two launches and one wait bound the call: with a launch that
+    // cleared the count and a wait for it between the two it took 35 us at 550 beads, 38 at 42,000
+    // and 62 at 420,000; now 21, 24 and 48. The count is zero between calls.
+    launch_terms<R>(ctx, s, x, slots, false, 3, nullptr, bad_count, bad_list);
+    launch_gather_plain<R>(ctx, s, 3, (const R*)slots, 0L, s.slot0[NFF], (const double*)nullptr, out, true, bad_count);
     HIPCHK(hipGetLastError());
-    HIPCHK(d2h(ctx, ctx->h_int, bad_count, sizeof(int)));
-    const int nbad = ctx->h_int[0];
-    // pairs whose closed-form forces are non-finite: the Simpson forceN rule, retried once with
-    // beads 1 and 2 moved out of plane (CylinderExclVolRepulsion.cpp:1198-1204); each pair writes
-    // only its own slots, so the order does not matter
-    for (int i = 0; i < nbad; i++) {
-        HIPCHK(d2h(ctx, ctx->h_int + 1, bad_list + i, sizeof(int)));
-        const int t = ctx->h_int[1];
-        int done = 0;
-        for (int mv = 0; mv < 2 && !done; mv++) {
-            hipLaunchKernelGGL(k_exvol_forceN_rows, dim3(FORCEN_BLOCKS), dim3(BLOCK), 0, ctx->stream, s, x, t, mv,
-                               partial);
-            hipLaunchKernelGGL(k_exvol_forceN_finish<R>, dim3(1), dim3(64), 0, ctx->stream, s, x, t, mv,
-                               FORCEN_BLOCKS, (const double*)partial, slots, ok);
-            HIPCHK(hipGetLastError());
-            HIPCHK(d2h(ctx, ctx->h_int + 2, ok, sizeof(int)));
-            done = ctx->h_int[2];
-        }
-        if (!done)
-            return fail(ctx, MDN_ERR_NONFINITE,
-                        "excluded-volume pair %d: force non-finite after the numerical fallback", t);
-    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (ctx->h_int[0] == 0) return MDN_OK;
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(1), 0, ctx->stream, bad_count, 0);
+    const int st = settle_pairs<R>(ctx, s, x, slots, bad_list, ctx->h_int[0], partial, ok);
+    if (st) return st;
     launch_gather_plain<R>(ctx, s, 3, (const R*)slots, 0L, s.slot0[NFF], (const double*)nullptr, out, true);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1864,24 +1904,28 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     ctx->cur = 0;
     // the reported energies are FP64 in both precisions; the minimizer's own energies and forces
     // are evaluated in the requested precision
-    if ((st = energy_report(ctx, ctx->x[0].p, MDN_PREC_FP64))) return st;
-    fill_report(ctx->h_eout, &res->energies_before);
-    double e_start = res->energies_before.total;
-    if (prec == MDN_PREC_MIXED) {
-        if ((st = energy_report(ctx, ctx->x[0].p, prec))) return st;
-        e_start = ctx->h_eout[6];
-    }
-    if ((st = eval_slots(ctx, ctx->x[0].p, prec, !ctx->bg_eval))) return st;
-    if ((st = gather(ctx, 3, 0, ctx->sys.slot0[NFF], nullptr, ctx->f.p, prec, ctx->bg_eval != 0))) return st;
-    // F.F and maxF on the device (fixed-order reduction), two doubles back
+    // (the reports, the forces and F.F and maxF, a fixed-order reduction, in one wait)
+    double *rep = ctx->h_eout, *rep_mixed = ctx->h_eout + 10, *stats = ctx->h_eout + 24;
+    launch_energy(ctx, ctx->x[0].p, MDN_PREC_FP64, rep);
+    if (prec == MDN_PREC_MIXED) launch_energy(ctx, ctx->x[0].p, prec, rep_mixed);
+    ForceEval fe{ctx, ctx->x[0].p, prec, 3, 0, ctx->sys.slot0[NFF], nullptr, ctx->f.p};
+    if ((st = fe.start())) return st;
     const int nsb = std::min(VSTAT_BLOCKS, std::max(1, ceil_div(nv, BLOCK)));
-    hipLaunchKernelGGL(k_vec_stats, dim3(nsb), dim3(BLOCK), 0, ctx->stream, (const double*)ctx->f.p, (long)nv,
-                       ctx->vstat.p);
-    hipLaunchKernelGGL(k_vec_stats_fin, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double*)ctx->vstat.p, nsb,
-                       ctx->eout.p + 16);
-    HIPCHK(hipMemcpyAsync(ctx->h_eout + 16, ctx->eout.p + 16, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    const double ff = ctx->h_eout[16], mx = ctx->h_eout[17];
+    bool redo = true;
+    for (int pass = 0; pass < 2 && redo; pass++) {   // again when a pair took the numerical fallback
+        hipLaunchKernelGGL(k_vec_stats, dim3(nsb), dim3(BLOCK), 0, ctx->stream, (const double*)ctx->f.p, (long)nv,
+                           ctx->vstat.p);
+        hipLaunchKernelGGL(k_vec_stats_fin, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double*)ctx->vstat.p, nsb, stats);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+        if (pass) break;
+        if ((st = check_energy(ctx, rep))) return st;
+        fill_report(rep, &res->energies_before);
+        if (prec == MDN_PREC_MIXED && (st = check_energy(ctx, rep_mixed))) return st;
+        if ((st = fe.finish(&redo))) return st;
+    }
+    const double e_start = prec == MDN_PREC_MIXED ? rep_mixed[6] : rep[6];
+    const double ff = stats[0], mx = stats[1];
     CgState& S = *ctx->h_cg;
     memset((void*)ctx->h_cg, 0, CG_BYTES);
     S.method = p->method;
@@ -2362,7 +2406,7 @@ static int bench_forces_t(mdn_ctx* ctx, int32_t iters, double* ms_per_eval, doub
     const int nb = std::max(1, force_blocks(s, pieces));
     int st;
     // warm-up (and fallback check) once
-    if ((st = eval_slots_t<R>(ctx, x, pieces, 3, nullptr))) return st;
+    if ((st = eval_slots(ctx, x, sizeof(R) == 4 ? MDN_PREC_MIXED : MDN_PREC_FP64, pieces))) return st;
     hipEvent_t e0, e1, k0, k1;
     HIPCHK(hipEventCreate(&e0)); HIPCHK(hipEventCreate(&e1)); HIPCHK(hipEventCreate(&k0)); HIPCHK(hipEventCreate(&k1));
     // whole evaluation: terms + gather
@@ -2484,7 +2528,7 @@ int mdn_bench_energy(mdn_ctx* ctx, int32_t precision, int32_t iters, double* ms_
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0)); HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, ctx->stream));
-    for (int i = 0; i < iters; i++) launch_energy(ctx, x, precision);
+    for (int i = 0; i < iters; i++) launch_energy(ctx, x, precision, ctx->h_eout);
     HIPCHK(hipEventRecord(e1, ctx->stream));
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventSynchronize(e1));
