@@ -733,15 +733,19 @@ __global__ void __launch_bounds__(BLOCK) k_gather_plain(DevSys s, int bmask, con
     f[3 * b] = acc.x; f[3 * b + 1] = acc.y; f[3 * b + 2] = acc.z;
 }
 
-// The FP64 gathers of several tangent products in one launch (k_gather_plain's gather of the
-// piece arrays and every slot, from zero): product k = blockIdx.y from its slots at
-// slots + k slot_stride and its pieces at piece + k piece_stride into f + k n_var.
+// The Hessian-vector products H v = -(dF/dx) v of the FP64 gathers of one or several tangents in
+// one launch (k_gather_plain's gather of the piece arrays and every slot, from zero): product
+// k = blockIdx.y from its slots at slots + k slot_stride and its pieces at piece + k piece_stride
+// into f + k n_var. The sign is taken here: a host loop over the copied products (16 of 42,000
+// beads: 16 MB) cost more than the kernel. *bad_host (pinned host memory) receives the tangent
+// kernel's count of pairs without a tangent.
 template <int GB>
 __global__ void __launch_bounds__(BLOCK) k_gather_tangents(DevSys s, const double* __restrict__ slots, long slot_stride,
                                                            double* piece, long piece_stride, double* __restrict__ f,
-                                                           long n_var) {
+                                                           long n_var, const int* __restrict__ bad, int* bad_host) {
     __shared__ double L[GCHUNK_BYTES / sizeof(double)];
     const long k = blockIdx.y;
+    if (k == 0 && blockIdx.x == 0 && threadIdx.x == 0) *bad_host = *bad;
     DevSys sk = s;
     sk.piece = piece + k * piece_stride;
     const int b = blockIdx.x * GB + threadIdx.x;
@@ -750,7 +754,7 @@ __global__ void __launch_bounds__(BLOCK) k_gather_tangents(DevSys s, const doubl
                                                    D3{0.0, 0.0, 0.0}, L);
     if (!mine) return;
     double* o = f + k * n_var;
-    o[3 * b] = acc.x; o[3 * b + 1] = acc.y; o[3 * b + 2] = acc.z;
+    o[3 * b] = -acc.x; o[3 * b + 1] = -acc.y; o[3 * b + 2] = -acc.z;
 }
 
 // Block-parallel Simpson energies (energyN) of the pairs deferred by the preceding kernel.

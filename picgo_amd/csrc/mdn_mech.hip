@@ -1546,7 +1546,8 @@ static void launch_tangents(mdn_ctx* ctx, const double* x, int prec, const doubl
                            piece, piece_stride, ctx->bad_count.p);
 }
 
-// (dF/dx) v of nv products into out + k n_var from their slots and pieces (one launch).
+// -(dF/dx) v of nv products into out + k n_var from their slots and pieces (one launch); the
+// count of pairs without a tangent into ctx->h_int[0].
 static void gather_tangents(mdn_ctx* ctx, int nv, const double* slots, long slot_stride, double* piece,
                             long piece_stride, double* out) {
     const DevSys& s = ctx->sys;
@@ -1554,27 +1555,20 @@ static void gather_tangents(mdn_ctx* ctx, int nv, const double* slots, long slot
     const long n_var = 3L * ctx->n_beads;
     if (gather_size(ctx) == 128)
         hipLaunchKernelGGL(k_gather_tangents<128>, g, b, 0, ctx->stream, s, slots, slot_stride, piece, piece_stride, out,
-                           n_var);
+                           n_var, (const int*)ctx->bad_count.p, ctx->h_int);
     else
         hipLaunchKernelGGL(k_gather_tangents<64>, g, b, 0, ctx->stream, s, slots, slot_stride, piece, piece_stride, out,
-                           n_var);
+                           n_var, (const int*)ctx->bad_count.p, ctx->h_int);
 }
 
-// (dF/dx) v of one product into out from its slots and pieces (the FP64 gather).
-static void gather_tangent(mdn_ctx* ctx, const double* slots, double* piece, double* out) {
-    DevSys s = ctx->sys;
-    s.piece = piece;
-    launch_gather_plain<double>(ctx, s, 3, slots, 0L, s.slot0[NFF], (const double*)nullptr, out, false);
-}
-
-// -H v into ctx->scratch_f for the device tangent ctx->tan_v at device coordinates x (the tangent
+// H v into ctx->scratch_f for the device tangent ctx->tan_v at device coordinates x (the tangent
 // pieces of every interaction, then the FP64 gather); excluded-volume pairs without a tangent are
 // counted in bad_count.
 static int hvp_launch(mdn_ctx* ctx, const double* x, int prec) {
     HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
     launch_tangents(ctx, x, prec, ctx->tan_v.p, 1, ctx->slots.p, 0L, ctx->piece.p, 0L);
     HIPCHK(hipGetLastError());
-    gather_tangent(ctx, ctx->slots.p, ctx->piece.p, ctx->scratch_f.p);
+    gather_tangents(ctx, 1, ctx->slots.p, 0L, ctx->piece.p, 0L, ctx->scratch_f.p);
     HIPCHK(hipGetLastError());
     return MDN_OK;
 }
@@ -1593,12 +1587,10 @@ static int hvp_impl(mdn_ctx* ctx, const double* coord, const double* v, double* 
     HIPCHK(hipMemcpyAsync(ctx->tan_v.p, v, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
     if ((st = hvp_launch(ctx, x, prec))) return st;
     HIPCHK(hipMemcpyAsync(out, ctx->scratch_f.p, sizeof(double) * n_var, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(ctx->h_int, ctx->bad_count.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->h_int[0] != 0)
         return fail(ctx, MDN_ERR_UNSUPPORTED, "%d excluded-volume pairs need the numerical force fallback (no tangent)",
                     ctx->h_int[0]);
-    for (int i = 0; i < n_var; i++) out[i] = -out[i];   // H v = -(dF/dx) v
     return MDN_OK;
 }
 
@@ -1645,13 +1637,10 @@ int mdn_hvp_batch(mdn_ctx* ctx, int32_t precision, const double* coord, const do
         HIPCHK(hipMemcpyAsync(out + (size_t)k0 * n_var, ctx->hb_out.p, sizeof(double) * nv * n_var,
                               hipMemcpyDeviceToHost, ctx->stream));
     }
-    HIPCHK(hipMemcpyAsync(ctx->h_int, ctx->bad_count.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->h_int[0] != 0)
         return fail(ctx, MDN_ERR_UNSUPPORTED, "%d excluded-volume pairs need the numerical force fallback (no tangent)",
                     ctx->h_int[0]);
-    const size_t total = (size_t)n_vec * n_var;
-    for (size_t i = 0; i < total; i++) out[i] = -out[i];   // H v = -(dF/dx) v
     return MDN_OK;
 }
 
