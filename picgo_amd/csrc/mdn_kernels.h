@@ -1898,10 +1898,13 @@ __device__ inline int nl_bin_id(const NLDev& n, int x, int y, int z) {
     return (tile << (3 * n.lt)) + (x & m) + ((y & m) << n.lt) + ((z & m) << (2 * n.lt));
 }
 
-// midpoints 0.5*(x1 + x2) (Cylinder.cpp:48) and bin index; flags out-of-grid cylinders
+// midpoints 0.5*(x1 + x2) (Cylinder.cpp:48), bin index and place in the bin; flags out-of-grid
+// cylinders; clears the counts' end (count[n_cyl], which the offsets' scan reads)
 __global__ void k_nl_bin(NLDev n, const double* __restrict__ x, double* __restrict__ mid, int* __restrict__ bin,
-                         int* __restrict__ bin_count, int* __restrict__ err) {
+                         int* __restrict__ place, int* __restrict__ bin_count, int* __restrict__ err,
+                         int* __restrict__ count) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c == n.n_cyl) count[c] = 0;
     if (c >= n.n_cyl) return;
     int b1 = n.cyl_b1[c], b2 = n.cyl_b2[c];
     int ix[3];
@@ -1916,39 +1919,37 @@ __global__ void k_nl_bin(NLDev n, const double* __restrict__ x, double* __restri
     }
     if (!ok) {
         atomicAdd(err, 1);
-        bin[c] = 0;
+        bin[c] = -1;
         return;
     }
     int bb = nl_bin_id(n, ix[0], ix[1], ix[2]);
     bin[c] = bb;
-    atomicAdd(&bin_count[bb], 1);
+    place[c] = atomicAdd(&bin_count[bb], 1);
 }
 
-// the members of each bin, with their bin and midpoint in the same (bin) order
-__global__ void k_nl_fill(int n_cyl, const int* __restrict__ bin, const int* __restrict__ bin_start,
-                          int* __restrict__ cursor, const double* __restrict__ mid, int* __restrict__ members,
+// What the list predicate reads of a cylinder besides its midpoint.
+struct __align__(16) NlRec { int c, fil, pos, type; };
+
+// the members of each bin: their records, bins and midpoints, in bin order
+__global__ void k_nl_fill(NLDev n, const int* __restrict__ bin, const int* __restrict__ bin_start,
+                          const int* __restrict__ place, const double* __restrict__ mid, NlRec* __restrict__ members,
                           int* __restrict__ mbin, double* __restrict__ mmid) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n_cyl) return;
+    if (c >= n.n_cyl) return;
     int bb = bin[c];
-    int k = atomicAdd(&cursor[bb], 1);
-    const int m = bin_start[bb] + k;
-    members[m] = c;
+    if (bb < 0) return;
+    const int m = bin_start[bb] + place[c];
+    members[m] = NlRec{c, n.cyl_fil[c], n.cyl_pos[c], n.cyl_type[c]};
     mbin[m] = bb;
     for (int q = 0; q < 3; q++) mmid[3 * (long)m + q] = mid[3 * (long)c + q];
 }
 
-// HybridNeighborListImpl.cpp:411-439 predicate, on explicit midpoints (a candidate's from LDS)
-__device__ inline bool nl_keep_at(const NLDev& n, int c, int cn, const double* mc, const double* mn) {
-    if (c <= cn) return false;
-    if (n.cyl_fil[c] == n.cyl_fil[cn]) {
-        int sep = abs(n.cyl_pos[c] - n.cyl_pos[cn]);
-        if (sep <= 2) return false;
-    }
-    if (n.ta >= 0) {
-        const int t1 = n.cyl_type[c], t2 = n.cyl_type[cn];
-        if (min(t1, t2) != n.ta || max(t1, t2) != n.tb) return false;
-    }
+// HybridNeighborListImpl.cpp:411-439 predicate, on explicit records and midpoints (a candidate's
+// from LDS)
+__device__ inline bool nl_keep_at(const NLDev& n, const NlRec& c, const NlRec& cn, const double* mc, const double* mn) {
+    if (c.c <= cn.c) return false;
+    if (c.fil == cn.fil && abs(c.pos - cn.pos) <= 2) return false;
+    if (n.ta >= 0 && (min(c.type, cn.type) != n.ta || max(c.type, cn.type) != n.tb)) return false;
     double d2 = 0.0;
     for (int q = 0; q < 3; q++) {
         double v = mn[q] - mc[q];
@@ -1962,22 +1963,35 @@ __device__ inline bool nl_keep_at(const NLDev& n, int c, int cn, const double* m
 //   1. each thread takes halo bins (the tile's bins and one bin around them, (T + 2)^3) and
 //      reads their member ranges; a block scan of the counts places every halo bin's members
 //      contiguously, in halo-bin order, in LDS with their midpoints,
-//   2. every cylinder of the tile tests the members of its 27 bins, read from LDS as nine
-//      x-rows of three consecutive halo bins.
+//   2. NL_LANES lanes per cylinder of the tile test the members of its 27 bins, each lane a row
+//      of three consecutive halo bins of LDS at a time (nine rows),
+//   3. the neighbours found, collected in LDS, are written in ascending order by rank.
 // A halo with more than NL_CAP members is read from global memory instead (the same 27 bins). The
 // bins are wider than the range, so the pair set is the predicate's whatever the bin size.
-// PASS 0: count per cylinder; PASS 1: emit into [off[c], off[c + 1]) and sort ascending.
-constexpr int NL_CAP = 768;
+// PASS 0: count per cylinder, the largest count, and the first NL_HITS neighbours into
+// found[NL_HITS c ...] (in order if there are no more): k_nl_emit then copies them into the list.
+// PASS 1, if a cylinder has more: emit into [off[c], off[c + 1]), sorted there.
+// Latency bound. With one lane per cylinder (36 of 256 lanes busy at 42,000 beads), the predicate's
+// records read from global memory and a second search that sorted in global memory, count and
+// emission took 105 us there, 205 us at 420,000 and 308 us for a binder's wider list at 42,000;
+// now 50, 74 and 63 us.
+constexpr int NL_CAP = 512;
 constexpr int NL_HMAX = 10 * 10 * 10;   // (T + 2)^3 for T <= 8
+constexpr int NL_RUN = (NL_HMAX + BLOCK - 1) / BLOCK;
+constexpr int NL_LANES = 8, NL_GROUPS = BLOCK / NL_LANES, NL_HITS = 32;
 
 template <int PASS>
 __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restrict__ bin_start,
-                                                   const int* __restrict__ members, const int* __restrict__ mbin,
+                                                   const NlRec* __restrict__ members, const int* __restrict__ mbin,
                                                    const double* __restrict__ mmid, int* __restrict__ count,
+                                                   int* __restrict__ most, int* __restrict__ found,
                                                    const int* __restrict__ off, int* __restrict__ pairs) {
-    __shared__ int s_a[NL_HMAX], s_start[NL_HMAX + 1], s_part[BLOCK];
-    __shared__ int s_sc[NL_CAP];
+    __shared__ int s_ah[NL_GROUPS * NL_HITS > NL_HMAX ? NL_GROUPS * NL_HITS : NL_HMAX];
+    __shared__ int s_start[NL_HMAX + 1], s_part[BLOCK / 64], s_cnt[NL_GROUPS];
+    __shared__ NlRec s_rec[NL_CAP];
     __shared__ double s_mid[3 * NL_CAP];
+    int* const s_a = s_ah;                                       // until the members are staged
+    int* const s_hit = s_ah + threadIdx.x / NL_LANES * NL_HITS;  // then the group's neighbours
     const int T = n.T, lt = n.lt, T3 = 1 << (3 * lt), H = T + 2, H3 = H * H * H;
     const int tile = blockIdx.x;
     const int i0 = bin_start[(long)tile * T3], i1 = bin_start[(long)(tile + 1) * T3];
@@ -1985,37 +1999,42 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
     const int tx = tile % n.nt[0], ty = (tile / n.nt[0]) % n.nt[1], tz = tile / (n.nt[0] * n.nt[1]);
     const int hx0 = tx * T - 1, hy0 = ty * T - 1, hz0 = tz * T - 1;
     // 1. the halo bins' member ranges (bins outside the grid are empty)
-    const int run = (H3 + BLOCK - 1) / BLOCK, r0 = threadIdx.x * run, r1 = min(r0 + run, H3);
-    int tot = 0;
-    for (int h = r0; h < r1; h++) {
-        const int X = hx0 + h % H, Y = hy0 + (h / H) % H, Z = hz0 + h / (H * H);
-        int a = 0, c = 0;
-        if (X >= 0 && Y >= 0 && Z >= 0 && X < n.nb[0] && Y < n.nb[1] && Z < n.nb[2]) {
+    const int run = (H3 + BLOCK - 1) / BLOCK, r0 = threadIdx.x * run;
+    const int inv = 65536 / H + 1;   // h / H = h * inv >> 16, exact for h < 1000 and H <= 10
+    int ra[NL_RUN], rc[NL_RUN], tot = 0;
+#pragma unroll
+    for (int j = 0; j < NL_RUN; j++) {
+        const int h = r0 + j, hz = (((h * inv) >> 16) * inv) >> 16, hy = ((h * inv) >> 16) - H * hz;
+        const int X = hx0 + h - H * (hy + H * hz), Y = hy0 + hy, Z = hz0 + hz;
+        ra[j] = rc[j] = 0;
+        if (j < run && h < H3 && X >= 0 && Y >= 0 && Z >= 0 && X < n.nb[0] && Y < n.nb[1] && Z < n.nb[2]) {
             const int g = nl_bin_id(n, X, Y, Z);
-            a = bin_start[g];
-            c = bin_start[g + 1] - a;
+            ra[j] = bin_start[g];
+            rc[j] = bin_start[g + 1];
         }
-        s_a[h] = a;
-        s_start[h] = c;
-        tot += c;
     }
-    s_part[threadIdx.x] = tot;
+#pragma unroll
+    for (int j = 0; j < NL_RUN; j++) {
+        rc[j] -= ra[j];
+        tot += rc[j];
+    }
+    int part = tot;   // inclusive scan of the runs' totals: in the wave, then over the waves
+    for (int step = 1; step < 64; step *= 2) {
+        const int v = __shfl_up(part, step);
+        if ((int)(threadIdx.x & 63) >= step) part += v;
+    }
+    if ((threadIdx.x & 63) == 63) s_part[threadIdx.x >> 6] = part;
     __syncthreads();
-    for (int step = 1; step < BLOCK; step *= 2) {   // inclusive scan of the runs' totals
-        const int v = threadIdx.x >= step ? s_part[threadIdx.x - step] : 0;
-        __syncthreads();
-        s_part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    {
-        int acc = s_part[threadIdx.x] - tot;   // exclusive prefix of this run
-        for (int h = r0; h < r1; h++) {
-            const int v = s_start[h];
-            s_start[h] = acc;
-            acc += v;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); w++) part += s_part[w];
+    int acc = part - tot;   // exclusive prefix of this run
+#pragma unroll
+    for (int j = 0; j < NL_RUN; j++)
+        if (j < run && r0 + j < H3) {
+            s_a[r0 + j] = ra[j];
+            s_start[r0 + j] = acc;
+            acc += rc[j];
         }
-        if (threadIdx.x == BLOCK - 1) s_start[H3] = s_part[BLOCK - 1];
-    }
+    if (threadIdx.x == BLOCK - 1) s_start[H3] = part;
     __syncthreads();
     const int nh = s_start[H3];
     const bool staged = nh <= NL_CAP;   // the same for the whole workgroup
@@ -2031,63 +2050,108 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
             }
             h = lo;
             const int m = s_a[h] + (j - s_start[h]);
-            s_sc[j] = members[m];
+            s_rec[j] = members[m];
             for (int q = 0; q < 3; q++) s_mid[3 * j + q] = mmid[3 * (long)m + q];
         }
         __syncthreads();
     }
-    // 2. the tile's cylinders
-    for (int i = i0 + threadIdx.x; i < i1; i += BLOCK) {
-        const int c = members[i];
-        const double mc[3] = {mmid[3 * (long)i], mmid[3 * (long)i + 1], mmid[3 * (long)i + 2]};
-        const int loc = mbin[i] & (T3 - 1);
-        const int lx = (loc & (T - 1)) + 1, ly = ((loc >> lt) & (T - 1)) + 1, lz = (loc >> (2 * lt)) + 1;   // halo coords
-        int cnt = 0;
-        const long base = PASS ? off[c] : 0;
-        if (staged) {
-            for (int dz = -1; dz <= 1; dz++)
-                for (int dy = -1; dy <= 1; dy++) {
+    // 2. the tile's cylinders, NL_GROUPS at a time
+    const int grp = threadIdx.x / NL_LANES, lane = threadIdx.x % NL_LANES;
+    for (int g0 = i0; g0 < i1; g0 += NL_GROUPS) {
+        const int i = g0 + grp;
+        const bool mine = i < i1;
+        const NlRec c = mine ? members[i] : NlRec{-1, 0, 0, 0};
+        const long base = PASS && mine ? off[c.c] : 0;
+        if (lane == 0) s_cnt[grp] = 0;
+        __syncthreads();
+        if (mine) {
+            const double mc[3] = {mmid[3 * (long)i], mmid[3 * (long)i + 1], mmid[3 * (long)i + 2]};
+            const int loc = mbin[i] & (T3 - 1);
+            const int lx = (loc & (T - 1)) + 1, ly = ((loc >> lt) & (T - 1)) + 1, lz = (loc >> (2 * lt)) + 1;   // halo coords
+            auto hit = [&](int cn) {
+                const int k = atomicAdd(&s_cnt[grp], 1);
+                if (k < NL_HITS) s_hit[k] = cn;
+                else if (PASS) pairs[2 * (base + k) + 1] = cn;
+            };
+            for (int r = lane; r < 9; r += NL_LANES) {
+                const int dy = r % 3 - 1, dz = r / 3 - 1;
+                if (staged) {
                     const int h = (lx - 1) + H * ((ly + dy) + H * (lz + dz));
-                    for (int k = s_start[h]; k < s_start[h + 3]; k++) {
-                        const int cn = s_sc[k];
-                        if (nl_keep_at(n, c, cn, mc, &s_mid[3 * k])) {
-                            if (PASS) pairs[2 * (base + cnt) + 1] = cn;
-                            cnt++;
-                        }
-                    }
-                }
-        } else {
-            for (int dz = -1; dz <= 1; dz++)
-                for (int dy = -1; dy <= 1; dy++)
+                    const int k1 = s_start[h + 3];
+                    for (int k = s_start[h]; k < k1; k++)
+                        if (nl_keep_at(n, c, s_rec[k], mc, &s_mid[3 * k])) hit(s_rec[k].c);
+                } else {
                     for (int dx = -1; dx <= 1; dx++) {
                         const int X = hx0 + lx + dx, Y = hy0 + ly + dy, Z = hz0 + lz + dz;
                         if (X < 0 || Y < 0 || Z < 0 || X >= n.nb[0] || Y >= n.nb[1] || Z >= n.nb[2]) continue;
                         const int nbin = nl_bin_id(n, X, Y, Z);
-                        for (int m = bin_start[nbin]; m < bin_start[nbin + 1]; m++) {
-                            const int cn = members[m];
-                            if (nl_keep_at(n, c, cn, mc, &mmid[3 * (long)m])) {
-                                if (PASS) pairs[2 * (base + cnt) + 1] = cn;
-                                cnt++;
-                            }
-                        }
+                        const int m1 = bin_start[nbin + 1];
+                        for (int m = bin_start[nbin]; m < m1; m++)
+                            if (nl_keep_at(n, c, members[m], mc, &mmid[3 * (long)m])) hit(members[m].c);
                     }
-        }
-        if (!PASS) {
-            count[c] = cnt;
-            continue;
-        }
-        // insertion sort of the neighbour ids, then the owning cylinder id
-        for (int a = 1; a < cnt; a++) {
-            const int v = pairs[2 * (base + a) + 1];
-            int j = a - 1;
-            while (j >= 0 && pairs[2 * (base + j) + 1] > v) {
-                pairs[2 * (base + j + 1) + 1] = pairs[2 * (base + j) + 1];
-                j--;
+                }
             }
-            pairs[2 * (base + j + 1) + 1] = v;
         }
-        for (int a = 0; a < cnt; a++) pairs[2 * (base + a)] = c;
+        __syncthreads();
+        // 3. in ascending order
+        const int cnt = mine ? s_cnt[grp] : 0;
+        const bool small = cnt <= NL_HITS;
+        for (int a = lane; a < min(cnt, NL_HITS); a += NL_LANES) {
+            const int v = s_hit[a];
+            int to = a;
+            if (small) {
+                to = 0;
+                for (int b = 0; b < cnt; b++) to += s_hit[b] < v;
+            }
+            if (PASS) {
+                pairs[2 * (base + to)] = c.c;
+                pairs[2 * (base + to) + 1] = v;
+            } else {
+                found[(long)NL_HITS * c.c + to] = v;
+            }
+        }
+        if (!PASS && mine && lane == 0) {
+            count[c.c] = cnt;
+            if (!small) atomicMax(most, cnt);
+        }
+        if (PASS && __syncthreads_or(!small) && !small && lane == 0) {
+            for (int a = 1; a < cnt; a++) {   // insertion sort in global memory
+                const int v = pairs[2 * (base + a) + 1];
+                int j = a - 1;
+                while (j >= 0 && pairs[2 * (base + j) + 1] > v) {
+                    pairs[2 * (base + j + 1) + 1] = pairs[2 * (base + j) + 1];
+                    j--;
+                }
+                pairs[2 * (base + j + 1) + 1] = v;
+                pairs[2 * (base + a)] = c.c;
+            }
+        }
+        __syncthreads();   // the group's counter and list are used again
     }
+}
+
+// the pairs of every cylinder from the neighbours that k_nl_tile<0> found (none has more than NL_HITS)
+__global__ void k_nl_emit(int n_cyl, const int* __restrict__ off, const int* __restrict__ found,
+                          int2* __restrict__ pairs) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= n_cyl) return;
+    const int o = off[c], cnt = off[c + 1] - o;
+    for (int a = 0; a < cnt; a++) pairs[o + a] = make_int2(c, found[(long)NL_HITS * c + a]);
+}
+
+// The counts that the host waits for between count and emission, into pinned host memory: the
+// pairs, the cylinders outside the grid (flags[0]), a cylinder's most neighbours if more than
+// NL_HITS (flags[1]) and, for each of ne + 1 boundary elements' bounds, the boundary interactions
+// before it.
+__global__ void k_nl_report(int nc, const int* __restrict__ off, const int* __restrict__ flags, int ne,
+                            const int* __restrict__ bnd_off, int* out) {
+    const int e = threadIdx.x;
+    if (e == 0) {
+        out[0] = off[nc];
+        out[1] = flags[0];
+        out[2] = flags[1];
+    }
+    for (int k = e; k <= ne && bnd_off; k += blockDim.x) out[3 + k] = bnd_off[(long)k * nc];
 }
 
 // HybridBindingSearchManager::updateAllPossibleBindingsstencilHYBD (HybridBindingSearchManager.cpp:
@@ -2107,6 +2171,7 @@ __global__ void k_bind_sites(NLDev n, BindDev b, const double* __restrict__ x, l
                              const int* __restrict__ pairs, int* __restrict__ count, const int* __restrict__ off,
                              uint32_t* __restrict__ out) {
     const long pi = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (!PASS && pi == n_pairs) count[pi] = 0;   // the counts' end, which the offsets' scan reads
     if (pi >= n_pairs) return;
     const int c = pairs[2 * pi], cn = pairs[2 * pi + 1];
     int cnt = 0;
@@ -2186,6 +2251,7 @@ __global__ void k_ev_vectorize(NLDev n, long n_pairs, const int* __restrict__ pa
 // interaction count (minus end adds its first bead, every cylinder its second bead)
 __global__ void k_bnd_count(NLDev n, DevSys s, double cutoff, const double* __restrict__ mid, int* __restrict__ cnt) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == (long)s.n_elem * n.n_cyl) cnt[i] = 0;   // the counts' end, which the offsets' scan reads
     if (i >= (long)s.n_elem * n.n_cyl) return;
     int e = (int)(i / n.n_cyl), c = (int)(i % n.n_cyl);
     D3 m{mid[3 * c], mid[3 * c + 1], mid[3 * c + 2]};
@@ -2256,58 +2322,63 @@ __global__ void k_load_forces(NLDev n, DevSys s, const double* __restrict__ x, c
 }
 
 // dynamic incidence lists: per bead, the excluded-volume and boundary slot ids, ascending
-__global__ void k_inc_count(DevSys s, int* __restrict__ cnt) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long nev = 4L * s.n[FF_EXVOL], nb = s.n[FF_BOUNDARY];
-    if (i < nev) atomicAdd(&cnt[s.ev_b[i]], 1);
-    else if (i < nev + nb) atomicAdd(&cnt[s.bnd_b[i - nev]], 1);
+__global__ void k_inc_static(int n_beads, const int* __restrict__ s_start, int* __restrict__ cnt) {
+    int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b <= n_beads) cnt[b] = b < n_beads ? s_start[b + 1] - s_start[b] : 0;
 }
-__global__ void k_inc_fill(DevSys s, const int* __restrict__ start, int* __restrict__ cursor, int* __restrict__ out) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long nev = 4L * s.n[FF_EXVOL], nb = s.n[FF_BOUNDARY];
+// the bead and the slot id of dynamic incidence i (excluded volume, then boundary)
+__device__ inline bool inc_dynamic(const DevSys& s, long i, int* bead, long* slot) {
+    const long nev = 4L * s.n[FF_EXVOL], nb = s.n[FF_BOUNDARY];
+    if (i >= nev + nb) return false;
+    *bead = i < nev ? s.ev_b[i] : s.bnd_b[i - nev];
+    *slot = i < nev ? s.slot0[FF_EXVOL] + i : s.slot0[FF_BOUNDARY] + (i - nev);
+    return true;
+}
+__global__ void k_inc_count(DevSys s, int* __restrict__ cnt) {
     int bead;
     long slot;
-    if (i < nev) { bead = s.ev_b[i]; slot = s.slot0[FF_EXVOL] + i; }
-    else if (i < nev + nb) { bead = s.bnd_b[i - nev]; slot = s.slot0[FF_BOUNDARY] + (i - nev); }
-    else return;
-    int k = atomicAdd(&cursor[bead], 1);
-    out[start[bead] + k] = (int)slot;
+    if (inc_dynamic(s, (long)blockIdx.x * blockDim.x + threadIdx.x, &bead, &slot)) atomicAdd(&cnt[bead], 1);
 }
-__global__ void k_inc_sort(int n_beads, const int* __restrict__ start, int* __restrict__ list) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_beads) return;
-    int lo = start[b], hi = start[b + 1];
-    for (int i = lo + 1; i < hi; i++) {
-        int v = list[i], j = i - 1;
-        while (j >= lo && list[j] > v) { list[j + 1] = list[j]; j--; }
-        list[j + 1] = v;
+// Bead-sorted layout: static slots then dynamic slots of each bead (static ids are smaller, so
+// the bead's range stays ascending); sorted_id[p] = slot id at p, pos[slot id] = p. k_inc_fill
+// places the static slots (by bead blocks, after the dynamic ones') and lists each bead's dynamic
+// ids in any order, counting cnt back down; k_inc_place places those by rank, one thread per
+// entry. With an insertion sort by one thread per bead (a bead in a dense spot has tens of entries)
+// and a scan and passes of its own for the dynamic part this took 73 us at 42,000 beads; now 16.
+__global__ void k_inc_fill(DevSys s, int dyn_blocks, const int* __restrict__ s_start, const int* __restrict__ s_list,
+                           const int* __restrict__ bstart, int* __restrict__ cnt, int* __restrict__ list,
+                           int* __restrict__ sorted_id, int* __restrict__ pos) {
+    int bead;
+    long slot;
+    if ((int)blockIdx.x < dyn_blocks) {
+        if (inc_dynamic(s, (long)blockIdx.x * blockDim.x + threadIdx.x, &bead, &slot))
+            list[bstart[bead] + atomicSub(&cnt[bead], 1) - 1] = (int)slot;
+        return;
     }
-}
-// per-bead slot count of the merged (static + dynamic) layout
-__global__ void k_inc_total(int n_beads, const int* __restrict__ s_start, const int* __restrict__ d_start,
-                            int* __restrict__ cnt) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_beads) return;
-    cnt[b] = (s_start[b + 1] - s_start[b]) + (d_start[b + 1] - d_start[b]);
-}
-// bead-sorted layout: static slots then dynamic slots of each bead (static ids are smaller, so
-// the bead's range stays ascending); sorted_id[p] = slot id at p, pos[slot id] = p
-__global__ void k_inc_merge(int n_beads, const int* __restrict__ s_start, const int* __restrict__ s_list,
-                            const int* __restrict__ d_start, const int* __restrict__ d_list,
-                            const int* __restrict__ bstart, int* __restrict__ sorted_id, int* __restrict__ pos) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_beads) return;
-    int p = bstart[b];
-    for (int q = s_start[b]; q < s_start[b + 1]; q++, p++) {
-        int id = s_list[q];
+    bead = (blockIdx.x - dyn_blocks) * blockDim.x + threadIdx.x;
+    if (bead >= s.n_beads) return;
+    int p = bstart[bead];
+    for (int q = s_start[bead]; q < s_start[bead + 1]; q++, p++) {
+        const int id = s_list[q];
+        list[p] = id;
         sorted_id[p] = id;
         pos[id] = p;
     }
-    for (int q = d_start[b]; q < d_start[b + 1]; q++, p++) {
-        int id = d_list[q];
-        sorted_id[p] = id;
-        pos[id] = p;
-    }
+}
+__global__ void k_inc_place(DevSys s, long total, const int* __restrict__ s_start, const int* __restrict__ bstart,
+                            const int* __restrict__ list, int* __restrict__ sorted_id, int* __restrict__ pos) {
+    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= total) return;
+    const int id = list[p];
+    int bead;
+    if (id >= s.slot0[FF_EXVOL] && id < s.slot0[FF_EXVOL + 1]) bead = s.ev_b[id - s.slot0[FF_EXVOL]];
+    else if (id >= s.slot0[FF_BOUNDARY] && id < s.slot0[FF_BOUNDARY + 1]) bead = s.bnd_b[id - s.slot0[FF_BOUNDARY]];
+    else return;   // static: placed
+    const int lo = bstart[bead] + (s_start[bead + 1] - s_start[bead]), hi = bstart[bead + 1];
+    int to = lo;
+    for (int q = lo; q < hi; q++) to += list[q] < id;
+    sorted_id[to] = id;
+    pos[id] = to;
 }
 
 }  // namespace mdn

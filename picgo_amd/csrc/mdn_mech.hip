@@ -105,7 +105,7 @@ struct mdn_ctx {
     int dof_next_n = -1;              // beads in dof_next (-1: none pending)
     DBuf<double> str_k, str_eql, bend_k, bend_eqt, lnk_k, lnk_eql, lnk_p1, lnk_p2, lnk_sf;
     DBuf<double> mot_k, mot_eql, mot_p1, mot_p2, mot_sf, ev_ks, bnd_krep, bnd_slen;
-    DBuf<int> inc_s_start, inc_s, inc_d_start, inc_d, inc_cnt, inc_cursor, bstart, sorted_id, pos;
+    DBuf<int> inc_s_start, inc_s, inc_cnt, inc_list, bstart, sorted_id, pos;
     DBuf<unsigned char> pmask;
     DBuf<int> bnbr, bterm;   // filament neighbours and term indices per bead (bonded_at_bead)
     DBuf<double> bsum;       // per-bead bonded sums, 3 * n_beads
@@ -126,14 +126,14 @@ struct mdn_ctx {
     DBuf<double> d_cyl_kexvol, d_cyl_eql, d_krep_e, d_slen_e;
     // NL workspace
     DBuf<double> mid;
-    DBuf<int> bin, bin_count, bin_start, bin_cursor, members, nl_count, nl_off, pairs, bnd_cnt, bnd_off;
+    DBuf<int> bin, bin_count, bin_start, place, nl_found, nl_count, nl_off, pairs, bnd_cnt, bnd_off;
     // the binding-site search's own list (mdn_binding_pairs) and its per-pair counts
     DBuf<double> b_mid, mmid, b_mmid;
-    DBuf<int> b_bin, b_bin_count, b_bin_start, b_bin_cursor, b_members, b_count, b_off, b_pairs, b_scount, b_soff;
+    DBuf<NlRec> members, b_members;
+    DBuf<int> b_bin, b_bin_count, b_bin_start, b_place, b_count, b_off, b_pairs, b_scount, b_soff;
     DBuf<int> mbin, b_mbin;
     DBuf<float> b_site, b_free;
     DBuf<uint32_t> b_out;
-    DBuf<int> nl_err;
     DBuf<unsigned char> cub_tmp;
     long n_pairs = 0;
     int n_bint = 0;
@@ -340,8 +340,11 @@ int ensure_eval_buffers(mdn_ctx* ctx) {
 }
 
 // The tile edge of the list kernel: the largest of 8, 4, 2 bins that still gives 1024 tiles (a
-// workgroup each), so that small grids keep the chip busy.
+// workgroup each), so that small grids keep the chip busy, and whose halo holds on average at most
+// half of what is staged in LDS: a halo beyond that is read from global memory, where a build took
+// three times as long (420,000 beads, T = 4 and 8 at twice the bin width: 420 and 1,250 us).
 void nl_tiles(NLDev& n) {
+    const double per_bin = n.n_cyl / ((double)n.nb[0] * n.nb[1] * n.nb[2]);
     for (int T = 8, lt = 3; T >= 2; T /= 2, lt--) {
         n.T = T;
         n.lt = lt;
@@ -350,8 +353,18 @@ void nl_tiles(NLDev& n) {
             n.nt[q] = (n.nb[q] + T - 1) / T;
             tiles *= n.nt[q];
         }
-        if (tiles >= 1024) break;
+        if (tiles >= 1024 && per_bin * (T + 2) * (T + 2) * (T + 2) <= NL_CAP / 2) break;
     }
+}
+
+// The bins of a list with n's range: 1.125 ranges wide (HybridNeighborListImpl.cpp:180).
+void nl_grid(mdn_ctx* ctx, NLDev& n) {
+    n.side = 1.125 * std::sqrt(n.rmaxsq);
+    for (int q = 0; q < 3; q++) {
+        n.grid[q] = ctx->grid[q];
+        n.nb[q] = std::max(1, (int)std::ceil(ctx->grid[q] / n.side));
+    }
+    nl_tiles(n);
 }
 
 NLDev nl_view(mdn_ctx* ctx) {
@@ -366,13 +379,8 @@ NLDev nl_view(mdn_ctx* ctx) {
     float rmaxsq = rmaxf * rmaxf, rminsq = rminf * rminf;
     n.rmaxsq = rmaxsq;
     n.rminsq = rminsq;
-    n.side = 1.125 * std::sqrt((double)rmaxsq);   // HybridNeighborListImpl.cpp:180
-    for (int q = 0; q < 3; q++) {
-        n.grid[q] = ctx->grid[q];
-        n.nb[q] = std::max(1, (int)std::ceil(ctx->grid[q] / n.side));
-    }
     n.ta = n.tb = -1;
-    nl_tiles(n);
+    nl_grid(ctx, n);
     return n;
 }
 
@@ -583,7 +591,7 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     if (ctx->ticket.ensure(8) != hipSuccess || ctx->eout.ensure(32) != hipSuccess ||
         ctx->vstat.ensure(2 * VSTAT_BLOCKS) != hipSuccess ||
         ctx->bad_count.ensure(1) != hipSuccess || ctx->cg.ensure(CG_BYTES / sizeof(CgState) + 1) != hipSuccess ||
-        ctx->nl_err.ensure(1) != hipSuccess || ctx->defer.ensure(DEFER_CAP) != hipSuccess ||
+        ctx->defer.ensure(DEFER_CAP) != hipSuccess ||
         ctx->defer_n.ensure(1) != hipSuccess) {
         delete ctx;
         return MDN_ERR_HIP;
@@ -604,14 +612,16 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
     }
     DBuf<int>* ib[] = {&ctx->str_b, &ctx->bend_b, &ctx->lnk_b, &ctx->mot_b, &ctx->lnk_ord, &ctx->mot_ord, &ctx->ev_b,
                        &ctx->bnd_b, &ctx->bnd_e,
-                       &ctx->inc_s_start, &ctx->inc_s, &ctx->inc_d_start, &ctx->inc_d, &ctx->inc_cnt,
-                       &ctx->inc_cursor, &ctx->d_cyl_b1, &ctx->d_cyl_b2, &ctx->d_cyl_fil, &ctx->d_cyl_pos,
-                       &ctx->d_cyl_type, &ctx->bin, &ctx->bin_count, &ctx->bin_start, &ctx->bin_cursor,
-                       &ctx->members, &ctx->nl_count, &ctx->nl_off, &ctx->pairs, &ctx->bnd_cnt, &ctx->bnd_off,
-                       &ctx->nl_err, &ctx->bad_count, &ctx->bad_list, &ctx->fallback_ok, &ctx->bstart,
+                       &ctx->inc_s_start, &ctx->inc_s, &ctx->inc_cnt, &ctx->inc_list,
+                       &ctx->d_cyl_b1, &ctx->d_cyl_b2, &ctx->d_cyl_fil, &ctx->d_cyl_pos,
+                       &ctx->d_cyl_type, &ctx->bin, &ctx->bin_count, &ctx->bin_start, &ctx->place,
+                       &ctx->nl_found, &ctx->nl_count, &ctx->nl_off, &ctx->pairs, &ctx->bnd_cnt, &ctx->bnd_off,
+                       &ctx->bad_count, &ctx->bad_list, &ctx->fallback_ok, &ctx->bstart,
                        &ctx->sorted_id, &ctx->pos, &ctx->dof_src, &ctx->b_bin, &ctx->b_bin_count,
-                       &ctx->b_bin_start, &ctx->b_bin_cursor, &ctx->b_members, &ctx->b_count, &ctx->b_off,
+                       &ctx->b_bin_start, &ctx->b_place, &ctx->b_count, &ctx->b_off,
                        &ctx->b_pairs, &ctx->b_scount, &ctx->b_soff};
+    ctx->members.release();
+    ctx->b_members.release();
     ctx->b_mid.release();
     ctx->mmid.release();
     ctx->b_mmid.release();
@@ -920,12 +930,6 @@ int mdn_system_upload(mdn_ctx* ctx, const mdn_system_desc* d, const double* coor
         for (size_t e = 0; e < ctx->elems.size(); e++) { ke[e] = ctx->elems[e].krep; se[e] = ctx->elems[e].slen; }
         HIPCHK(upload(ctx, ctx->d_krep_e, ke)); HIPCHK(upload(ctx, ctx->d_slen_e, se));
     }
-    // empty dynamic CSR until the neighbor lists are built
-    {
-        std::vector<int> z(ctx->n_beads + 1, 0);
-        HIPCHK(upload(ctx, ctx->inc_d_start, z));
-        HIPCHK(ctx->inc_d.ensure(1));
-    }
     // state vectors
     size_t nv = 3 * (size_t)ctx->n_beads;
     for (auto* b : {&ctx->x[0], &ctx->x[1], &ctx->f, &ctx->f2, &ctx->xh, &ctx->d[0], &ctx->d[1],
@@ -1059,9 +1063,9 @@ int mdn_get_coords(mdn_ctx* ctx, double* coord) {
     return MDN_OK;
 }
 
-// The block / slot layout for the current interaction counts, the dynamic incidence (excluded-
-// volume and boundary slots per bead, from the tables of the last neighbor-list build) and the
-// merged bead-sorted slot layout with the static crosslink incidence.
+// The block / slot layout for the current interaction counts and the bead-sorted slot layout: the
+// static crosslink incidence, then the excluded-volume and boundary slots from the tables of the
+// last neighbor-list build.
 int relayout(mdn_ctx* ctx) {
     int st = MDN_OK;
     const long np = ctx->sys.n[FF_EXVOL];
@@ -1069,34 +1073,24 @@ int relayout(mdn_ctx* ctx) {
     layout(ctx);
     if ((st = ensure_eval_buffers(ctx))) return st;
     refresh_ptrs(ctx);
-    // dynamic incidence CSR
     HIPCHK(ctx->inc_cnt.ensure(ctx->n_beads + 1));
-    HIPCHK(ctx->inc_cursor.ensure(ctx->n_beads + 1));
-    HIPCHK(ctx->inc_d_start.ensure(ctx->n_beads + 1));
-    const long ndyn = 4L * np + nbi;
-    HIPCHK(ctx->inc_d.ensure(std::max(1L, ndyn)));
-    HIPCHK(hipMemsetAsync(ctx->inc_cnt.p, 0, sizeof(int) * (ctx->n_beads + 1), ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->inc_cursor.p, 0, sizeof(int) * (ctx->n_beads + 1), ctx->stream));
-    refresh_ptrs(ctx);
-    if (ndyn > 0)
-        hipLaunchKernelGGL(k_inc_count, dim3(ceil_div(ndyn, BLOCK)), dim3(BLOCK), 0, ctx->stream, ctx->sys,
-                           ctx->inc_cnt.p);
-    if ((st = exclusive_scan(ctx, ctx->inc_cnt.p, ctx->inc_d_start.p, ctx->n_beads + 1))) return st;
-    if (ndyn > 0) {
-        hipLaunchKernelGGL(k_inc_fill, dim3(ceil_div(ndyn, BLOCK)), dim3(BLOCK), 0, ctx->stream, ctx->sys,
-                           ctx->inc_d_start.p, ctx->inc_cursor.p, ctx->inc_d.p);
-        hipLaunchKernelGGL(k_inc_sort, dim3(bead_blocks(ctx)), dim3(BLOCK), 0, ctx->stream, ctx->n_beads,
-                           ctx->inc_d_start.p, ctx->inc_d.p);
-    }
-    // bead-sorted slot layout (static then dynamic slots of each bead)
     HIPCHK(ctx->bstart.ensure(ctx->n_beads + 1));
-    hipLaunchKernelGGL(k_inc_total, dim3(bead_blocks(ctx)), dim3(BLOCK), 0, ctx->stream, ctx->n_beads,
-                       ctx->inc_s_start.p, ctx->inc_d_start.p, ctx->inc_cnt.p);
-    HIPCHK(hipMemsetAsync(ctx->inc_cnt.p + ctx->n_beads, 0, sizeof(int), ctx->stream));
+    const long ndyn = 4L * np + nbi, total = ctx->sys.slot0[NFF];
+    HIPCHK(ctx->inc_list.ensure((size_t)std::max(1L, total)));
+    refresh_ptrs(ctx);
+    const int dyn_blocks = ceil_div(ndyn, BLOCK), bb = bead_blocks(ctx);
+    hipLaunchKernelGGL(k_inc_static, dim3(ceil_div(ctx->n_beads + 1, BLOCK)), dim3(BLOCK), 0, ctx->stream, ctx->n_beads,
+                       (const int*)ctx->inc_s_start.p, ctx->inc_cnt.p);
+    if (ndyn > 0)
+        hipLaunchKernelGGL(k_inc_count, dim3(dyn_blocks), dim3(BLOCK), 0, ctx->stream, ctx->sys, ctx->inc_cnt.p);
     if ((st = exclusive_scan(ctx, ctx->inc_cnt.p, ctx->bstart.p, ctx->n_beads + 1))) return st;
-    hipLaunchKernelGGL(k_inc_merge, dim3(bead_blocks(ctx)), dim3(BLOCK), 0, ctx->stream, ctx->n_beads,
-                       ctx->inc_s_start.p, ctx->inc_s.p, ctx->inc_d_start.p, ctx->inc_d.p, ctx->bstart.p,
-                       ctx->sorted_id.p, ctx->pos.p);
+    hipLaunchKernelGGL(k_inc_fill, dim3(dyn_blocks + bb), dim3(BLOCK), 0, ctx->stream, ctx->sys, dyn_blocks,
+                       (const int*)ctx->inc_s_start.p, (const int*)ctx->inc_s.p, (const int*)ctx->bstart.p,
+                       ctx->inc_cnt.p, ctx->inc_list.p, ctx->sorted_id.p, ctx->pos.p);
+    if (ndyn > 0)
+        hipLaunchKernelGGL(k_inc_place, dim3(ceil_div(total, BLOCK)), dim3(BLOCK), 0, ctx->stream, ctx->sys, total,
+                           (const int*)ctx->inc_s_start.p, (const int*)ctx->bstart.p, (const int*)ctx->inc_list.p,
+                           ctx->sorted_id.p, ctx->pos.p);
     HIPCHK(hipGetLastError());
     refresh_ptrs(ctx);
     ctx->sys_gen++;
@@ -1107,48 +1101,56 @@ int relayout(mdn_ctx* ctx) {
 // and offsets, the pair array).
 struct NlBufs {
     DBuf<double>& mid;
-    DBuf<int>& bin; DBuf<int>& bin_count; DBuf<int>& bin_start; DBuf<int>& bin_cursor; DBuf<int>& members;
+    DBuf<int>& bin; DBuf<int>& bin_count; DBuf<int>& bin_start; DBuf<int>& place; DBuf<NlRec>& members;
     DBuf<int>& count; DBuf<int>& off; DBuf<int>& pairs;
     DBuf<int>& mbin; DBuf<double>& mmid;   // each member's bin and midpoint, in bin order
 };
 
 // HybridCylinderCylinderNL::reset for one list: midpoints, counting sort into bins, the
-// 27-bin stencil (count, scan, emit, per-cylinder sort). *np = the pairs, ordered by cylinder
-// then neighbour.
-static int build_pairs(mdn_ctx* ctx, const NLDev& n, const double* x, NlBufs& B, long* np, const char* what) {
+// 27-bin stencil (count, scan, emit in order). Queued; the pairs are counted in B.off[n_cyl], the
+// flags of k_nl_report follow the bins' counts.
+static long nl_tile_count(const NLDev& n) { return (long)n.nt[0] * n.nt[1] * n.nt[2]; }
+static long nl_flags(const NLDev& n) { return nl_tile_count(n) * n.T * n.T * n.T + 1; }   // in bin_count
+static int count_pairs(mdn_ctx* ctx, const NLDev& n, const double* x, NlBufs& B) {
     int st = MDN_OK;
-    const long ntiles = (long)n.nt[0] * n.nt[1] * n.nt[2];
-    const long nbins = ntiles * n.T * n.T * n.T;   // tile by tile, the last tiles padded
+    const long nbins = nl_flags(n) - 1;   // tile by tile, the last tiles padded
     if (nbins > (1L << 30)) return fail(ctx, MDN_ERR_UNSUPPORTED, "neighbor-list grid too large (%ld bins)", nbins);
     const int nc = n.n_cyl;
-    HIPCHK(B.mid.ensure(3 * (size_t)std::max(1, nc)));
-    HIPCHK(B.bin.ensure(std::max(1, nc)));
-    HIPCHK(B.bin_count.ensure(nbins + 1));
+    const size_t n1 = std::max(1, nc);
+    HIPCHK(B.mid.ensure(3 * n1));
+    HIPCHK(B.bin.ensure(n1));
+    HIPCHK(B.bin_count.ensure(nbins + 3));
     HIPCHK(B.bin_start.ensure(nbins + 1));
-    HIPCHK(B.bin_cursor.ensure(nbins + 1));
-    HIPCHK(B.members.ensure(std::max(1, nc)));
-    HIPCHK(B.mbin.ensure(std::max(1, nc)));
-    HIPCHK(B.mmid.ensure(3 * (size_t)std::max(1, nc)));
+    HIPCHK(B.place.ensure(n1));
+    HIPCHK(B.members.ensure(n1));
+    HIPCHK(B.mbin.ensure(n1));
+    HIPCHK(B.mmid.ensure(3 * n1));
     HIPCHK(B.count.ensure(nc + 1));
     HIPCHK(B.off.ensure(nc + 1));
-    HIPCHK(hipMemsetAsync(B.bin_count.p, 0, sizeof(int) * (nbins + 1), ctx->stream));
-    HIPCHK(hipMemsetAsync(B.bin_cursor.p, 0, sizeof(int) * (nbins + 1), ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->nl_err.p, 0, sizeof(int), ctx->stream));
-    const int G = std::max(1, ceil_div(nc, BLOCK));
-    hipLaunchKernelGGL(k_nl_bin, dim3(G), dim3(BLOCK), 0, ctx->stream, n, x, B.mid.p, B.bin.p, B.bin_count.p,
-                       ctx->nl_err.p);
+    HIPCHK(ctx->nl_found.ensure(NL_HITS * n1));
+    HIPCHK(hipMemsetAsync(B.bin_count.p, 0, sizeof(int) * (nbins + 3), ctx->stream));
+    int* flags = B.bin_count.p + nl_flags(n);
+    hipLaunchKernelGGL(k_nl_bin, dim3(ceil_div(nc + 1, BLOCK)), dim3(BLOCK), 0, ctx->stream, n, x, B.mid.p, B.bin.p,
+                       B.place.p, B.bin_count.p, flags, B.count.p);
     HIPCHK(hipGetLastError());
     if ((st = exclusive_scan(ctx, B.bin_count.p, B.bin_start.p, nbins + 1))) return st;
-    hipLaunchKernelGGL(k_nl_fill, dim3(G), dim3(BLOCK), 0, ctx->stream, nc, B.bin.p, B.bin_start.p, B.bin_cursor.p,
-                       (const double*)B.mid.p, B.members.p, B.mbin.p, B.mmid.p);
-    hipLaunchKernelGGL(k_nl_tile<0>, dim3(ntiles), dim3(BLOCK), 0, ctx->stream, n, (const int*)B.bin_start.p,
-                       (const int*)B.members.p, (const int*)B.mbin.p, (const double*)B.mmid.p, B.count.p,
-                       (const int*)nullptr, (int*)nullptr);
+    hipLaunchKernelGGL(k_nl_fill, dim3(ceil_div(n1, BLOCK)), dim3(BLOCK), 0, ctx->stream, n, B.bin.p, B.bin_start.p,
+                       (const int*)B.place.p, (const double*)B.mid.p, B.members.p, B.mbin.p, B.mmid.p);
+    hipLaunchKernelGGL(k_nl_tile<0>, dim3(nl_tile_count(n)), dim3(BLOCK), 0, ctx->stream, n, (const int*)B.bin_start.p,
+                       (const NlRec*)B.members.p, (const int*)B.mbin.p, (const double*)B.mmid.p, B.count.p, flags + 1,
+                       ctx->nl_found.p, (const int*)nullptr, (int*)nullptr);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemsetAsync(B.count.p + nc, 0, sizeof(int), ctx->stream));
-    if ((st = exclusive_scan(ctx, B.count.p, B.off.p, nc + 1))) return st;
-    HIPCHK(hipMemcpyAsync(ctx->h_int, B.off.p + nc, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(ctx->h_int + 1, ctx->nl_err.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    return exclusive_scan(ctx, B.count.p, B.off.p, nc + 1);
+}
+// After count_pairs: one wait for the counts (with the boundary interactions before each of ne + 1
+// element bounds, from their offsets, if given), then the pairs, ordered by cylinder then
+// neighbour (queued). *np = the pairs.
+static int emit_pairs(mdn_ctx* ctx, const NLDev& n, NlBufs& B, int ne, const int* bnd_off, long* np, const char* what) {
+    const int nc = n.n_cyl;
+    int* flags = B.bin_count.p + nl_flags(n);
+    hipLaunchKernelGGL(k_nl_report, dim3(1), dim3(64), 0, ctx->stream, nc, (const int*)B.off.p, (const int*)flags, ne,
+                       bnd_off, ctx->h_int);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->h_int[1] != 0) {
         return fail(ctx, MDN_ERR_NL_BOUNDS, "%d cylinder midpoints outside the neighbor-list grid [0, %g)x[0, %g)x[0, %g)",
@@ -1157,9 +1159,14 @@ static int build_pairs(mdn_ctx* ctx, const NLDev& n, const double* x, NlBufs& B,
     *np = ctx->h_int[0];
     if (*np > 0x7fffffffL / 4) return fail(ctx, MDN_ERR_UNSUPPORTED, "too many %s pairs (%ld)", what, *np);
     HIPCHK(B.pairs.ensure(2 * (size_t)std::max(1L, *np)));
-    hipLaunchKernelGGL(k_nl_tile<1>, dim3(ntiles), dim3(BLOCK), 0, ctx->stream, n, (const int*)B.bin_start.p,
-                       (const int*)B.members.p, (const int*)B.mbin.p, (const double*)B.mmid.p, B.count.p,
-                       (const int*)B.off.p, B.pairs.p);
+    if (ctx->h_int[2] == 0)
+        hipLaunchKernelGGL(k_nl_emit, dim3(std::max(1, ceil_div(nc, BLOCK))), dim3(BLOCK), 0, ctx->stream, nc,
+                           (const int*)B.off.p, (const int*)ctx->nl_found.p, (int2*)B.pairs.p);
+    else
+        hipLaunchKernelGGL(k_nl_tile<1>, dim3(nl_tile_count(n)), dim3(BLOCK), 0, ctx->stream, n,
+                           (const int*)B.bin_start.p, (const NlRec*)B.members.p, (const int*)B.mbin.p,
+                           (const double*)B.mmid.p, B.count.p, flags + 1, ctx->nl_found.p, (const int*)B.off.p,
+                           B.pairs.p);
     HIPCHK(hipGetLastError());
     return MDN_OK;
 }
@@ -1177,11 +1184,24 @@ int mdn_nl_build(mdn_ctx* ctx, const double* coord, int64_t* n_pairs_out) {
     NLDev n = nl_view(ctx);
     const int nc = ctx->n_cyl;
     long np = 0;
-    {
-        NlBufs B{ctx->mid, ctx->bin, ctx->bin_count, ctx->bin_start, ctx->bin_cursor, ctx->members,
-                 ctx->nl_count, ctx->nl_off, ctx->pairs, ctx->mbin, ctx->mmid};
-        if ((st = build_pairs(ctx, n, x, B, &np, "excluded-volume"))) return st;
-    }
+    NlBufs B{ctx->mid, ctx->bin, ctx->bin_count, ctx->bin_start, ctx->place, ctx->members,
+             ctx->nl_count, ctx->nl_off, ctx->pairs, ctx->mbin, ctx->mmid};
+    if ((st = count_pairs(ctx, n, x, B))) return st;
+    // boundary NL (BoundaryCylinderRepulsion::vectorize): counted before the one wait for both
+    const int ne = (int)ctx->elems.size();
+    const long nbc = (long)ne * nc;
+    ctx->sys.n_elem = ne;
+    HIPCHK(ctx->bnd_cnt.ensure(nbc + 1));
+    HIPCHK(ctx->bnd_off.ensure(nbc + 1));
+    hipLaunchKernelGGL(k_bnd_count, dim3(ceil_div(nbc + 1, BLOCK)), dim3(BLOCK), 0, ctx->stream, n, ctx->sys,
+                       ctx->bnd_cutoff, ctx->mid.p, ctx->bnd_cnt.p);
+    if ((st = exclusive_scan(ctx, ctx->bnd_cnt.p, ctx->bnd_off.p, nbc + 1))) return st;
+    if ((st = emit_pairs(ctx, n, B, ne, ctx->bnd_off.p, &np, "excluded-volume"))) return st;
+    // per-element counts (nneighbors) come from the offsets at element boundaries
+    const int* eoff = ctx->h_int + 3;
+    const int nbi = eoff[ne];
+    ctx->bnd_nneighbors.assign(ne, 0);
+    for (int e = 0; e < ne; e++) ctx->bnd_nneighbors[e] = eoff[e + 1] - eoff[e];
     // CylinderExclVolume::vectorize
     HIPCHK(ctx->ev_b.ensure(4 * (size_t)std::max(1L, np)));
     HIPCHK(ctx->ev_ks.ensure((size_t)std::max(1L, np)));
@@ -1189,26 +1209,6 @@ int mdn_nl_build(mdn_ctx* ctx, const double* coord, int64_t* n_pairs_out) {
         hipLaunchKernelGGL(k_ev_vectorize, dim3(ceil_div(np, BLOCK)), dim3(BLOCK), 0, ctx->stream, n, np,
                            ctx->pairs.p, ctx->ev_b.p, ctx->ev_ks.p);
     ctx->n_pairs = np;
-    // boundary NL + BoundaryCylinderRepulsion::vectorize
-    const int ne = (int)ctx->elems.size();
-    const long nbc = (long)ne * nc;
-    ctx->sys.n_elem = ne;
-    HIPCHK(ctx->bnd_cnt.ensure(nbc + 1));
-    HIPCHK(ctx->bnd_off.ensure(nbc + 1));
-    if (nbc > 0)
-        hipLaunchKernelGGL(k_bnd_count, dim3(ceil_div(nbc, BLOCK)), dim3(BLOCK), 0, ctx->stream, n, ctx->sys,
-                           ctx->bnd_cutoff, ctx->mid.p, ctx->bnd_cnt.p);
-    HIPCHK(hipMemsetAsync(ctx->bnd_cnt.p + nbc, 0, sizeof(int), ctx->stream));
-    if ((st = exclusive_scan(ctx, ctx->bnd_cnt.p, ctx->bnd_off.p, nbc + 1))) return st;
-    HIPCHK(hipMemcpyAsync(ctx->h_int, ctx->bnd_off.p + nbc, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    // per-element counts (nneighbors) come from the offsets at element boundaries
-    std::vector<int> eoff(ne + 1, 0);
-    for (int e = 0; e <= ne; e++)
-        HIPCHK(hipMemcpyAsync(&eoff[e], ctx->bnd_off.p + (long)e * nc, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    const int nbi = ctx->h_int[0];
-    ctx->bnd_nneighbors.assign(ne, 0);
-    for (int e = 0; e < ne; e++) ctx->bnd_nneighbors[e] = eoff[e + 1] - eoff[e];
     HIPCHK(ctx->bnd_b.ensure(std::max(1, nbi)));
     HIPCHK(ctx->bnd_e.ensure(std::max(1, nbi)));
     HIPCHK(ctx->bnd_krep.ensure(std::max(1, nbi)));
@@ -1300,17 +1300,21 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     NLDev n = nl_view(ctx);
     n.rmaxsq = rmax_l * rmax_l;
     n.rminsq = rmin_l * rmin_l;
-    n.side = 1.125 * std::sqrt(n.rmaxsq);
-    for (int q = 0; q < 3; q++) n.nb[q] = std::max(1, (int)std::ceil(ctx->grid[q] / n.side));
-    nl_tiles(n);
+    nl_grid(ctx, n);
     n.ta = std::min(p->ftype1, p->ftype2);
     n.tb = std::max(p->ftype1, p->ftype2);
-    long np = 0;
-    {
-        NlBufs B{ctx->b_mid, ctx->b_bin, ctx->b_bin_count, ctx->b_bin_start, ctx->b_bin_cursor, ctx->b_members,
-                 ctx->b_count, ctx->b_off, ctx->b_pairs, ctx->b_mbin, ctx->b_mmid};
-        if ((st = build_pairs(ctx, n, x, B, &np, "binding-list"))) return st;
+    HIPCHK(ctx->b_site.ensure(p->n_sites));
+    HIPCHK(hipMemcpyAsync(ctx->b_site.p, p->site_pos, sizeof(float) * p->n_sites, hipMemcpyHostToDevice, ctx->stream));
+    if (p->site_free) {
+        const size_t nf = (size_t)ctx->n_cyl * p->n_sites;
+        HIPCHK(ctx->b_free.ensure(std::max<size_t>(1, nf)));
+        HIPCHK(hipMemcpyAsync(ctx->b_free.p, p->site_free, sizeof(float) * nf, hipMemcpyHostToDevice, ctx->stream));
     }
+    long np = 0;
+    NlBufs B{ctx->b_mid, ctx->b_bin, ctx->b_bin_count, ctx->b_bin_start, ctx->b_place, ctx->b_members,
+             ctx->b_count, ctx->b_off, ctx->b_pairs, ctx->b_mbin, ctx->b_mmid};
+    if ((st = count_pairs(ctx, n, x, B))) return st;
+    if ((st = emit_pairs(ctx, n, B, 0, nullptr, &np, "binding-list"))) return st;
     BindDev b{};
     b.n_sites = p->n_sites;
     b.shift = p->shift_bits;
@@ -1321,24 +1325,14 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     b.rmaxsq = rmaxsq_b;
     b.p2_first = p->p2_first;
     b.p2_last = p->p2_last;
-    {
-        std::vector<float> site(p->site_pos, p->site_pos + p->n_sites);
-        HIPCHK(upload(ctx, ctx->b_site, site));
-        if (p->site_free) {
-            std::vector<float> fr(p->site_free, p->site_free + (size_t)ctx->n_cyl * p->n_sites);
-            HIPCHK(upload(ctx, ctx->b_free, fr));
-        }
-        HIPCHK(hipStreamSynchronize(ctx->stream));   // the host vectors end with this scope
-    }
     b.site = ctx->b_site.p;
     b.free = p->site_free ? ctx->b_free.p : nullptr;
     HIPCHK(ctx->b_scount.ensure(np + 1));
     HIPCHK(ctx->b_soff.ensure(np + 1));
-    const int G = std::max(1, ceil_div(np, BLOCK));
+    const int G = ceil_div(np + 1, BLOCK);
     hipLaunchKernelGGL(k_bind_sites<0>, dim3(G), dim3(BLOCK), 0, ctx->stream, n, b, x, np, (const int*)ctx->b_pairs.p,
                        ctx->b_scount.p, (const int*)nullptr, (uint32_t*)nullptr);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemsetAsync(ctx->b_scount.p + np, 0, sizeof(int), ctx->stream));
     if ((st = exclusive_scan(ctx, ctx->b_scount.p, ctx->b_soff.p, np + 1))) return st;
     HIPCHK(d2h(ctx, ctx->h_int, ctx->b_soff.p + np, sizeof(int)));
     const long total = ctx->h_int[0];
