@@ -181,6 +181,14 @@ __device__ inline int ff_of_block(const DevSys& s, int b) {
     return k < NFF ? s.dff[k] : NFF;   // NFF means a bead block
 }
 
+// The FP64 line search evaluates the excluded-volume forces in blocks of their own, ahead of the
+// interaction blocks, whose excluded-volume blocks then take the energies alone: the two chains run
+// side by side instead of one after the other (term_ef says why the mixed path does not).
+template <typename R>
+__device__ __host__ inline int ev_force_blocks(const DevSys& s) {
+    return sizeof(R) == 8 ? (s.n[FF_EXVOL] + BLOCK - 1) / BLOCK : 0;
+}
+
 // ---- deterministic reduction helpers (64-wide waves) ----------------------------------
 // A wave reduction in six DPP steps on the VALU (no LDS traffic): row shifts by 1, 2, 4 and 8
 // leave each 16-lane row's total in its lane 15, row_bcast:15 adds row 0's total into row 1 and
@@ -362,11 +370,12 @@ __device__ inline void push_defer(const DevSys& s, int code, int t, D3 c1, D3 c2
 // form divides a bracket that vanishes like the squared triple product of the pair by that
 // square, so FP32 rounding is amplified like 1/tau^2 for near-coplanar pairs (tau the normalized
 // triple product), and FP32 gains nothing on gfx950 for this latency-bound term.
-// SPLIT: an excluded-volume pair's energy and forces by two calls, each forming the pair's
-// invariants: more arithmetic, fewer registers live at once, for kernels whose register budget
-// the shared form overflows. The FP64 path's values are the same bit for bit; the mixed path's
-// FMA-contracted forms may fuse differently in the other context (differences at rounding level).
-template <typename R, bool SPLIT = false>
+// The FP64 path evaluates an excluded-volume pair for its forces (code < 0, into the slots) or for
+// its energy (code >= 0), never for both at once: each is one long chain of FP64 operations, and
+// the forces of a near-coplanar pair take other invariants than its energy. The mixed path takes
+// both in one call where both are wanted: its FMA-contracted forms fuse differently in separate
+// code (differences at rounding level, which a minimization amplifies).
+template <typename R>
 __device__ inline double term_ef(const DevSys& s, int ff, int t, const Pos& p, R* __restrict__ slots,
                                  int code, int* fbad, int* bad_t = nullptr) {
     D3 out[4];
@@ -418,24 +427,15 @@ __device__ inline double term_ef(const DevSys& s, int ff, int t, const Pos& p, R
         constexpr bool fast = sizeof(R) == 4;
         int deferred = 0;
         double U = 0.0;
-        if (slots) {
+        if (fast ? slots != nullptr : code < 0) {
             bool ok = true;
-            if (fast) {
-                if (code < 0) {
-                    ok = exvol_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], out);
-                } else if (SPLIT) {
-                    U = exvol_energy_fast(c1, c2, c3, c4, s.ev_ks[tp], &deferred);
-                    ok = exvol_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], out);
-                } else {
-                    U = exvol_energy_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], &deferred, &ok, out);
-                }
+            if (!fast) {
+                ok = exvol_forces<double>(c1, c2, c3, c4, s.ev_ks[tp], out);
             } else if (code < 0) {
-                ok = exvol_forces<double>(c1, c2, c3, c4, s.ev_ks[tp], out);
-            } else if (SPLIT) {
-                U = exvol_energy<double>(c1, c2, c3, c4, s.ev_ks[tp], &deferred);
-                ok = exvol_forces<double>(c1, c2, c3, c4, s.ev_ks[tp], out);
+                ok = exvol_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], out);
             } else {
-                U = exvol_energy_forces<double>(c1, c2, c3, c4, s.ev_ks[tp], &deferred, &ok, out);
+                U = exvol_energy_fast(c1, c2, c3, c4, s.ev_ks[tp], &deferred);
+                ok = exvol_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], out);
             }
             if (!ok) {
                 out[0] = out[1] = out[2] = out[3] = D3{0.0, 0.0, 0.0};
@@ -1201,9 +1201,12 @@ __device__ inline void bead_ls(const DevSys& s, const CgBufs& B, int j, bool mov
 }
 
 // ---- line search, interaction part: trial energies, speculative forces -----------------
-// Grid: the interaction blocks. Phase PH_LS: E(lambda) with its forces at x_next (into the
-// slots), E(lambda / 2) at x_half after a rejection, E(x) when the current energy is not known;
-// block partials E(lambda), E(lambda / 2), E(x). Phase PH_MOVE: the forces at x_next.
+// Grid: the excluded-volume force blocks, the interaction blocks, the bead blocks. Phase PH_LS:
+// E(lambda) with its forces at x_next (into the slots), E(lambda / 2) at x_half after a rejection,
+// E(x) when the current energy is not known; block partials E(lambda), E(lambda / 2), E(x). Phase
+// PH_MOVE: the forces at x_next. Bound by the FP64 chain of one excluded-volume pair where the
+// blocks are fewer than the chip holds: with a pair's energy and forces in one thread an
+// FP64 minimization took 3068 us at 42,000 beads and 1630 at 550 (by a team), now 2930 and 1432.
 // 3 waves per SIMD (at most 168 VGPRs) measured faster than the unconstrained 2.
 template <typename R>
 __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __restrict__ st, CgBufs B) {
@@ -1216,23 +1219,37 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     if (phase != PH_LS && phase != PH_MOVE) return;
     const bool first = ls_active == 0;
     const bool need_e0 = first && !ecur_valid;
-    // with bonded_gather bead blocks follow the interaction blocks and carry the filament terms'
+    // the excluded-volume pairs' forces come first, in blocks of their own (ev_force_blocks); then
+    // the interaction blocks; with bonded_gather bead blocks follow and carry the filament terms'
     // forces (and, with bead_energy, their energies: then the filament terms' blocks are left out)
+    const int nevf = ev_force_blocks<R>(s);
     const int nint = (s.bonded_gather && s.bead_energy) ? s.blk_nb : s.blk[NFF];
-    if ((int)blockIdx.x >= nint) {   // (or the one block of a grid without interactions)
-        if (s.bonded_gather)
-            bead_ls<R>(s, B, blockIdx.x - nint, phase == PH_MOVE, first, need_e0, par, s.bead_energy != 0, lds);
-        return;
-    }
-    const int ff = ff_of_block(s, blockIdx.x);
-    const int t = (blockIdx.x - s.fblk[ff]) * BLOCK + threadIdx.x;
+    const int blk = (int)blockIdx.x - nevf;
     const double* __restrict__ xn = B.x[par ^ 1];
     const Pos p1{xn, nullptr, nullptr, 0.0, 0.0, 0};
-    // with bonded_gather (and not bead_energy) the filament terms' blocks take energies only
-    const bool bonded_e = s.bonded_gather && (ff == FF_STRETCH || ff == FF_BEND);
-    R* const tslots = bonded_e ? nullptr : static_cast<R*>(B.slots);
+    R* const slots = static_cast<R*>(B.slots);
+    if (blk < 0) {
+        const int t = blockIdx.x * BLOCK + threadIdx.x;
+        if (t < s.n[FF_EXVOL]) {
+            int fbad = 0;
+            (void)term_ef<R>(s, FF_EXVOL, t, p1, slots, -1, &fbad);
+            if (fbad) atomicAdd(B.bad_count, 1);
+        }
+        return;
+    }
+    if (blk >= nint) {   // (or the one block of a grid without interactions)
+        if (s.bonded_gather)
+            bead_ls<R>(s, B, blk - nint, phase == PH_MOVE, first, need_e0, par, s.bead_energy != 0, lds);
+        return;
+    }
+    const int ff = ff_of_block(s, blk);
+    const int t = (blk - s.fblk[ff]) * BLOCK + threadIdx.x;
+    // FP64 excluded volume and, with bonded_gather (and not bead_energy), the filament terms:
+    // energies only
+    const bool only_e = (nevf > 0 && ff == FF_EXVOL) || (s.bonded_gather && (ff == FF_STRETCH || ff == FF_BEND));
+    R* const tslots = only_e ? nullptr : slots;
     if (phase == PH_MOVE) {
-        if (t < s.n[ff] && !bonded_e) {
+        if (t < s.n[ff] && !only_e) {
             int fbad = 0;
             (void)term_ef<R>(s, ff, t, p1, tslots, -1, &fbad);
             if (fbad) atomicAdd(B.bad_count, 1);
@@ -1242,7 +1259,7 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     double v[3] = {0.0, 0.0, 0.0};
     if (t < s.n[ff]) {
         int fbad = 0;
-        v[0] = term_ef<R, true>(s, ff, t, p1, tslots, 0, &fbad);   // split: no register spills at 3 waves
+        v[0] = term_ef<R>(s, ff, t, p1, tslots, 0, &fbad);
         if (fbad) atomicAdd(B.bad_count, 1);
         if (!first) {   // the first launch of a search evaluates lambda0 alone (see ls_control)
             const Pos p2{B.xh, nullptr, nullptr, 0.0, 0.0, 0};
@@ -1256,7 +1273,7 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     const int op3[3] = {0, 0, 0};
     block_reduce_n<3>(v, op3, lds);
     if (threadIdx.x == 0) {
-        const long np = s.lsp, k = blockIdx.x;   // value-major
+        const long np = s.lsp, k = blk;   // value-major
         B.partial[k] = v[0];
         B.partial[np + k] = v[1];
         B.partial[2 * np + k] = v[2];

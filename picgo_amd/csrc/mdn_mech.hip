@@ -1786,9 +1786,10 @@ template <typename R>
 static void launch_slot(mdn_ctx* ctx, const DevSys& s, const CgBufs& B) {
     const int gbk = gather_blocks(ctx);
     hipLaunchKernelGGL(k_cg_pos, dim3(bead_blocks(ctx)), dim3(BLOCK), 0, ctx->stream, s, (const CgState*)ctx->cg.p, B);
-    // all interaction blocks, then (bonded_gather) the bead blocks; with bead_energy the filament
-    // terms' blocks are left out
-    const int lsg = s.bonded_gather ? (s.bead_energy ? s.blk_nb : s.blk[NFF]) + s.nbb : s.blk[NFF];
+    // the excluded-volume force blocks, all interaction blocks, then (bonded_gather) the bead blocks;
+    // with bead_energy the filament terms' blocks are left out
+    const int lsg = ev_force_blocks<R>(s) +
+                    (s.bonded_gather ? (s.bead_energy ? s.blk_nb : s.blk[NFF]) + s.nbb : s.blk[NFF]);
     hipLaunchKernelGGL(k_cg_ls<R>, dim3(std::max(1, lsg)), dim3(BLOCK), 0, ctx->stream, s,
                        (const CgState*)ctx->cg.p, B);
     launch_cg_gather<R>(ctx, s, (const CgState*)ctx->cg.p, B);

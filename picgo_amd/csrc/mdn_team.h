@@ -206,7 +206,7 @@ __device__ inline void team_ls(const DevSys& s, const CgBufs& B, const CgState& 
     const bool need_e0 = !move && first && !S.ecur_valid, need_half = !move && !first;
     const int par = S.parity, T = s.blk[NFF];
     const bool be = s.bead_energy != 0;
-    const int nint = be ? s.blk_nb : T, total = 4 * (nint + s.nbb);
+    const int nint = be ? s.blk_nb : T, nevf = 4 * ev_force_blocks<R>(s), total = nevf + 4 * (nint + s.nbb);
     const long nc = SUM == SUM_STRIDED ? team_items(s) : 4L * (T + s.nbb);   // entries per value
     const double* __restrict__ xn = B.x[par ^ 1];
     const Pos p1{xn, nullptr, nullptr, 0.0, 0.0, 0};
@@ -214,7 +214,17 @@ __device__ inline void team_ls(const DevSys& s, const CgBufs& B, const CgState& 
     const Pos p0{B.x[par], nullptr, nullptr, 0.0, 0.0, 0};
     R* const slots = static_cast<R*>(B.slots);
     for (int iv = t.gw; iv < total; iv += t.nw) {
-        const int i = __builtin_amdgcn_readfirstlane(iv);
+        const int iw = __builtin_amdgcn_readfirstlane(iv);
+        if (iw < nevf) {   // an excluded-volume force block
+            const int q = 64 * iw + lane;
+            if (q < s.n[FF_EXVOL]) {
+                int fbad = 0;
+                (void)term_ef<R>(s, FF_EXVOL, q, p1, slots, -1, &fbad);
+                if (fbad) atomicAdd(B.bad_count, 1);
+            }
+            continue;
+        }
+        const int i = iw - nevf;
         const int blk = i >> 2;
         double v[3] = {0.0, 0.0, 0.0};
         long col = i, item = -1;
@@ -236,15 +246,16 @@ __device__ inline void team_ls(const DevSys& s, const CgBufs& B, const CgState& 
         } else {
             const int ff = ff_of_block(s, blk);
             const int q = (blk - s.fblk[ff]) * BLOCK + 64 * (i & 3) + lane;
-            const bool bonded = ff == FF_STRETCH || ff == FF_BEND;   // energies only: the bead blocks hold the forces
+            // energies only: the bead blocks or the blocks above hold the forces
+            const bool only_e = ff == FF_STRETCH || ff == FF_BEND || (nevf > 0 && ff == FF_EXVOL);
             if (q < s.n[ff]) {
                 item = q + (ff > FF_LINKER ? s.n[FF_LINKER] : 0) + (ff > FF_MOTOR ? s.n[FF_MOTOR] : 0) +
                        (ff > FF_EXVOL ? s.n[FF_EXVOL] : 0);
                 int fbad = 0;
                 if (move) {
-                    if (!bonded) (void)term_ef<R>(s, ff, q, p1, slots, -1, &fbad);
+                    if (!only_e) (void)term_ef<R>(s, ff, q, p1, slots, -1, &fbad);
                 } else {
-                    v[0] = term_ef<R, true>(s, ff, q, p1, bonded ? nullptr : slots, 0, &fbad);
+                    v[0] = term_ef<R>(s, ff, q, p1, only_e ? nullptr : slots, 0, &fbad);
                 }
                 if (fbad) atomicAdd(B.bad_count, 1);
                 if (need_half) v[1] = term_ef<R>(s, ff, q, p2, (R*)nullptr, 1, &fbad);
