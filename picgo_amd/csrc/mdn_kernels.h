@@ -2398,4 +2398,26 @@ __global__ void k_inc_place(DevSys s, long total, const int* __restrict__ s_star
     pos[id] = to;
 }
 
+// Copies of several pieces at once between device memory and pinned host memory: a grid row per
+// piece, 16 bytes per lane where both sides are aligned. Bound by the host link; against a
+// runtime copy per piece it saves the copy engine's start (10 us) each time.
+constexpr int COPY_PIECES = 24;
+struct CopyPieces { const void* src[COPY_PIECES]; void* dst[COPY_PIECES]; unsigned bytes[COPY_PIECES]; };
+__global__ void __launch_bounds__(BLOCK) k_copy_pieces(CopyPieces p) {
+    const int k = blockIdx.y;
+    const unsigned n = p.bytes[k], i0 = blockIdx.x * BLOCK + threadIdx.x, step = gridDim.x * BLOCK;
+    const char* src = static_cast<const char*>(p.src[k]);
+    char* dst = static_cast<char*>(p.dst[k]);
+    unsigned done = 0;
+    if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0) {
+        done = n / 16;
+        for (unsigned i = i0; i < done; i += step)
+            reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+        done *= 16;
+    }
+    for (unsigned i = done / 4 + i0; i < n / 4; i += step)
+        reinterpret_cast<unsigned*>(dst)[i] = reinterpret_cast<const unsigned*>(src)[i];
+    for (unsigned i = n / 4 * 4 + i0; i < n; i += step) dst[i] = src[i];
+}
+
 }  // namespace mdn

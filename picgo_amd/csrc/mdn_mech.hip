@@ -5,6 +5,7 @@
 // Citations are relative to medyan-5.4.0/ in the reference tree.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <cmath>
@@ -83,6 +84,8 @@ struct HipErr {
 
 }  // namespace
 
+constexpr int STAGE_SLOTS = 16;   // chunks of a host copy in flight
+
 struct mdn_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -155,6 +158,7 @@ struct mdn_ctx {
     CgState* h_cg = nullptr;   // pinned
     double* h_eout = nullptr;  // pinned
     int* h_int = nullptr;      // pinned
+    hipEvent_t stage_ev[STAGE_SLOTS] = {};   // copy_parts
 
     DevSys sys{};
     int cur = 0;   // which x buffer holds the current coordinates
@@ -218,6 +222,174 @@ hipError_t d2h(mdn_ctx* ctx, void* dst, const void* src, size_t bytes) {
     return hipStreamSynchronize(ctx->stream);
 }
 
+// ---- host copies through pinned memory ------------------------------------------------------
+// A runtime copy of pageable memory of 16 KB to 256 KB takes 18 to 110 us, and one of megabytes
+// into pages that the caller has not touched yet spends most of its time in page faults (10 MB:
+// 2,300 us, into touched pages 580). Here the data goes through a pinned ring: a kernel moves the
+// pieces between device and ring (k_copy_pieces), the CPU between ring and caller, chunk by chunk
+// side by side (16 KB 11 us, 256 KB 20, 10 MB 385 into touched pages), and fresh pages are mapped
+// in one call per chunk ahead of the copy (10 MB: 560 us of 1,700 in faults). Between STAGE_SMALL
+// and STAGE_LARGE the runtime's copy is as fast (320 KB in: 15 us, 28 here; 1 MB out: 52, 57 here),
+// and inputs beyond that too (10 MB: 297 us, 272 to 293 here).
+// Rings belong to the process, at most STAGE_RINGS per device: a call holds one while it copies
+// and gives it back; a call that finds none free takes the runtime's copy. They are freed with
+// the device's last context.
+constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_SMALL = 256u << 10, STAGE_LARGE = 2u << 20;
+constexpr int STAGE_RINGS = 4;
+struct StagePool {
+    std::mutex mu;
+    std::vector<char*> free;
+    int made = 0, users = 0;
+};
+StagePool g_stage[64];   // per device
+StagePool* stage_pool(int device) { return device >= 0 && device < 64 ? &g_stage[device] : nullptr; }
+
+// the current device's ring for this call, or null
+char* stage_acquire(int device) {
+    StagePool* P = stage_pool(device);
+    if (!P) return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(P->mu);
+        if (!P->free.empty()) {
+            char* r = P->free.back();
+            P->free.pop_back();
+            return r;
+        }
+        if (P->made >= STAGE_RINGS) return nullptr;
+        P->made++;
+    }
+    char* r = nullptr;
+    if (hipHostMalloc(&r, STAGE_BYTES) == hipSuccess) return r;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lk(P->mu);
+    P->made--;
+    return nullptr;
+}
+void stage_release(int device, char* r) {   // nothing queued reads or writes it
+    StagePool* P = stage_pool(device);
+    std::lock_guard<std::mutex> lk(P->mu);
+    P->free.push_back(r);
+}
+void stage_join(int device) {
+    if (StagePool* P = stage_pool(device)) {
+        std::lock_guard<std::mutex> lk(P->mu);
+        P->users++;
+    }
+}
+void stage_leave(int device) {   // with the device current
+    StagePool* P = stage_pool(device);
+    if (!P) return;
+    std::vector<char*> drop;
+    {
+        std::lock_guard<std::mutex> lk(P->mu);
+        if (--P->users > 0) return;
+        drop.swap(P->free);
+        P->made -= (int)drop.size();
+    }
+    for (char* r : drop) (void)hipHostFree(r);
+}
+
+// ordinary pageable memory (anything else, pinned or on a device, is the runtime's to copy)
+bool pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+// Maps the whole pages of [p, p + bytes) if the first is not mapped yet; their contents stay.
+void map_pages(void* p, size_t bytes) {
+    const uintptr_t pg = 4096, a = (reinterpret_cast<uintptr_t>(p) + pg - 1) & ~(pg - 1),
+                    b = (reinterpret_cast<uintptr_t>(p) + bytes) & ~(pg - 1);
+    if (b < a + 16 * pg) return;
+    unsigned char there = 0;
+    constexpr int POPULATE_WRITE = 23;   // MADV_POPULATE_WRITE (Linux 5.14; an older kernel refuses it)
+    if (mincore(reinterpret_cast<void*>(a), pg, &there) == 0 && !(there & 1))
+        (void)madvise(reinterpret_cast<void*>(a), b - a, POPULATE_WRITE);
+}
+
+struct HostCopy { char* host; char* dev; size_t bytes; };
+
+// The parts through a ring on the stream; complete on return. The events are the context's own: they
+// end with its stream.
+hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host) {
+    size_t total = 0;
+    for (int i = 0; i < np; i++) total += parts[i].bytes;
+    char* r = total ? stage_acquire(ctx->device) : nullptr;
+    hipError_t e = hipSuccess;
+    if (!r) {
+        for (int i = 0; i < np && e == hipSuccess; i++)
+            e = to_host ? hipMemcpyAsync(parts[i].host, parts[i].dev, parts[i].bytes, hipMemcpyDeviceToHost, ctx->stream)
+                        : hipMemcpyAsync(parts[i].dev, parts[i].host, parts[i].bytes, hipMemcpyHostToDevice, ctx->stream);
+        return e == hipSuccess ? hipStreamSynchronize(ctx->stream) : e;
+    }
+    const size_t chunk = total <= (2u << 20) ? 256u << 10 : 1u << 20;
+    const int slots = (int)(STAGE_BYTES / chunk);
+    struct Slot { HostCopy piece[COPY_PIECES]; size_t at[COPY_PIECES]; int n; } S[STAGE_SLOTS];
+    int part = 0, put = 0, got = 0;   // slots filled and emptied
+    size_t from = 0;
+    auto fill = [&](int k) {   // the next chunk's pieces into slot k
+        Slot& sl = S[k];
+        sl.n = 0;
+        for (size_t used = 0; part < np && sl.n < COPY_PIECES && used < chunk;) {
+            const HostCopy& c = parts[part];
+            const size_t len = std::min(c.bytes - from, chunk - used);
+            if (len) {
+                sl.piece[sl.n] = HostCopy{c.host + from, c.dev + from, len};
+                sl.at[sl.n++] = k * chunk + used;
+            }
+            used += (len + 15) & ~(size_t)15;
+            from += len;
+            if (from == c.bytes) { part++; from = 0; }
+        }
+        CopyPieces cp;
+        size_t most = 0;
+        for (int q = 0; q < sl.n; q++) {
+            char* pin = r + sl.at[q];
+            if (!to_host) memcpy(pin, sl.piece[q].host, sl.piece[q].bytes);
+            cp.src[q] = to_host ? sl.piece[q].dev : pin;
+            cp.dst[q] = to_host ? pin : sl.piece[q].dev;
+            cp.bytes[q] = (unsigned)sl.piece[q].bytes;
+            most = std::max(most, sl.piece[q].bytes);
+        }
+        if (sl.n == 0) return;
+        hipLaunchKernelGGL(k_copy_pieces, dim3((unsigned)std::min<size_t>(32, (most + 16 * BLOCK - 1) / (16 * BLOCK)), sl.n),
+                           dim3(BLOCK), 0, ctx->stream, cp);
+        if ((e = hipGetLastError()) == hipSuccess) e = hipEventRecord(ctx->stage_ev[k], ctx->stream);
+    };
+    while (e == hipSuccess && (part < np || got < put)) {
+        if (part < np && put - got < slots) {
+            fill(put++ % slots);
+            continue;
+        }
+        const int k = got++ % slots;
+        if ((e = hipEventSynchronize(ctx->stage_ev[k])) != hipSuccess || !to_host) continue;
+        for (int q = 0; q < S[k].n; q++) {
+            map_pages(S[k].piece[q].host, S[k].piece[q].bytes);
+            memcpy(S[k].piece[q].host, r + S[k].at[q], S[k].piece[q].bytes);
+        }
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(ctx->stream);
+    stage_release(ctx->device, r);
+    return e;
+}
+
+// Host data onto the device: complete (through a ring) or queued on return.
+hipError_t copy_in(mdn_ctx* ctx, void* dev, const void* host, size_t bytes) {
+    if (bytes < STAGE_MIN || bytes > STAGE_SMALL || !pageable(host))
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+    const HostCopy c{const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes};
+    return copy_parts(ctx, &c, 1, false);
+}
+// Device data to the host after everything queued on the stream; complete on return.
+hipError_t copy_out(mdn_ctx* ctx, void* host, const void* dev, size_t bytes) {
+    if (bytes < STAGE_MIN || (bytes > STAGE_SMALL && bytes < STAGE_LARGE) || !pageable(host))
+        return d2h(ctx, host, dev, bytes);
+    const HostCopy c{static_cast<char*>(host), const_cast<char*>(static_cast<const char*>(dev)), bytes};
+    return copy_parts(ctx, &c, 1, true);
+}
+
 bool call_limit_host(const CgState& S) {
     return (S.energy_call_limit != 0 && S.num_energy_call > S.energy_call_limit) ||
            (S.force_call_limit != 0 && S.num_force_call > S.force_call_limit);
@@ -227,7 +399,7 @@ template <typename T>
 hipError_t upload(mdn_ctx* ctx, DBuf<T>& b, const std::vector<T>& v) {
     hipError_t e = b.ensure(v.size());
     if (e != hipSuccess) return e;
-    if (!v.empty()) e = hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, ctx->stream);
+    if (!v.empty()) e = copy_in(ctx, b.p, v.data(), v.size() * sizeof(T));
     return e;
 }
 
@@ -401,8 +573,7 @@ int need_system(mdn_ctx* ctx, bool need_nl) {
 
 int set_coords_dev(mdn_ctx* ctx, const double* coord) {
     if (coord)
-        HIPCHK(hipMemcpyAsync(ctx->x[ctx->cur].p, coord, sizeof(double) * 3 * ctx->n_beads,
-                              hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->x[ctx->cur].p, coord, sizeof(double) * 3 * ctx->n_beads));
     return MDN_OK;
 }
 
@@ -598,6 +769,13 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     }
     (void)hipMemset(ctx->ticket.p, 0, sizeof(unsigned) * 8);
     (void)hipMemset(ctx->defer_n.p, 0, sizeof(int));
+    for (hipEvent_t& e : ctx->stage_ev)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            delete ctx;
+            return MDN_ERR_HIP;
+        }
+    stage_join(device);
+    if (char* r = stage_acquire(device)) stage_release(device, r);   // made before the first call needs it
     *out = ctx;
     return MDN_OK;
 }
@@ -674,6 +852,8 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
     if (ctx->h_cg) (void)hipHostFree(ctx->h_cg);
     if (ctx->h_eout) (void)hipHostFree(ctx->h_eout);
     if (ctx->h_int) (void)hipHostFree(ctx->h_int);
+    for (hipEvent_t e : ctx->stage_ev) (void)hipEventDestroy(e);
+    stage_leave(ctx->device);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return MDN_OK;
@@ -937,7 +1117,7 @@ int mdn_system_upload(mdn_ctx* ctx, const mdn_system_desc* d, const double* coor
         HIPCHK(b->ensure(nv));
     ctx->cur = 0;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->x[0].p, coord, sizeof(double) * nv, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->x[0].p, coord, sizeof(double) * nv));
     } else {
         HIPCHK(hipMemcpyAsync(ctx->x[0].p, ctx->dof_next.p, sizeof(double) * nv, hipMemcpyDeviceToDevice, ctx->stream));
     }
@@ -1057,9 +1237,7 @@ int mdn_perturb(mdn_ctx* ctx, uint64_t seed, uint64_t stream, double sigma) {
 int mdn_get_coords(mdn_ctx* ctx, double* coord) {
     int st = need_system(ctx, false);
     if (st) return st;
-    HIPCHK(hipMemcpyAsync(coord, ctx->x[ctx->cur].p, sizeof(double) * 3 * ctx->n_beads, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(copy_out(ctx, coord, ctx->x[ctx->cur].p, sizeof(double) * 3 * ctx->n_beads));
     return MDN_OK;
 }
 
@@ -1252,7 +1430,7 @@ int mdn_boundary_load_forces(mdn_ctx* ctx, const double* coord, int32_t n_types,
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads));
         x = ctx->ext.p;
     }
     const long n_out = 2L * ctx->n_fil * stride;
@@ -1290,7 +1468,7 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads));
         x = ctx->ext.p;
     }
     // the list's range in float, as addtoHNeighborList and setneighborsearchparameters form it
@@ -1308,7 +1486,7 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     if (p->site_free) {
         const size_t nf = (size_t)ctx->n_cyl * p->n_sites;
         HIPCHK(ctx->b_free.ensure(std::max<size_t>(1, nf)));
-        HIPCHK(hipMemcpyAsync(ctx->b_free.p, p->site_free, sizeof(float) * nf, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->b_free.p, p->site_free, sizeof(float) * nf));
     }
     long np = 0;
     NlBufs B{ctx->b_mid, ctx->b_bin, ctx->b_bin_count, ctx->b_bin_start, ctx->b_place, ctx->b_members,
@@ -1345,7 +1523,7 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     hipLaunchKernelGGL(k_bind_sites<1>, dim3(G), dim3(BLOCK), 0, ctx->stream, n, b, x, np, (const int*)ctx->b_pairs.p,
                        ctx->b_scount.p, (const int*)ctx->b_soff.p, ctx->b_out.p);
     HIPCHK(hipGetLastError());
-    HIPCHK(d2h(ctx, out, ctx->b_out.p, sizeof(uint32_t) * 2 * total));
+    HIPCHK(copy_out(ctx, out, ctx->b_out.p, sizeof(uint32_t) * 2 * total));
     return MDN_OK;
 }
 
@@ -1355,7 +1533,7 @@ int mdn_nl_pairs(mdn_ctx* ctx, int32_t* out, int64_t cap, int64_t* n_pairs) {
     if (n_pairs) *n_pairs = ctx->n_pairs;
     if (cap < ctx->n_pairs) return fail(ctx, MDN_ERR_CAPACITY, "need room for %ld pairs", ctx->n_pairs);
     if (ctx->n_pairs > 0)
-        HIPCHK(d2h(ctx, out, ctx->pairs.p, sizeof(int) * 2 * ctx->n_pairs));
+        HIPCHK(copy_out(ctx, out, ctx->pairs.p, sizeof(int) * 2 * ctx->n_pairs));
     return MDN_OK;
 }
 
@@ -1366,7 +1544,7 @@ int mdn_boundary_list(mdn_ctx* ctx, int32_t* out_beads, int64_t cap, int32_t* ou
     if (n_interactions) *n_interactions = ctx->n_bint;
     if (cap < ctx->n_bint) return fail(ctx, MDN_ERR_CAPACITY, "need room for %d interactions", ctx->n_bint);
     if (ctx->n_bint > 0 && out_beads)
-        HIPCHK(d2h(ctx, out_beads, ctx->bnd_b.p, sizeof(int) * ctx->n_bint));
+        HIPCHK(copy_out(ctx, out_beads, ctx->bnd_b.p, sizeof(int) * ctx->n_bint));
     if (out_nneighbors)
         for (size_t e = 0; e < ctx->bnd_nneighbors.size(); e++) out_nneighbors[e] = ctx->bnd_nneighbors[e];
     return MDN_OK;
@@ -1379,7 +1557,7 @@ static int energy_impl(mdn_ctx* ctx, const double* coord, mdn_energy_report* out
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads));
         x = ctx->ext.p;
     }
     if ((st = energy_report(ctx, x, prec))) return st;
@@ -1402,7 +1580,7 @@ static int forces_impl(mdn_ctx* ctx, int ff, const double* coord, double* force,
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * n_var));
         x = ctx->ext.p;
     }
     long lo = 0, hi = ctx->sys.slot0[NFF];
@@ -1410,7 +1588,7 @@ static int forces_impl(mdn_ctx* ctx, int ff, const double* coord, double* force,
     if (ff >= 0) {
         lo = ctx->sys.slot0[ff];
         hi = ctx->sys.slot0[ff + 1];
-        HIPCHK(hipMemcpyAsync(ctx->scratch_f.p, force, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->scratch_f.p, force, sizeof(double) * n_var));
         base = ctx->scratch_f.p;
     }
     const int bmask = ff < 0 ? 3 : ff == FF_STRETCH ? 1 : ff == FF_BEND ? 2 : 0;
@@ -1419,8 +1597,7 @@ static int forces_impl(mdn_ctx* ctx, int ff, const double* coord, double* force,
     HIPCHK(hipStreamSynchronize(ctx->stream));
     bool redone;
     if ((st = ev.finish(&redone))) return st;
-    HIPCHK(hipMemcpyAsync(force, ctx->f.p, sizeof(double) * n_var, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(copy_out(ctx, force, ctx->f.p, sizeof(double) * n_var));
     return MDN_OK;
 }
 
@@ -1504,14 +1681,13 @@ static int param_grad_impl(mdn_ctx* ctx, const double* coord, double* out, int64
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * 3 * ctx->n_beads));
         x = ctx->ext.p;
     }
     HIPCHK(ctx->ev_U.ensure(std::max(1, ctx->sys.n[FF_EXVOL])));
     HIPCHK(ctx->grad_out.ensure(3 * (size_t)std::max(1, ctx->n_cyl)));
     if ((st = param_grad_launch(ctx, x, prec, true))) return st;
-    HIPCHK(hipMemcpyAsync(out, ctx->grad_out.p, sizeof(double) * 3 * ctx->n_cyl, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(copy_out(ctx, out, ctx->grad_out.p, sizeof(double) * 3 * ctx->n_cyl));
     return MDN_OK;
 }
 
@@ -1574,14 +1750,13 @@ static int hvp_impl(mdn_ctx* ctx, const double* coord, const double* v, double* 
     HIPCHK(hipSetDevice(ctx->device));
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * n_var));
         x = ctx->ext.p;
     }
     HIPCHK(ctx->tan_v.ensure(n_var));
-    HIPCHK(hipMemcpyAsync(ctx->tan_v.p, v, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(copy_in(ctx, ctx->tan_v.p, v, sizeof(double) * n_var));
     if ((st = hvp_launch(ctx, x, prec))) return st;
-    HIPCHK(hipMemcpyAsync(out, ctx->scratch_f.p, sizeof(double) * n_var, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(copy_out(ctx, out, ctx->scratch_f.p, sizeof(double) * n_var));
     if (ctx->h_int[0] != 0)
         return fail(ctx, MDN_ERR_UNSUPPORTED, "%d excluded-volume pairs need the numerical force fallback (no tangent)",
                     ctx->h_int[0]);
@@ -1608,7 +1783,7 @@ int mdn_hvp_batch(mdn_ctx* ctx, int32_t precision, const double* coord, const do
     const DevSys& s = ctx->sys;
     const double* x = ctx->x[ctx->cur].p;
     if (coord) {
-        HIPCHK(hipMemcpyAsync(ctx->ext.p, coord, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->ext.p, coord, sizeof(double) * n_var));
         x = ctx->ext.p;
     }
     // per product: its tangent, its slots (with the gather's padding), its pieces, its result
@@ -1622,14 +1797,12 @@ int mdn_hvp_batch(mdn_ctx* ctx, int32_t precision, const double* coord, const do
     HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
     for (int k0 = 0; k0 < n_vec; k0 += chunk) {
         const int nv = std::min(chunk, n_vec - k0);
-        HIPCHK(hipMemcpyAsync(ctx->hb_v.p, V + (size_t)k0 * n_var, sizeof(double) * nv * n_var, hipMemcpyHostToDevice,
-                              ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->hb_v.p, V + (size_t)k0 * n_var, sizeof(double) * nv * n_var));
         launch_tangents(ctx, x, precision, ctx->hb_v.p, nv, ctx->hb_slots.p, slot_stride, ctx->hb_piece.p, piece_stride);
         HIPCHK(hipGetLastError());
         gather_tangents(ctx, nv, ctx->hb_slots.p, slot_stride, ctx->hb_piece.p, piece_stride, ctx->hb_out.p);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(out + (size_t)k0 * n_var, ctx->hb_out.p, sizeof(double) * nv * n_var,
-                              hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(copy_out(ctx, out + (size_t)k0 * n_var, ctx->hb_out.p, sizeof(double) * nv * n_var));
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->h_int[0] != 0)
@@ -1643,7 +1816,7 @@ int mdn_set_params(mdn_ctx* ctx, const double* kstr, const double* eql, const do
     if (st) return st;
     HIPCHK(hipSetDevice(ctx->device));
     const int nc = ctx->n_cyl;
-    if (kstr) HIPCHK(hipMemcpyAsync(ctx->str_k.p, kstr, sizeof(double) * nc, hipMemcpyHostToDevice, ctx->stream));
+    if (kstr) HIPCHK(copy_in(ctx, ctx->str_k.p, kstr, sizeof(double) * nc));
     if (eql) {
         for (int c = 0; c < nc; c++) ctx->cyl_eql[c] = eql[c];
         HIPCHK(upload(ctx, ctx->str_eql, ctx->cyl_eql));
@@ -1881,7 +2054,7 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     const int nv = 3 * ctx->n_beads;
     // startMinimization + initial energy / forces (CGMethod.hpp:876-896); the start is in x[0]
     if (coord)
-        HIPCHK(hipMemcpyAsync(ctx->x[0].p, coord, sizeof(double) * nv, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->x[0].p, coord, sizeof(double) * nv));
     else if (ctx->cur != 0)   // the context's device coordinates
         HIPCHK(hipMemcpyAsync(ctx->x[0].p, ctx->x[ctx->cur].p, sizeof(double) * nv, hipMemcpyDeviceToDevice,
                               ctx->stream));
@@ -1972,6 +2145,7 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
         if (team && !done) {
             if (n_forcen) HIPCHK(hipMemsetAsync(team_ctl(ctx->cg.p), 0, sizeof(TeamCtl), ctx->stream));
             if ((st = launch_team(ctx, prec, team))) return st;
+            if (force_out) map_pages(force_out, sizeof(double) * nv);   // while the device works
             done = true;
         }
         while (!done && launched < max_batches) {
@@ -1989,6 +2163,7 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
             HIPCHK(hipMemcpyAsync(&h_done[k], &ctx->cg.p->done, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
             HIPCHK(hipEventRecord(ev[k], ctx->stream));
             if (here > 1) {
+                if (launched == 2 && force_out) map_pages(force_out, sizeof(double) * nv);   // while the device works
                 HIPCHK(hipEventSynchronize(ev[k ^ 1]));
                 if (h_done[k ^ 1]) done = true;
             }
@@ -2052,10 +2227,8 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
         fill_report(ctx->h_eout, &res->energies_after);
         res->num_energy_call += 1;
     }
-    if (coord) HIPCHK(hipMemcpyAsync(coord, xres, sizeof(double) * nv, hipMemcpyDeviceToHost, ctx->stream));
-    if (force_out)
-        HIPCHK(hipMemcpyAsync(force_out, (S.fpar ? ctx->f2 : ctx->f).p, sizeof(double) * nv, hipMemcpyDeviceToHost,
-                              ctx->stream));
+    if (coord) HIPCHK(copy_out(ctx, coord, xres, sizeof(double) * nv));
+    if (force_out) HIPCHK(copy_out(ctx, force_out, (S.fpar ? ctx->f2 : ctx->f).p, sizeof(double) * nv));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (S.error_flags & MDN_MIN_ERR_LINESEARCH) return fail(ctx, MDN_ERR_LINESEARCH, "line search failed (recovery disabled)");
     return MDN_OK;
@@ -2193,6 +2366,7 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     // the systems that start from their device coordinates: x[cur] -> x[0], all in one launch (a
     // zero count copies nothing)
     std::vector<BatchCopy> copies((size_t)n);
+    std::vector<HostCopy> in;   // what goes onto the device: the given coordinates, then the tables
     long max_nv = 1;
     int max_blk = 1, max_nbb = 1, max_terms = 1;
     for (int i = 0; i < n; i++) {
@@ -2200,7 +2374,7 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         const long nv = 3L * c->n_beads;
         max_nv = std::max(max_nv, nv);
         if (coords[i])
-            HIPCHK_CTX(L, hipMemcpyAsync(c->x[0].p, coords[i], sizeof(double) * nv, hipMemcpyHostToDevice, L->stream));
+            in.push_back(HostCopy{(char*)coords[i], (char*)c->x[0].p, sizeof(double) * nv});
         else if (c->cur != 0)   // the context's device coordinates
             copies[i] = BatchCopy{c->x[c->cur].p, c->x[0].p, nv};
         c->cur = 0;
@@ -2245,17 +2419,15 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     HIPCHK_CTX(L, L->batch_slot.ensure(plan.slot.size()));
     HIPCHK_CTX(L, L->batch_team.ensure(plan.team.size()));
     HIPCHK_CTX(L, L->batch_ctl.ensure(plan.team.size()));
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_items.p, items.data(), sizeof(BatchItem) * n, hipMemcpyHostToDevice,
-                                 L->stream));
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * n, hipMemcpyHostToDevice,
-                                 L->stream));
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_slot.p, plan.slot.data(), sizeof(TeamSlot) * plan.slot.size(),
-                                 hipMemcpyHostToDevice, L->stream));
-    HIPCHK_CTX(L, hipMemcpyAsync(L->batch_team.p, plan.team.data(), sizeof(TeamInfo) * plan.team.size(),
-                                 hipMemcpyHostToDevice, L->stream));
-    if (!plan.order.empty())
-        HIPCHK_CTX(L, hipMemcpyAsync(L->batch_order.p, plan.order.data(), sizeof(int) * plan.order.size(),
-                                     hipMemcpyHostToDevice, L->stream));
+    auto table = [&](void* dev, const void* host, size_t bytes) {
+        if (bytes) in.push_back(HostCopy{(char*)host, (char*)dev, bytes});
+    };
+    table(L->batch_items.p, items.data(), sizeof(BatchItem) * n);
+    table(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * n);
+    table(L->batch_slot.p, plan.slot.data(), sizeof(TeamSlot) * plan.slot.size());
+    table(L->batch_team.p, plan.team.data(), sizeof(TeamInfo) * plan.team.size());
+    table(L->batch_order.p, plan.order.data(), sizeof(int) * plan.order.size());
+    HIPCHK_CTX(L, copy_parts(L, in.data(), (int)in.size(), false));
     HIPCHK_CTX(L, hipMemsetAsync(L->batch_ctl.p, 0, sizeof(TeamCtl) * plan.team.size(), L->stream));
     HIPCHK_CTX(L, hipMemsetAsync(L->batch_queue.p, 0, sizeof(int), L->stream));
     const BatchItem* di = L->batch_items.p;
@@ -2303,24 +2475,22 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     std::vector<CgState> states(n);
     std::vector<double> reports(27 * (size_t)n);
     std::vector<TeamCtl> ctl(plan.team.size());
-    HIPCHK_CTX(L, hipMemcpyAsync(states.data(), L->batch_states.p, sizeof(CgState) * n, hipMemcpyDeviceToHost,
-                                 L->stream));
-    HIPCHK_CTX(L, hipMemcpyAsync(ctl.data(), L->batch_ctl.p, sizeof(TeamCtl) * ctl.size(), hipMemcpyDeviceToHost,
-                                 L->stream));
-    HIPCHK_CTX(L, d2h(L, reports.data(), L->batch_reports.p, sizeof(double) * 27 * n));
+    const HostCopy head[3] = {{(char*)states.data(), (char*)L->batch_states.p, sizeof(CgState) * n},
+                              {(char*)ctl.data(), (char*)L->batch_ctl.p, sizeof(TeamCtl) * ctl.size()},
+                              {(char*)reports.data(), (char*)L->batch_reports.p, sizeof(double) * 27 * n}};
+    HIPCHK_CTX(L, copy_parts(L, head, 3, true));
     for (const TeamCtl& c : ctl)
         if (c.failed) return fail(L, MDN_ERR_STATE, "a workgroup of the minimizer gave up waiting for the others");
+    std::vector<HostCopy> out;
     for (int i = 0; i < n; i++) {
         mdn_ctx* c = ctxs[i];
         const CgState& S = states[i];
-        const int nv = 3 * c->n_beads;
-        if (coords[i])
-            HIPCHK_CTX(L, hipMemcpyAsync(coords[i], c->x[S.parity].p, sizeof(double) * nv, hipMemcpyDeviceToHost,
-                                         L->stream));
+        const size_t bytes = sizeof(double) * 3 * c->n_beads;
+        if (coords[i]) out.push_back(HostCopy{(char*)coords[i], (char*)c->x[S.parity].p, bytes});
         if (forces_out && forces_out[i])
-            HIPCHK_CTX(L, hipMemcpyAsync(forces_out[i], (S.fpar ? c->f2 : c->f).p, sizeof(double) * nv,
-                                         hipMemcpyDeviceToHost, L->stream));
+            out.push_back(HostCopy{(char*)forces_out[i], (char*)(S.fpar ? c->f2 : c->f).p, bytes});
     }
+    HIPCHK_CTX(L, copy_parts(L, out.data(), (int)out.size(), true));
     HIPCHK_CTX(L, hipStreamSynchronize(L->stream));
     int first_err = MDN_OK;
     for (int i = 0; i < n; i++) {
@@ -2457,7 +2627,7 @@ int mdn_bench_adjoint(mdn_ctx* ctx, int32_t precision, int32_t iters, const doub
     const long piece_stride = (long)NBOND * 3 * ctx->n_beads;
     if (n_vec == 1) {
         HIPCHK(ctx->tan_v.ensure(n_var));
-        HIPCHK(hipMemcpyAsync(ctx->tan_v.p, v, sizeof(double) * n_var, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(copy_in(ctx, ctx->tan_v.p, v, sizeof(double) * n_var));
     } else {
         HIPCHK(ctx->hb_v.ensure((size_t)n_vec * n_var));
         HIPCHK(ctx->hb_slots.ensure((size_t)n_vec * slot_stride));
