@@ -1068,6 +1068,7 @@ struct CgBufs {
     double* partial;    // line-search partials, value-major: [value][interaction blocks + bead blocks]
     double* gpartial;   // gather partials, value-major: [value][gather blocks]
     int* bad_count;     // excluded-volume pairs needing the numerical fallback in a CG move
+    int* done_host;     // pinned host memory: set to 1 by the slot that ends the minimization
 };
 
 __device__ inline bool call_limit(const CgState* st) {
@@ -1726,6 +1727,7 @@ __global__ void __launch_bounds__(FIN) k_cg_fin(DevSys s, CgState* __restrict__ 
         if (gather) gather_control(S, acc + 8, bad);
         if (bad != sh_bad) *B.bad_count = bad;
         *st = S;
+        if (S.done) *B.done_host = 1;
     }
 }
 
