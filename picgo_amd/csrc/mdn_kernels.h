@@ -1964,17 +1964,16 @@ __global__ void k_nl_fill(NLDev n, const int* __restrict__ bin, const int* __res
 }
 
 // HybridNeighborListImpl.cpp:411-439 predicate, on explicit records and midpoints (a candidate's
-// from LDS)
+// from LDS). Every part is evaluated: the reads of a candidate are in flight together.
 __device__ inline bool nl_keep_at(const NLDev& n, const NlRec& c, const NlRec& cn, const double* mc, const double* mn) {
-    if (c.c <= cn.c) return false;
-    if (c.fil == cn.fil && abs(c.pos - cn.pos) <= 2) return false;
-    if (n.ta >= 0 && (min(c.type, cn.type) != n.ta || max(c.type, cn.type) != n.tb)) return false;
     double d2 = 0.0;
     for (int q = 0; q < 3; q++) {
         double v = mn[q] - mc[q];
         d2 += v * v;
     }
-    return !(d2 < n.rminsq || d2 > n.rmaxsq);
+    const bool near = (c.fil == cn.fil) & (abs(c.pos - cn.pos) <= 2);
+    const bool typed = (n.ta < 0) | ((min(c.type, cn.type) == n.ta) & (max(c.type, cn.type) == n.tb));
+    return (c.c > cn.c) & !near & typed & !((d2 < n.rminsq) | (d2 > n.rmaxsq));
 }
 
 // Cell-list pairs, one workgroup per tile of T^3 bins (HybridCylinderCylinderNL::updateNeighborsbin,
@@ -1982,8 +1981,8 @@ __device__ inline bool nl_keep_at(const NLDev& n, const NlRec& c, const NlRec& c
 //   1. each thread takes halo bins (the tile's bins and one bin around them, (T + 2)^3) and
 //      reads their member ranges; a block scan of the counts places every halo bin's members
 //      contiguously, in halo-bin order, in LDS with their midpoints,
-//   2. NL_LANES lanes per cylinder of the tile test the members of its 27 bins, each lane a row
-//      of three consecutive halo bins of LDS at a time (nine rows),
+//   2. NL_LANES lanes per cylinder of the tile test the members of its 27 bins, nine rows of three
+//      consecutive halo bins of LDS taken as one list, a candidate per lane at a time,
 //   3. the neighbours found, collected in LDS, are written in ascending order by rank.
 // A halo with more than NL_CAP members is read from global memory instead (the same 27 bins). The
 // bins are wider than the range, so the pair set is the predicate's whatever the bin size.
@@ -1993,7 +1992,7 @@ __device__ inline bool nl_keep_at(const NLDev& n, const NlRec& c, const NlRec& c
 // Latency bound. With one lane per cylinder (36 of 256 lanes busy at 42,000 beads), the predicate's
 // records read from global memory and a second search that sorted in global memory, count and
 // emission took 105 us there, 205 us at 420,000 and 308 us for a binder's wider list at 42,000;
-// now 50, 74 and 63 us.
+// now 34, 62 and 42 us (50, 74 and 63 with a row per lane instead of the rows as one list).
 constexpr int NL_CAP = 512;
 constexpr int NL_HMAX = 10 * 10 * 10;   // (T + 2)^3 for T <= 8
 constexpr int NL_RUN = (NL_HMAX + BLOCK - 1) / BLOCK;
@@ -2074,41 +2073,58 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
         }
         __syncthreads();
     }
-    // 2. the tile's cylinders, NL_GROUPS at a time
+    // 2. the tile's cylinders, NL_GROUPS at a time; the next ones' records are loaded ahead
     const int grp = threadIdx.x / NL_LANES, lane = threadIdx.x % NL_LANES;
+    struct Own { NlRec c; double m[3]; int bin; };
+    auto own = [&](int i) {
+        Own o{NlRec{-1, 0, 0, 0}, {0.0, 0.0, 0.0}, 0};
+        if (i < i1) o = Own{members[i], {mmid[3 * (long)i], mmid[3 * (long)i + 1], mmid[3 * (long)i + 2]}, mbin[i]};
+        return o;
+    };
+    Own next = own(i0 + grp);
     for (int g0 = i0; g0 < i1; g0 += NL_GROUPS) {
-        const int i = g0 + grp;
-        const bool mine = i < i1;
-        const NlRec c = mine ? members[i] : NlRec{-1, 0, 0, 0};
+        const bool mine = g0 + grp < i1;
+        const Own o = next;
+        next = own(g0 + NL_GROUPS + grp);
+        const NlRec c = o.c;
+        const double* mc = o.m;
         const long base = PASS && mine ? off[c.c] : 0;
         if (lane == 0) s_cnt[grp] = 0;
         __syncthreads();
         if (mine) {
-            const double mc[3] = {mmid[3 * (long)i], mmid[3 * (long)i + 1], mmid[3 * (long)i + 2]};
-            const int loc = mbin[i] & (T3 - 1);
+            const int loc = o.bin & (T3 - 1);
             const int lx = (loc & (T - 1)) + 1, ly = ((loc >> lt) & (T - 1)) + 1, lz = (loc >> (2 * lt)) + 1;   // halo coords
             auto hit = [&](int cn) {
                 const int k = atomicAdd(&s_cnt[grp], 1);
                 if (k < NL_HITS) s_hit[k] = cn;
                 else if (PASS) pairs[2 * (base + k) + 1] = cn;
             };
-            for (int r = lane; r < 9; r += NL_LANES) {
-                const int dy = r % 3 - 1, dz = r / 3 - 1;
-                if (staged) {
-                    const int h = (lx - 1) + H * ((ly + dy) + H * (lz + dz));
-                    const int k1 = s_start[h + 3];
-                    for (int k = s_start[h]; k < k1; k++)
-                        if (nl_keep_at(n, c, s_rec[k], mc, &s_mid[3 * k])) hit(s_rec[k].c);
-                } else {
+            if (staged) {
+                int first[9], before[10];   // the rows' first members in LDS, the candidates before each
+                before[0] = 0;
+#pragma unroll
+                for (int r = 0; r < 9; r++) {
+                    const int h = (lx - 1) + H * ((ly + r % 3 - 1) + H * (lz + r / 3 - 1));
+                    first[r] = s_start[h];
+                    before[r + 1] = before[r] + s_start[h + 3] - first[r];
+                }
+                for (int f = lane; f < before[9]; f += NL_LANES) {
+                    int k = f + first[0];
+#pragma unroll
+                    for (int r = 1; r < 9; r++) k = f >= before[r] ? f - before[r] + first[r] : k;
+                    const NlRec cn = s_rec[k];
+                    if (nl_keep_at(n, c, cn, mc, &s_mid[3 * k])) hit(cn.c);
+                }
+            } else {
+                for (int r = lane; r < 9; r += NL_LANES)
                     for (int dx = -1; dx <= 1; dx++) {
-                        const int X = hx0 + lx + dx, Y = hy0 + ly + dy, Z = hz0 + lz + dz;
+                        const int X = hx0 + lx + dx, Y = hy0 + ly + r % 3 - 1, Z = hz0 + lz + r / 3 - 1;
                         if (X < 0 || Y < 0 || Z < 0 || X >= n.nb[0] || Y >= n.nb[1] || Z >= n.nb[2]) continue;
                         const int nbin = nl_bin_id(n, X, Y, Z);
                         const int m1 = bin_start[nbin + 1];
                         for (int m = bin_start[nbin]; m < m1; m++)
                             if (nl_keep_at(n, c, members[m], mc, &mmid[3 * (long)m])) hit(members[m].c);
                     }
-                }
             }
         }
         __syncthreads();
