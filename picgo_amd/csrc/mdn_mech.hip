@@ -2003,19 +2003,26 @@ static long team_cost(const DevSys& s) {
 // of up to 12,000 beads take 2.3, 2.6 and 4.4 ms with 256, 2.8, 3.0 and 4.7 ms with 1024, 3.5, 3.8
 // and 5.7 ms with 2048.
 static const long TEAM_SHARE = 256;
-// A single network's team: 16 workgroups at most (32 are 5 to 10 % slower below TEAM_WIDE, where
-// their dearer barriers count more than the work they share: 1,300 beads in a cube 1.74 against
-// 1.92 ms per 80 iterations), 32 from there to TEAM_COST_MAX (8,400 beads in a sphere, work 36,000:
-// 2.10 against 2.34 ms), and from there on the four-kernel slots over the whole chip (10,500 beads
-// in a sphere, work 43,000: 2.30 ms against 2.38 ms with 32 workgroups; 3,100 in a cube, work
-// 40,000: 2.35 against 2.27 ms; 550 beads: 2.14 against 1.55 ms).
-static const long TEAM_WIDE = 33000, TEAM_COST_MAX = 41000;
+// A single network's work, in which a pair counts less than in a batch (its two chains run side by
+// side): TEAM_ONE_SHARE of it per workgroup up to 16 workgroups, 24 from TEAM_WIDE on (below, their
+// dearer barriers count more than the work they share) and from TEAM_ONE_MAX on the four-kernel
+// slots over the whole chip. FP64 / mixed, ms per 80 iterations without the rebuild:
+//   550 beads, work 1,200: 6, 8, 10 and 16 workgroups 1.30, 1.32, 1.36, 1.39 / 1.41, 1.41, 1.41, 1.44
+//   4,200 in a sphere, 8,800: 16 and 24 workgroups 1.73, 1.67 / 1.60, 1.72
+//   7,350 in a sphere, 13,900: 16, 24, 32, slots 2.13, 1.87, 1.91, 2.02 / 1.95, 1.87, 1.82, 2.17
+//   3,150 in a cube, 14,200: 2.19, 1.93, 1.94, 2.12 / 2.01, 1.84, 1.90, 2.17
+//   9,450 in a sphere, 19,100: 2.50, 2.11, 2.06, 2.04 / 2.23, 1.94, 2.01, 2.10
+//   4,830 in a cube, 21,200: 2.69, 2.36, 2.22, 2.17 / 2.28, 2.18, 2.07, 2.17
+static long team_one_work(const DevSys& s) {
+    return s.n_beads + s.n[FF_LINKER] + s.n[FF_MOTOR] + 2L * s.n[FF_EXVOL] + s.n[FF_BOUNDARY];
+}
+static const long TEAM_ONE_SHARE = 160, TEAM_WIDE = 9000, TEAM_ONE_MAX = 17500;
 // Workgroups of the persistent minimizer for a single network; 0: the four-kernel slots.
 static int team_workgroups(const mdn_ctx* ctx) {
     if (!cg_bonded_sums(ctx, 0) || ctx->n_beads >= GB_LARGE_BEADS) return 0;
     if (ctx->team_size >= 0) return ctx->team_size;
-    const long c = team_cost(ctx->sys);
-    return c > TEAM_COST_MAX ? 0 : c > TEAM_WIDE ? TEAM_MAX : (int)std::min<long>(16, (c + TEAM_SHARE - 1) / TEAM_SHARE);
+    const long c = team_one_work(ctx->sys);
+    return c > TEAM_ONE_MAX ? 0 : c > TEAM_WIDE ? 24 : (int)std::min<long>(16, (c + TEAM_ONE_SHARE - 1) / TEAM_ONE_SHARE);
 }
 
 // The persistent minimizer on one system from its device state until that is done. The barrier's
