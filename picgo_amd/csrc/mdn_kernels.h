@@ -181,12 +181,12 @@ __device__ inline int ff_of_block(const DevSys& s, int b) {
     return k < NFF ? s.dff[k] : NFF;   // NFF means a bead block
 }
 
-// The FP64 line search evaluates the excluded-volume forces in blocks of their own, ahead of the
+// The FP64 line search can evaluate the excluded-volume forces in blocks of their own, ahead of the
 // interaction blocks, whose excluded-volume blocks then take the energies alone: the two chains run
 // side by side instead of one after the other (term_ef says why the mixed path does not).
-template <typename R>
+template <typename R, bool SPLIT>
 __device__ __host__ inline int ev_force_blocks(const DevSys& s) {
-    return sizeof(R) == 8 ? (s.n[FF_EXVOL] + BLOCK - 1) / BLOCK : 0;
+    return SPLIT && sizeof(R) == 8 ? (s.n[FF_EXVOL] + BLOCK - 1) / BLOCK : 0;
 }
 
 // ---- deterministic reduction helpers (64-wide waves) ----------------------------------
@@ -370,12 +370,12 @@ __device__ inline void push_defer(const DevSys& s, int code, int t, D3 c1, D3 c2
 // form divides a bracket that vanishes like the squared triple product of the pair by that
 // square, so FP32 rounding is amplified like 1/tau^2 for near-coplanar pairs (tau the normalized
 // triple product), and FP32 gains nothing on gfx950 for this latency-bound term.
-// The FP64 path evaluates an excluded-volume pair for its forces (code < 0, into the slots) or for
-// its energy (code >= 0), never for both at once: each is one long chain of FP64 operations, and
-// the forces of a near-coplanar pair take other invariants than its energy. The mixed path takes
-// both in one call where both are wanted: its FMA-contracted forms fuse differently in separate
-// code (differences at rounding level, which a minimization amplifies).
-template <typename R>
+// SPLIT: the FP64 path evaluates an excluded-volume pair for its forces (code < 0, into the slots)
+// or for its energy (code >= 0), never for both in one call: each is one long chain of FP64
+// operations, and the forces of a near-coplanar pair take other invariants than its energy. The
+// mixed path always takes both where both are wanted: its FMA-contracted forms fuse differently in
+// separate code (differences at rounding level, which a minimization amplifies).
+template <typename R, bool SPLIT = true>
 __device__ inline double term_ef(const DevSys& s, int ff, int t, const Pos& p, R* __restrict__ slots,
                                  int code, int* fbad, int* bad_t = nullptr) {
     D3 out[4];
@@ -427,9 +427,10 @@ __device__ inline double term_ef(const DevSys& s, int ff, int t, const Pos& p, R
         constexpr bool fast = sizeof(R) == 4;
         int deferred = 0;
         double U = 0.0;
-        if (fast ? slots != nullptr : code < 0) {
+        if (fast || !SPLIT ? slots != nullptr : code < 0) {
             bool ok = true;
             if (!fast) {
+                if (!SPLIT && code >= 0) U = exvol_energy<double>(c1, c2, c3, c4, s.ev_ks[tp], &deferred);
                 ok = exvol_forces<double>(c1, c2, c3, c4, s.ev_ks[tp], out);
             } else if (code < 0) {
                 ok = exvol_forces_fast(c1, c2, c3, c4, s.ev_ks[tp], out);
@@ -1209,7 +1210,7 @@ __device__ inline void bead_ls(const DevSys& s, const CgBufs& B, int j, bool mov
 // blocks are fewer than the chip holds: with a pair's energy and forces in one thread an
 // FP64 minimization took 3068 us at 42,000 beads and 1630 at 550 (by a team), now 2930 and 1432.
 // 3 waves per SIMD (at most 168 VGPRs) measured faster than the unconstrained 2.
-template <typename R>
+template <typename R, bool SPLIT>
 __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __restrict__ st, CgBufs B) {
     __shared__ double lds[3 * (BLOCK / 64)];
     // the state fields, loaded before the first branch (one round trip)
@@ -1223,7 +1224,7 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     // the excluded-volume pairs' forces come first, in blocks of their own (ev_force_blocks); then
     // the interaction blocks; with bonded_gather bead blocks follow and carry the filament terms'
     // forces (and, with bead_energy, their energies: then the filament terms' blocks are left out)
-    const int nevf = ev_force_blocks<R>(s);
+    const int nevf = ev_force_blocks<R, SPLIT>(s);
     const int nint = (s.bonded_gather && s.bead_energy) ? s.blk_nb : s.blk[NFF];
     const int blk = (int)blockIdx.x - nevf;
     const double* __restrict__ xn = B.x[par ^ 1];
@@ -1247,7 +1248,7 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     const int t = (blk - s.fblk[ff]) * BLOCK + threadIdx.x;
     // FP64 excluded volume and, with bonded_gather (and not bead_energy), the filament terms:
     // energies only
-    const bool only_e = (nevf > 0 && ff == FF_EXVOL) || (s.bonded_gather && (ff == FF_STRETCH || ff == FF_BEND));
+    const bool only_e = (SPLIT && nevf > 0 && ff == FF_EXVOL) || (s.bonded_gather && (ff == FF_STRETCH || ff == FF_BEND));
     R* const tslots = only_e ? nullptr : slots;
     if (phase == PH_MOVE) {
         if (t < s.n[ff] && !only_e) {
@@ -1260,7 +1261,7 @@ __global__ void __launch_bounds__(BLOCK, 3) k_cg_ls(DevSys s, const CgState* __r
     double v[3] = {0.0, 0.0, 0.0};
     if (t < s.n[ff]) {
         int fbad = 0;
-        v[0] = term_ef<R>(s, ff, t, p1, tslots, 0, &fbad);
+        v[0] = term_ef<R, SPLIT>(s, ff, t, p1, tslots, 0, &fbad);
         if (fbad) atomicAdd(B.bad_count, 1);
         if (!first) {   // the first launch of a search evaluates lambda0 alone (see ls_control)
             const Pos p2{B.xh, nullptr, nullptr, 0.0, 0.0, 0};

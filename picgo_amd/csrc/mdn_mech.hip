@@ -1956,16 +1956,27 @@ static DevSys cg_sys(const mdn_ctx* ctx, int prec) {
 }
 
 extern "C++" {
+// FP64 excluded-volume force blocks of their own pay while the chip is not full without them (80
+// iterations without the rebuild, one thread per pair -> two: 14,700 beads in a cube 2.22 -> 2.07 ms,
+// 42,000 2.53 -> 2.48, 84,000 3.04 -> 3.02, 126,000 3.31 -> 3.42; in a sphere 42,000 2.26 -> 2.08,
+// 84,000 2.47 -> 2.42, 126,000 2.62 -> 2.69, 420,000 4.84 -> 4.93).
+static const int EV_SPLIT_BEADS = 100000;
 template <typename R>
 static void launch_slot(mdn_ctx* ctx, const DevSys& s, const CgBufs& B) {
     const int gbk = gather_blocks(ctx);
     hipLaunchKernelGGL(k_cg_pos, dim3(bead_blocks(ctx)), dim3(BLOCK), 0, ctx->stream, s, (const CgState*)ctx->cg.p, B);
     // the excluded-volume force blocks, all interaction blocks, then (bonded_gather) the bead blocks;
     // with bead_energy the filament terms' blocks are left out
-    const int lsg = ev_force_blocks<R>(s) +
-                    (s.bonded_gather ? (s.bead_energy ? s.blk_nb : s.blk[NFF]) + s.nbb : s.blk[NFF]);
-    hipLaunchKernelGGL(k_cg_ls<R>, dim3(std::max(1, lsg)), dim3(BLOCK), 0, ctx->stream, s,
-                       (const CgState*)ctx->cg.p, B);
+    const int lsg = s.bonded_gather ? (s.bead_energy ? s.blk_nb : s.blk[NFF]) + s.nbb : s.blk[NFF];
+    bool split = false;
+    if constexpr (sizeof(R) == 8) split = s.n_beads < EV_SPLIT_BEADS;
+    if constexpr (sizeof(R) == 8)
+        if (split)
+            hipLaunchKernelGGL((k_cg_ls<R, true>), dim3(std::max(1, ev_force_blocks<R, true>(s) + lsg)), dim3(BLOCK), 0,
+                               ctx->stream, s, (const CgState*)ctx->cg.p, B);
+    if (!split)
+        hipLaunchKernelGGL((k_cg_ls<R, false>), dim3(std::max(1, lsg)), dim3(BLOCK), 0, ctx->stream, s,
+                           (const CgState*)ctx->cg.p, B);
     launch_cg_gather<R>(ctx, s, (const CgState*)ctx->cg.p, B);
     hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(FIN), 0, ctx->stream, s, ctx->cg.p, B, gbk);
 }

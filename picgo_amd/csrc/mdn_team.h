@@ -206,7 +206,7 @@ __device__ inline void team_ls(const DevSys& s, const CgBufs& B, const CgState& 
     const bool need_e0 = !move && first && !S.ecur_valid, need_half = !move && !first;
     const int par = S.parity, T = s.blk[NFF];
     const bool be = s.bead_energy != 0;
-    const int nint = be ? s.blk_nb : T, nevf = 4 * ev_force_blocks<R>(s), total = nevf + 4 * (nint + s.nbb);
+    const int nint = be ? s.blk_nb : T, nevf = 4 * ev_force_blocks<R, true>(s), total = nevf + 4 * (nint + s.nbb);
     const long nc = SUM == SUM_STRIDED ? team_items(s) : 4L * (T + s.nbb);   // entries per value
     const double* __restrict__ xn = B.x[par ^ 1];
     const Pos p1{xn, nullptr, nullptr, 0.0, 0.0, 0};
