@@ -230,11 +230,12 @@ hipError_t d2h(mdn_ctx* ctx, void* dst, const void* src, size_t bytes) {
 // side by side (16 KB 11 us, 256 KB 20, 10 MB 385 into touched pages), and fresh pages are mapped
 // in one call per chunk ahead of the copy (10 MB: 560 us of 1,700 in faults). Between STAGE_SMALL
 // and STAGE_LARGE the runtime's copy is as fast (320 KB in: 15 us, 28 here; 1 MB out: 52, 57 here),
-// and inputs beyond that too (10 MB: 297 us, 272 to 293 here).
+// and inputs beyond that too (10 MB: 297 us, 272 to 293 here); inputs below STAGE_IN_MIN it queues
+// without a wait.
 // Rings belong to the process, at most STAGE_RINGS per device: a call holds one while it copies
 // and gives it back; a call that finds none free takes the runtime's copy. They are freed with
 // the device's last context.
-constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_SMALL = 256u << 10, STAGE_LARGE = 2u << 20;
+constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_IN_MIN = 32u << 10, STAGE_SMALL = 256u << 10, STAGE_LARGE = 2u << 20;
 constexpr int STAGE_RINGS = 4;
 struct StagePool {
     std::mutex mu;
@@ -354,6 +355,7 @@ hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host)
             most = std::max(most, sl.piece[q].bytes);
         }
         if (sl.n == 0) return;
+        if (!ctx->stage_ev[k] && (e = hipEventCreateWithFlags(&ctx->stage_ev[k], hipEventDisableTiming)) != hipSuccess) return;
         hipLaunchKernelGGL(k_copy_pieces, dim3((unsigned)std::min<size_t>(32, (most + 16 * BLOCK - 1) / (16 * BLOCK)), sl.n),
                            dim3(BLOCK), 0, ctx->stream, cp);
         if ((e = hipGetLastError()) == hipSuccess) e = hipEventRecord(ctx->stage_ev[k], ctx->stream);
@@ -364,6 +366,7 @@ hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host)
             continue;
         }
         const int k = got++ % slots;
+        if (S[k].n == 0) continue;
         if ((e = hipEventSynchronize(ctx->stage_ev[k])) != hipSuccess || !to_host) continue;
         for (int q = 0; q < S[k].n; q++) {
             map_pages(S[k].piece[q].host, S[k].piece[q].bytes);
@@ -377,7 +380,7 @@ hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host)
 
 // Host data onto the device: complete (through a ring) or queued on return.
 hipError_t copy_in(mdn_ctx* ctx, void* dev, const void* host, size_t bytes) {
-    if (bytes < STAGE_MIN || bytes > STAGE_SMALL || !pageable(host))
+    if (bytes < STAGE_IN_MIN || bytes > STAGE_SMALL || !pageable(host))
         return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
     const HostCopy c{const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes};
     return copy_parts(ctx, &c, 1, false);
@@ -769,11 +772,6 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     }
     (void)hipMemset(ctx->ticket.p, 0, sizeof(unsigned) * 8);
     (void)hipMemset(ctx->defer_n.p, 0, sizeof(int));
-    for (hipEvent_t& e : ctx->stage_ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            delete ctx;
-            return MDN_ERR_HIP;
-        }
     stage_join(device);
     if (char* r = stage_acquire(device)) stage_release(device, r);   // made before the first call needs it
     *out = ctx;
@@ -852,7 +850,8 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
     if (ctx->h_cg) (void)hipHostFree(ctx->h_cg);
     if (ctx->h_eout) (void)hipHostFree(ctx->h_eout);
     if (ctx->h_int) (void)hipHostFree(ctx->h_int);
-    for (hipEvent_t e : ctx->stage_ev) (void)hipEventDestroy(e);
+    for (hipEvent_t e : ctx->stage_ev)
+        if (e) (void)hipEventDestroy(e);
     stage_leave(ctx->device);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
