@@ -2425,7 +2425,7 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     P.lambda_max = p->lambda_max;
     P.grad_tol = p->grad_tol;
     P.energy_rel_tol = p->energy_rel_tol;
-    // one workgroup per CU (12 wavefronts at 168 VGPRs fill it); MDN_BATCH_MAX_WORKGROUPS caps
+    // one workgroup per CU (8 wavefronts at 179 to 250 VGPRs fill it); MDN_BATCH_MAX_WORKGROUPS caps
     // them, so that every workgroup pulls several systems (what a batch larger than the chip does)
     int n_cu = 0;
     HIPCHK_CTX(L, hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, L->device));
