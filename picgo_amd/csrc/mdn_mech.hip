@@ -223,19 +223,24 @@ hipError_t d2h(mdn_ctx* ctx, void* dst, const void* src, size_t bytes) {
 }
 
 // ---- host copies through pinned memory ------------------------------------------------------
-// A runtime copy of pageable memory of 16 KB to 256 KB takes 18 to 110 us, and one of megabytes
-// into pages that the caller has not touched yet spends most of its time in page faults (10 MB:
-// 2,300 us, into touched pages 580). Here the data goes through a pinned ring: a kernel moves the
-// pieces between device and ring (k_copy_pieces), the CPU between ring and caller, chunk by chunk
-// side by side (16 KB 11 us, 256 KB 20, 10 MB 385 into touched pages), and fresh pages are mapped
-// in one call per chunk ahead of the copy (10 MB: 560 us of 1,700 in faults). Between STAGE_SMALL
-// and STAGE_LARGE the runtime's copy is as fast (320 KB in: 15 us, 28 here; 1 MB out: 52, 57 here),
-// and inputs beyond that too (10 MB: 297 us, 272 to 293 here); inputs below STAGE_IN_MIN it queues
-// without a wait.
+// Results go through a pinned ring where that is the faster way: a kernel moves the pieces between
+// device and ring (k_copy_pieces), the CPU between ring and caller, chunk by chunk side by side, and
+// pages that the caller has not touched yet are mapped in one call per chunk ahead of the copy. The
+// runtime's copy and the ring, us:
+//     result into touched pages  16 KB 21, 13;  24 KB 10, 14;  256 KB 19, 23;  1 MB 62, 78;
+//                                2 MB 122, 129;  3 MB 182, 135;  8 MB 485, 385
+//     result into fresh pages    16 KB 23, 16;  24 KB 14, 18;  64 KB 22, 22;  96 KB 29, 26;
+//                                256 KB 63, 49;  1 MB 280, 180;  8 MB 2240, 1490
+//     input                      16 KB 13, 14;  64 KB 11, 15;  256 KB 16, 21;  1 MB 55, 78;
+//                                8 MB 250, 280
+// So results up to STAGE_TINY and beyond STAGE_LARGE take the ring, those between only into fresh
+// pages from STAGE_FRESH on, and inputs never: the runtime queues them, while each one through the
+// ring is a wait (four parameter uploads of 144 KB: 61 us, through the ring 111). A batch's many
+// tables and coordinates take the ring together in both directions.
 // Rings belong to the process, at most STAGE_RINGS per device: a call holds one while it copies
 // and gives it back; a call that finds none free takes the runtime's copy. They are freed with
 // the device's last context.
-constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_IN_MIN = 32u << 10, STAGE_SMALL = 256u << 10, STAGE_LARGE = 2u << 20;
+constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_TINY = 16u << 10, STAGE_FRESH = 96u << 10, STAGE_LARGE = 2u << 20;
 constexpr int STAGE_RINGS = 4;
 struct StagePool {
     std::mutex mu;
@@ -299,14 +304,24 @@ bool pageable(const void* p) {
     }
     return a.type == hipMemoryTypeUnregistered;
 }
-// Maps the whole pages of [p, p + bytes) if the first is not mapped yet; their contents stay.
-void map_pages(void* p, size_t bytes) {
-    const uintptr_t pg = 4096, a = (reinterpret_cast<uintptr_t>(p) + pg - 1) & ~(pg - 1),
-                    b = (reinterpret_cast<uintptr_t>(p) + bytes) & ~(pg - 1);
-    if (b < a + 16 * pg) return;
+// The whole pages of [p, p + bytes), if there are enough of them for a call of their own.
+constexpr uintptr_t HOST_PAGE = 4096;
+bool whole_pages(const void* p, size_t bytes, uintptr_t* a, uintptr_t* b) {
+    *a = (reinterpret_cast<uintptr_t>(p) + HOST_PAGE - 1) & ~(HOST_PAGE - 1);
+    *b = (reinterpret_cast<uintptr_t>(p) + bytes) & ~(HOST_PAGE - 1);
+    return *b >= *a + 16 * HOST_PAGE;
+}
+// Whether the first of them is not mapped yet.
+bool fresh_pages(const void* p, size_t bytes) {
+    uintptr_t a, b;
     unsigned char there = 0;
+    return whole_pages(p, bytes, &a, &b) && mincore(reinterpret_cast<void*>(a), HOST_PAGE, &there) == 0 && !(there & 1);
+}
+// Maps them if the first is not mapped yet; their contents stay.
+void map_pages(void* p, size_t bytes) {
     constexpr int POPULATE_WRITE = 23;   // MADV_POPULATE_WRITE (Linux 5.14; an older kernel refuses it)
-    if (mincore(reinterpret_cast<void*>(a), pg, &there) == 0 && !(there & 1))
+    uintptr_t a, b;
+    if (fresh_pages(p, bytes) && whole_pages(p, bytes, &a, &b))
         (void)madvise(reinterpret_cast<void*>(a), b - a, POPULATE_WRITE);
 }
 
@@ -378,17 +393,15 @@ hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host)
     return e;
 }
 
-// Host data onto the device: complete (through a ring) or queued on return.
+// Host data onto the device, queued.
 hipError_t copy_in(mdn_ctx* ctx, void* dev, const void* host, size_t bytes) {
-    if (bytes < STAGE_IN_MIN || bytes > STAGE_SMALL || !pageable(host))
-        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
-    const HostCopy c{const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes};
-    return copy_parts(ctx, &c, 1, false);
+    return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
 }
 // Device data to the host after everything queued on the stream; complete on return.
 hipError_t copy_out(mdn_ctx* ctx, void* host, const void* dev, size_t bytes) {
-    if (bytes < STAGE_MIN || (bytes > STAGE_SMALL && bytes < STAGE_LARGE) || !pageable(host))
-        return d2h(ctx, host, dev, bytes);
+    const bool ring = bytes <= STAGE_TINY ? bytes >= STAGE_MIN
+                                          : bytes > STAGE_LARGE || (bytes >= STAGE_FRESH && fresh_pages(host, bytes));
+    if (!ring || !pageable(host)) return d2h(ctx, host, dev, bytes);
     const HostCopy c{static_cast<char*>(host), const_cast<char*>(static_cast<const char*>(dev)), bytes};
     return copy_parts(ctx, &c, 1, true);
 }
