@@ -2349,6 +2349,16 @@ static TeamPlan plan_teams(const std::vector<long>& cost, int groups) {
     return P;
 }
 
+// One system's coordinates or forces: among the parts that go through the ring together, or, from
+// pinned or device memory (which the ring's copies by the CPU must not touch), queued by the runtime.
+static hipError_t batch_copy(mdn_ctx* L, std::vector<HostCopy>& parts, double* host, double* dev, size_t bytes, bool to_host) {
+    if (!pageable(host))
+        return to_host ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, L->stream)
+                       : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, L->stream);
+    parts.push_back(HostCopy{(char*)host, (char*)dev, bytes});
+    return hipSuccess;
+}
+
 // The persistent kernel of a planned batch.
 static int launch_batch(mdn_ctx* L, const TeamPlan& P, int prec) {
     const BatchItem* items = L->batch_items.p;
@@ -2409,7 +2419,7 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         const long nv = 3L * c->n_beads;
         max_nv = std::max(max_nv, nv);
         if (coords[i])
-            in.push_back(HostCopy{(char*)coords[i], (char*)c->x[0].p, sizeof(double) * nv});
+            HIPCHK_CTX(L, batch_copy(L, in, coords[i], c->x[0].p, sizeof(double) * nv, false));
         else if (c->cur != 0)   // the context's device coordinates
             copies[i] = BatchCopy{c->x[c->cur].p, c->x[0].p, nv};
         c->cur = 0;
@@ -2521,9 +2531,9 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         mdn_ctx* c = ctxs[i];
         const CgState& S = states[i];
         const size_t bytes = sizeof(double) * 3 * c->n_beads;
-        if (coords[i]) out.push_back(HostCopy{(char*)coords[i], (char*)c->x[S.parity].p, bytes});
+        if (coords[i]) HIPCHK_CTX(L, batch_copy(L, out, coords[i], c->x[S.parity].p, bytes, true));
         if (forces_out && forces_out[i])
-            out.push_back(HostCopy{(char*)forces_out[i], (char*)(S.fpar ? c->f2 : c->f).p, bytes});
+            HIPCHK_CTX(L, batch_copy(L, out, forces_out[i], (S.fpar ? c->f2 : c->f).p, bytes, true));
     }
     HIPCHK_CTX(L, copy_parts(L, out.data(), (int)out.size(), true));
     HIPCHK_CTX(L, hipStreamSynchronize(L->stream));
