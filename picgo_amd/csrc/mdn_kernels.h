@@ -762,21 +762,32 @@ __global__ void __launch_bounds__(BLOCK) k_gather_tangents(DevSys s, const doubl
 // Thread 0 receives, per code, the sum of the energies in (code, pair index) order and a flag for
 // a pair that stays non-finite (the reference's -1 sentinel); the deferred list is reset.
 // Returns the number of deferred pairs (DEFER_CAP exceeded when larger). The count is read and
-// reset with atomics: in the batched minimizer the pairs were pushed by other waves of the same
-// workgroup within the kernel.
-// run_defers_eval: the energies alone (into each entry's U); defer_sums: the sums by one thread;
-// run_defers_n: both and the reset, with the count n already read (by every thread).
-template <int NTH = BLOCK>
-__device__ inline void run_defers_eval(const DevSys& s, int n, double* lds) {
+// reset with atomics: in the persistent minimizer any workgroup of the team pushes pairs within the
+// kernel (they are visible after its barrier).
+// run_defers_eval: the energies alone (into each entry's U), by NTH threads that sum the samples as
+// VT threads do (block_reduce_n's order), so that a team's energies are the finalize kernel's bit for
+// bit; defer_sums: the sums by one thread; run_defers_n: both and the reset, with the count n already
+// read (by every thread).
+template <int NTH = BLOCK, int VT = NTH>
+__device__ inline void run_defers_eval(const DevSys& s, int n, double* lds /* >= VT / 64 */) {
+    static_assert(VT % NTH == 0, "whole rounds of the block");
+    constexpr int NW = NTH / 64;
     const int m = min(n, DEFER_CAP);
-    const int op1[1] = {0};
     for (int k = 0; k < m; k++) {
         EnDefer& e = s.defer[k];
         const D3 c1{e.c[0], e.c[1], e.c[2]}, c2{e.c[3], e.c[4], e.c[5]}, c3{e.c[6], e.c[7], e.c[8]},
             c4{e.c[9], e.c[10], e.c[11]};
-        double r = exvol_energyN_share(c1, c2, c3, c4, threadIdx.x, NTH);
-        block_reduce_n<1, NTH>(&r, op1, lds);
-        if (threadIdx.x == 0) e.U = exvol_energyN_finish(c1, c2, c3, c4, e.ks, r);
+        double r[VT / NTH];
+        for (int h = 0; h < VT / NTH; h++) r[h] = wave_sum(exvol_energyN_share(c1, c2, c3, c4, threadIdx.x + h * NTH, VT));
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0)
+            for (int h = 0; h < VT / NTH; h++) lds[h * NW + (threadIdx.x >> 6)] = r[h];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double sum = lds[0];
+            for (int q = 1; q < VT / 64; q++) sum += lds[q];
+            e.U = exvol_energyN_finish(c1, c2, c3, c4, e.ks, sum);
+        }
     }
 }
 __device__ inline void defer_sums(const DevSys& s, int m, double* sum, int* badc, int ncode) {

@@ -90,7 +90,7 @@ struct TeamShared {
     CgState S;
     double fold[8 * (FIN / 8)];
     double res[8];
-    double red[16];
+    double red[FIN / 64];
     int bad, ndef, ok, k;
 };
 
@@ -579,7 +579,7 @@ __device__ inline bool team_fin(const DevSys& s, const CgBufs& B, TeamShared& sh
     const bool reset = bad0 != 0 || ndef > 0;   // the same in every workgroup
     if (ls && ndef > 0) {
         // the deferred Simpson energies: one workgroup evaluates them, all read its results
-        if (t.member == 0) run_defers_eval<NT>(s, ndef, sh.red);
+        if (t.member == 0) run_defers_eval<NT, SUM == SUM_SLOTS ? FIN : SUM_NT>(s, ndef, sh.red);
         if (!team_barrier<true>(t, sh)) return false;
         if (threadIdx.x == 0) defer_sums(s, min(ndef, DEFER_CAP), dsum, dbad, 3);
     }
