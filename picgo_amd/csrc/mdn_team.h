@@ -490,7 +490,7 @@ __device__ inline void team_columns(const DevSys& s, TeamShared& sh, const doubl
         double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (64 * vw < nmax) {
             auto ecol = [&](int c) { return 4L * (c < ne0 ? c : T + (c - ne0)); };
-            const double* e = wen + ecol(min(v, ne - 1));
+            const double* e = wen + ecol(max(0, min(v, ne - 1)));   // (a network may have no interactions)
             const double* p = wpos + 4L * min(v, s.nbb - 1);
             const double* g = wg + min(v, ngb - 1);
             double x[12], y[3];
