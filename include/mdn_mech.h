@@ -260,6 +260,12 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* params, double* coord, doubl
  * out[3] CG iterations. */
 int mdn_last_min_stats(mdn_ctx* ctx, int64_t* out);
 
+/* How the last minimization on this context (of a batch: on its lead context) ran: out2[0] the
+ * workgroups that minimized in teams (mdn_minimize: of the team, 0: kernels without waits; a batch:
+ * of all teams of more than one), out2[1] the systems taken over from a team that gave up waiting
+ * for its workgroups. Neither changes a result. */
+int mdn_last_team(mdn_ctx* ctx, int32_t* out2);
+
 /* ---- device-resident variants (benchmarking, zero host traffic) ---------------------- */
 
 /* Time `iters` force evaluations (mdn_forces semantics) on the context's current device

@@ -165,6 +165,9 @@ struct mdn_ctx {
 
     DBuf<double> team_part;   // wavefront partials of the persistent minimizer
     int team_size = -1;       // workgroups of the persistent minimizer: -1 by size, 0 never (MDN_CG_TEAM)
+    int team_stride = 8, team_polls = TEAM_START_POLLS;   // MDN_TEAM_STRIDE, MDN_TEAM_POLLS
+    int n_cu = 0;             // the device's
+    int last_team[2] = {0, 0};   // mdn_last_team
     // batched minimizer (the lead context of a batch owns these)
     DBuf<TeamSlot> batch_slot;
     DBuf<TeamInfo> batch_team;
@@ -173,8 +176,7 @@ struct mdn_ctx {
     DBuf<CgState> batch_states;   // the batch's final states and reports, gathered for one read-back
     DBuf<double> batch_reports;
     DBuf<int> batch_order, batch_queue;
-    DBuf<BatchCopy> batch_copy;   // [start copies | start backups | restores], one per system each
-    int batch_nt = TEAM_NT;
+    DBuf<BatchCopy> batch_copy;   // start copies, backups
 
     bool use_graph = true;   // replay the CG slots as a captured hipGraph (MDN_CG_GRAPH=0: launch them directly)
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};   // per precision (MDN_PREC_*)
@@ -760,7 +762,14 @@ int mdn_ctx_create(int device, mdn_ctx** out) {
     // workgroups of one XCD for every network; unset: by the network's size (team_workgroups)
     // (the result does not depend on it)
     if (const char* env = getenv("MDN_CG_TEAM")) ctx->team_size = std::max(0, std::min(TEAM_MAX, atoi(env)));
-    if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
+    // for tests, at context creation: MDN_TEAM_POLLS = a team's wait for its workgroups at the start,
+    // in polls (0: whoever is not the last gives up, -1: everyone does); MDN_TEAM_STRIDE = the distance of a single network's team
+    // members in the grid (8: one XCD; 1: spread over all of them). The result depends on neither.
+    if (const char* env = getenv("MDN_TEAM_POLLS")) ctx->team_polls = std::max(-1, std::min(TEAM_START_POLLS, atoi(env)));
+    if (const char* env = getenv("MDN_TEAM_STRIDE")) ctx->team_stride = std::max(1, std::min(8, atoi(env)));
+    if (hipSetDevice(device) != hipSuccess ||
+        hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
         return MDN_ERR_HIP;
     }
@@ -2017,35 +2026,18 @@ static int cg_graph(mdn_ctx* ctx, int prec) {
     return MDN_OK;
 }
 
-// The work of a network in the persistent minimizer, in beads: an excluded-volume pair costs what
-// about eight beads do.
+// The work of a network in the persistent minimizer, in beads: in a batch an excluded-volume pair
+// costs what about eight beads do.
 static long team_cost(const DevSys& s) {
     return s.n_beads + s.n[FF_LINKER] + s.n[FF_MOTOR] + 8L * s.n[FF_EXVOL] + s.n[FF_BOUNDARY];
 }
-// Work per workgroup below which another workgroup does not pay: batches of 8, 16 and 48 networks
-// of up to 12,000 beads take 2.3, 2.6 and 4.4 ms with 256, 2.8, 3.0 and 4.7 ms with 1024, 3.5, 3.8
-// and 5.7 ms with 2048.
-static const long TEAM_SHARE = 256;
-// A single network's work, in which a pair counts less than in a batch (its two chains run side by
-// side): TEAM_ONE_SHARE of it per workgroup up to 16 workgroups, 24 from TEAM_WIDE on (below, their
-// dearer barriers count more than the work they share) and from TEAM_ONE_MAX on the four-kernel
-// slots over the whole chip. FP64 / mixed, ms per 80 iterations without the rebuild:
-//   550 beads, work 1,200: 6, 8, 10 and 16 workgroups 1.30, 1.32, 1.36, 1.39 / 1.41, 1.41, 1.41, 1.44
-//   4,200 in a sphere, 8,800: 16 and 24 workgroups 1.73, 1.67 / 1.60, 1.72
-//   7,350 in a sphere, 13,900: 16, 24, 32, slots 2.13, 1.87, 1.91, 2.02 / 1.95, 1.87, 1.82, 2.17
-//   3,150 in a cube, 14,200: 2.19, 1.93, 1.94, 2.12 / 2.01, 1.84, 1.90, 2.17
-//   9,450 in a sphere, 19,100: 2.50, 2.11, 2.06, 2.04 / 2.23, 1.94, 2.01, 2.10
-//   4,830 in a cube, 21,200: 2.69, 2.36, 2.22, 2.17 / 2.28, 2.18, 2.07, 2.17
 static long team_one_work(const DevSys& s) {
     return s.n_beads + s.n[FF_LINKER] + s.n[FF_MOTOR] + 2L * s.n[FF_EXVOL] + s.n[FF_BOUNDARY];
 }
-static const long TEAM_ONE_SHARE = 160, TEAM_WIDE = 9000, TEAM_ONE_MAX = 17500;
 // Workgroups of the persistent minimizer for a single network; 0: the four-kernel slots.
 static int team_workgroups(const mdn_ctx* ctx) {
     if (!cg_bonded_sums(ctx, 0) || ctx->n_beads >= GB_LARGE_BEADS) return 0;
-    if (ctx->team_size >= 0) return ctx->team_size;
-    const long c = team_one_work(ctx->sys);
-    return c > TEAM_ONE_MAX ? 0 : c > TEAM_WIDE ? 24 : (int)std::min<long>(16, (c + TEAM_ONE_SHARE - 1) / TEAM_ONE_SHARE);
+    return ctx->team_size >= 0 ? ctx->team_size : team_size_one(team_one_work(ctx->sys));
 }
 
 // The persistent minimizer on one system from its device state until that is done. The barrier's
@@ -2056,13 +2048,13 @@ static int launch_team(mdn_ctx* ctx, int prec, int size) {
     CgState* st = ctx->cg.p;
     TeamCtl* ctl = team_ctl(st);
     double* wp = ctx->team_part.p;
-    int stride = size > 1 ? 8 : 1;
-    void* args[] = {&s, &B, &st, &ctl, &wp, &size, &stride};
+    int stride = size > 1 ? ctx->team_stride : 1, polls = ctx->team_polls;
+    void* args[] = {&s, &B, &st, &ctl, &wp, &size, &stride, &polls};
     const dim3 g(stride * (size - 1) + 1), b(TEAM_NT);
     auto launch = [&](auto k) {
         // the workgroups of a team wait for each other: a cooperative launch has them all resident
         if (size > 1) return hipLaunchCooperativeKernel(k, g, b, args, 0, ctx->stream);
-        hipLaunchKernelGGL(k, g, b, 0, ctx->stream, s, B, st, ctl, wp, size, stride);
+        hipLaunchKernelGGL(k, g, b, 0, ctx->stream, s, B, st, ctl, wp, size, stride, polls);
         return hipGetLastError();
     };
     if (prec == MDN_PREC_MIXED) HIPCHK(launch(k_cg_team_one<float, TEAM_NT>));
@@ -2070,18 +2062,29 @@ static int launch_team(mdn_ctx* ctx, int prec, int size) {
     return MDN_OK;
 }
 
-int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* force_out, mdn_min_result* res) {
-    int st = need_system(ctx, true);
-    if (st) return st;
-    if (!p || !res) return fail(ctx, MDN_ERR_ARG, "null argument");
-    if (p->precision != MDN_PREC_FP64 && p->precision != MDN_PREC_MIXED)
-        return fail(ctx, MDN_ERR_ARG, "unknown precision %d", p->precision);
+// The two events that mark the last batches of slots.
+struct SlotEvents {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    hipError_t create() {
+        const hipError_t r = hipEventCreateWithFlags(&e[0], hipEventDisableTiming);
+        return r != hipSuccess ? r : hipEventCreateWithFlags(&e[1], hipEventDisableTiming);
+    }
+    ~SlotEvents() {
+        for (hipEvent_t v : e)
+            if (v) (void)hipEventDestroy(v);
+    }
+};
+
+// One minimization. With teams, by a team where that is the faster form; *gave_up: its workgroups
+// waited for each other too long, and the start is as it was (coord has not been written; without it
+// the device coordinates are put back).
+static int minimize_run(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* force_out, mdn_min_result* res,
+                        bool teams, bool* gave_up) {
+    int st;
     const int prec = p->precision;
-    if (p->method < 0 || p->method > 2) return fail(ctx, MDN_ERR_ARG, "unknown descent method %d", p->method);
-    if (p->line_search != MDN_LS_BACKTRACKING && p->line_search != MDN_LS_QUADRATIC)
-        return fail(ctx, MDN_ERR_ARG, "unknown line search %d", p->line_search);
-    HIPCHK(hipSetDevice(ctx->device));
     memset(res, 0, sizeof(*res));
+    ctx->last_team[0] = 0;
+    ctx->last_team[1] = teams ? 0 : 1;
     const int nv = 3 * ctx->n_beads;
     // startMinimization + initial energy / forces (CGMethod.hpp:876-896); the start is in x[0]
     if (coord)
@@ -2149,12 +2152,15 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     HIPCHK(hipMemsetAsync(ctx->d[0].p, 0, sizeof(double) * nv, ctx->stream));   // searchDir.assign(numDof, 0)
     HIPCHK(hipMemcpyAsync(ctx->cg.p, &S, CG_BYTES, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
-    const int team = team_workgroups(ctx);
-    // The slots are captured into a graph once a layout is minimized a second time: a graph made
+    const int team = teams ? team_workgroups(ctx) : 0;
+    if (!S.done) ctx->last_team[0] = team;
+    if (team > 1 && !S.done && !coord)   // the start, should the team give up
+        HIPCHK(hipMemcpyAsync(ctx->ext.p, ctx->x[0].p, sizeof(double) * nv, hipMemcpyDeviceToDevice, ctx->stream));
+    // The slots are captured into a graph once they minimize a layout a second time: a graph made
     // for one minimization (a layout that the next neighbor-list rebuild replaces) costs more to
     // instantiate than its replays save over launching the same kernels directly.
     const bool graph = !team && ctx->use_graph && (ctx->graph_gen[prec] == ctx->sys_gen || ctx->min_gen[prec] == ctx->sys_gen);
-    ctx->min_gen[prec] = ctx->sys_gen;
+    if (!team) ctx->min_gen[prec] = ctx->sys_gen;
     if (graph && (st = cg_graph(ctx, prec))) return st;
     const DevSys slot_sys = cg_sys(ctx, prec);
     const CgBufs slot_bufs = cg_bufs(ctx);
@@ -2168,9 +2174,8 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     const int per = graph ? CG_BATCH : LAUNCH_BATCH;
     const long max_batches = ((slots_per_force_call(S) * ((long)S.force_call_limit + 16)) / CG_BATCH + 8) * (CG_BATCH / per);
     long launched = 0;
-    hipEvent_t ev[2];
-    HIPCHK(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
+    SlotEvents ev;
+    if (!team) HIPCHK(ev.create());
     int n_forcen = 0;
     for (;;) {
         bool done = S.done != 0;
@@ -2196,16 +2201,22 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
             }
             launched++;
             here++;
-            HIPCHK(hipEventRecord(ev[k], ctx->stream));
+            HIPCHK(hipEventRecord(ev.e[k], ctx->stream));
             if (here > 1) {
                 if (launched == 2 && force_out) map_pages(force_out, sizeof(double) * nv);   // while the device works
-                HIPCHK(hipEventSynchronize(ev[k ^ 1]));
+                HIPCHK(hipEventSynchronize(ev.e[k ^ 1]));
                 if (*h_done) done = true;
             }
             k ^= 1;
         }
         HIPCHK(d2h(ctx, ctx->h_cg, ctx->cg.p, CG_BYTES));
-        if (team_ctl(ctx->h_cg)->failed) return fail(ctx, MDN_ERR_STATE, "a workgroup of the minimizer gave up waiting for the others");
+        if (team_ctl(ctx->h_cg)->failed) {
+            HIPCHK(hipMemsetAsync(ctx->defer_n.p, 0, sizeof(int), ctx->stream));   // (bad_count: cleared by the evaluation)
+            if (!coord)
+                HIPCHK(hipMemcpyAsync(ctx->x[0].p, ctx->ext.p, sizeof(double) * nv, hipMemcpyDeviceToDevice, ctx->stream));
+            *gave_up = true;
+            return MDN_OK;
+        }
         if (!(S.done && S.status == ST_NEED_FORCEN)) break;
         // The step's forces need the numerical excluded-volume fallback (forceN,
         // CylinderExclVolRepulsion.cpp:984-1254): recompute them at the new coordinates with it
@@ -2229,8 +2240,6 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
         // before the pinned copy is overwritten
         HIPCHK(d2h(ctx, &S, ctx->cg.p, sizeof(CgState)));
     }
-    (void)hipEventDestroy(ev[0]);
-    (void)hipEventDestroy(ev[1]);
     ctx->last_cg = S;
     if (!S.done) return fail(ctx, MDN_ERR_STATE, "minimizer did not terminate within %ld batches", launched);
     ctx->cur = S.parity;
@@ -2269,6 +2278,21 @@ int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* fo
     return MDN_OK;
 }
 
+int mdn_minimize(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, double* force_out, mdn_min_result* res) {
+    int st = need_system(ctx, true);
+    if (st) return st;
+    if (!p || !res) return fail(ctx, MDN_ERR_ARG, "null argument");
+    if (p->precision != MDN_PREC_FP64 && p->precision != MDN_PREC_MIXED)
+        return fail(ctx, MDN_ERR_ARG, "unknown precision %d", p->precision);
+    if (p->method < 0 || p->method > 2) return fail(ctx, MDN_ERR_ARG, "unknown descent method %d", p->method);
+    if (p->line_search != MDN_LS_BACKTRACKING && p->line_search != MDN_LS_QUADRATIC)
+        return fail(ctx, MDN_ERR_ARG, "unknown line search %d", p->line_search);
+    HIPCHK(hipSetDevice(ctx->device));
+    bool gave_up = false;
+    st = minimize_run(ctx, p, coord, force_out, res, true, &gave_up);
+    return gave_up ? minimize_run(ctx, p, coord, force_out, res, false, &gave_up) : st;
+}
+
 }  // extern "C"
 
 // ----------------------------------------------------------------------------------------
@@ -2297,58 +2321,6 @@ static void fill_result(const CgState& S, const double* rep_before, const double
     res->restored_min_energy = S.reserved[0];
 }
 
-// A batch's workgroups: which team each is in, and which system each team has. Large systems get
-// teams of their own, sized to their share of the work; the others are pulled from a queue,
-// largest first, by single workgroups. A workgroup b runs on XCD b % 8, and a team's workgroups
-// are taken from one XCD.
-struct TeamPlan {
-    std::vector<TeamSlot> slot;
-    std::vector<TeamInfo> team;
-    std::vector<int> order;   // the queue
-    bool wait = false;        // some team has more than one workgroup
-};
-static TeamPlan plan_teams(const std::vector<long>& cost, int groups) {
-    const int n = (int)cost.size(), NX = 8;
-    TeamPlan P;
-    std::vector<int> room(NX, 0);
-    for (int b = 0; b < groups; b++) room[b % NX]++;
-    long total = 0;
-    for (long c : cost) total += c;
-    std::vector<int> k(n, 1), by(n);
-    for (int i = 0; i < n; i++) by[i] = i;
-    std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    // the share of work per workgroup, raised until the teams and the queue's workgroups fit
-    for (double share = std::max<double>(TEAM_SHARE, (double)total / groups);; share *= 1.1) {
-        int used = 0, small = 0;
-        double rest = 0;
-        for (int i = 0; i < n; i++) {
-            k[i] = (int)std::max(1.0, std::min<double>(std::min(TEAM_MAX, room[0]), std::ceil(cost[i] / share)));
-            if (k[i] > 1) used += k[i];
-            else { small++; rest += cost[i]; }
-        }
-        if (used + std::min<double>(small, std::ceil(rest / share)) <= groups) break;
-    }
-    P.slot.assign(groups, TeamSlot{-1, 0});
-    std::vector<int> taken(NX, 0);
-    auto place = [&](int want, int sys) {   // a team of `want` workgroups on the XCD with the most room
-        int x = 0;
-        for (int q = 1; q < NX; q++)
-            if (room[q] - taken[q] > room[x] - taken[x]) x = q;
-        const int size = std::min(want, room[x] - taken[x]);
-        if (size <= 0) return false;
-        for (int m = 0; m < size; m++) P.slot[x + NX * (taken[x] + m)] = TeamSlot{(int)P.team.size(), m};
-        taken[x] += size;
-        P.team.push_back(TeamInfo{size, sys});
-        P.wait = P.wait || size > 1;
-        return true;
-    };
-    for (int i : by)
-        if (k[i] == 1 || !place(k[i], i)) P.order.push_back(i);
-    for (size_t j = 0; j < P.order.size(); j++)
-        if (!place(1, -1)) break;
-    return P;
-}
-
 // One system's coordinates or forces: among the parts that go through the ring together, or, from
 // pinned or device memory (which the ring's copies by the CPU must not touch), queued by the runtime.
 static hipError_t batch_copy(mdn_ctx* L, std::vector<HostCopy>& parts, double* host, double* dev, size_t bytes, bool to_host) {
@@ -2366,13 +2338,13 @@ static int launch_batch(mdn_ctx* L, const TeamPlan& P, int prec) {
     const TeamInfo* team = L->batch_team.p;
     TeamCtl* ctl = L->batch_ctl.p;
     const int* order = L->batch_order.p;
-    int n = (int)P.order.size();
+    int n = (int)P.order.size(), polls = L->team_polls;
     int* queue = L->batch_queue.p;
-    void* args[] = {&items, &slot, &team, &ctl, &order, &n, &queue};
+    void* args[] = {&items, &slot, &team, &ctl, &order, &n, &queue, &polls};
     const dim3 g(P.slot.size()), b(TEAM_NT);
     auto launch = [&](auto k) {
-        if (P.wait) return hipLaunchCooperativeKernel(k, g, b, args, 0, L->stream);
-        hipLaunchKernelGGL(k, g, b, 0, L->stream, items, slot, team, ctl, order, n, queue);
+        if (P.teamed > 0) return hipLaunchCooperativeKernel(k, g, b, args, 0, L->stream);
+        hipLaunchKernelGGL(k, g, b, 0, L->stream, items, slot, team, ctl, order, n, queue, polls);
         return hipGetLastError();
     };
     if (prec == MDN_PREC_MIXED) HIPCHK_CTX(L, launch(k_cg_team<float, TEAM_NT>));
@@ -2382,35 +2354,20 @@ static int launch_batch(mdn_ctx* L, const TeamPlan& P, int prec) {
 
 extern "C" {
 
-int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p, double* const* coords,
-                         double* const* forces_out, mdn_min_result* results) {
-    if (!ctxs || n <= 0 || !ctxs[0]) return MDN_ERR_ARG;
-    mdn_ctx* L = ctxs[0];
-    if (!p || !coords || !results) return fail(L, MDN_ERR_ARG, "null argument");
-    if (p->precision != MDN_PREC_FP64 && p->precision != MDN_PREC_MIXED)
-        return fail(L, MDN_ERR_ARG, "unknown precision %d", p->precision);
-    if (p->method < 0 || p->method > 2) return fail(L, MDN_ERR_ARG, "unknown descent method %d", p->method);
-    if (p->line_search != MDN_LS_BACKTRACKING && p->line_search != MDN_LS_QUADRATIC)
-        return fail(L, MDN_ERR_ARG, "unknown line search %d", p->line_search);
-    long beads = 0;
-    for (int i = 0; i < n; i++) {
-        mdn_ctx* c = ctxs[i];
-        if (!c) return fail(L, MDN_ERR_ARG, "system %d: null context", i);
-        if (c->device != L->device) return fail(L, MDN_ERR_ARG, "system %d is on another device", i);
-        for (int j = 0; j < i; j++)
-            if (ctxs[j] == c) return fail(L, MDN_ERR_ARG, "system %d repeats context %d", i, j);
-        int st = need_system(c, true);
-        if (st) return fail(L, st, "system %d: %s", i, c->err.c_str());
-        beads += c->n_beads;
-    }
-    HIPCHK_CTX(L, hipSetDevice(L->device));
+// One batch on the lead context L's stream and buffers. code[i]: system i's status. With teams, large
+// systems by teams; again: the systems whose team gave up waiting for its workgroups, each at its
+// start (their results are not set).
+static int batched_run(mdn_ctx* L, mdn_ctx* const* ctxs, int n, const mdn_cg_params* p, double* const* coords,
+                       double* const* forces_out, mdn_min_result* results, int* code, bool teams, std::vector<int>* again) {
     // every context's own work is complete before the lead stream reads its buffers
-    for (int i = 1; i < n; i++) HIPCHK_CTX(L, hipStreamSynchronize(ctxs[i]->stream));
+    for (int i = 0; i < n; i++)
+        if (ctxs[i] != L) HIPCHK_CTX(L, hipStreamSynchronize(ctxs[i]->stream));
     std::vector<BatchItem> items(n);
     std::vector<long> cost(n);
-    // the systems that start from their device coordinates: x[cur] -> x[0], all in one launch (a
-    // zero count copies nothing)
-    std::vector<BatchCopy> copies((size_t)n);
+    // the systems that start from their device coordinates: x[cur] -> x[0], and where a team takes
+    // them into ext, all in one launch
+    std::vector<BatchCopy> copies;
+    std::vector<const double*> start(n, nullptr);
     std::vector<HostCopy> in;   // what goes onto the device: the given coordinates, then the tables
     long max_nv = 1;
     int max_blk = 1, max_nbb = 1, max_terms = 1;
@@ -2420,8 +2377,9 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         max_nv = std::max(max_nv, nv);
         if (coords[i])
             HIPCHK_CTX(L, batch_copy(L, in, coords[i], c->x[0].p, sizeof(double) * nv, false));
-        else if (c->cur != 0)   // the context's device coordinates
-            copies[i] = BatchCopy{c->x[c->cur].p, c->x[0].p, nv};
+        else   // the context's device coordinates
+            start[i] = c->x[c->cur].p;
+        if (start[i] && c->cur != 0) copies.push_back(BatchCopy{start[i], c->x[0].p, nv});
         c->cur = 0;
         BatchItem& it = items[i];
         it.s = c->sys;
@@ -2450,17 +2408,18 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     P.energy_rel_tol = p->energy_rel_tol;
     // one workgroup per CU (8 wavefronts at 179 to 250 VGPRs fill it); MDN_BATCH_MAX_WORKGROUPS caps
     // them, so that every workgroup pulls several systems (what a batch larger than the chip does)
-    int n_cu = 0;
-    HIPCHK_CTX(L, hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, L->device));
-    int groups = std::max(1, n_cu);
+    int groups = std::max(1, L->n_cu);
     if (const char* env = getenv("MDN_BATCH_MAX_WORKGROUPS"))
         if (atoi(env) > 0) groups = std::min(groups, atoi(env));
-    const TeamPlan plan = plan_teams(cost, groups);
+    const TeamPlan plan = plan_teams(cost, groups, teams ? TEAM_MAX : 1);
+    for (const TeamInfo& t : plan.team)
+        if (t.size > 1 && start[t.sys])
+            copies.push_back(BatchCopy{start[t.sys], ctxs[t.sys]->ext.p, 3L * ctxs[t.sys]->n_beads});
     const size_t nq = std::max<size_t>(1, plan.order.size());
     HIPCHK_CTX(L, L->batch_items.ensure(n));
     HIPCHK_CTX(L, L->batch_order.ensure(nq));
     HIPCHK_CTX(L, L->batch_queue.ensure(1));
-    HIPCHK_CTX(L, L->batch_copy.ensure((size_t)n));
+    HIPCHK_CTX(L, L->batch_copy.ensure(std::max<size_t>(1, copies.size())));
     HIPCHK_CTX(L, L->batch_slot.ensure(plan.slot.size()));
     HIPCHK_CTX(L, L->batch_team.ensure(plan.team.size()));
     HIPCHK_CTX(L, L->batch_ctl.ensure(plan.team.size()));
@@ -2468,7 +2427,7 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         if (bytes) in.push_back(HostCopy{(char*)host, (char*)dev, bytes});
     };
     table(L->batch_items.p, items.data(), sizeof(BatchItem) * n);
-    table(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * n);
+    table(L->batch_copy.p, copies.data(), sizeof(BatchCopy) * copies.size());
     table(L->batch_slot.p, plan.slot.data(), sizeof(TeamSlot) * plan.slot.size());
     table(L->batch_team.p, plan.team.data(), sizeof(TeamInfo) * plan.team.size());
     table(L->batch_order.p, plan.order.data(), sizeof(int) * plan.order.size());
@@ -2476,9 +2435,12 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     HIPCHK_CTX(L, hipMemsetAsync(L->batch_ctl.p, 0, sizeof(TeamCtl) * plan.team.size(), L->stream));
     HIPCHK_CTX(L, hipMemsetAsync(L->batch_queue.p, 0, sizeof(int), L->stream));
     const BatchItem* di = L->batch_items.p;
-    const dim3 cgrid((unsigned)std::min(64L, std::max(1L, (long)ceil_div(max_nv, 256L))), (unsigned)std::min(n, 4096));
     int st;
-    hipLaunchKernelGGL(k_batch_copy, cgrid, dim3(256), 0, L->stream, (const BatchCopy*)L->batch_copy.p, n);
+    if (!copies.empty()) {
+        const dim3 cgrid((unsigned)std::min(64L, std::max(1L, (long)ceil_div(max_nv, 256L))),
+                         (unsigned)std::min<size_t>(copies.size(), 4096));
+        hipLaunchKernelGGL(k_batch_copy, cgrid, dim3(256), 0, L->stream, (const BatchCopy*)L->batch_copy.p, (int)copies.size());
+    }
     // a grid's second dimension holds at most 65535 systems: the launches below go in parts
     for (int i0 = 0; i0 < n; i0 += 32768) {
         const unsigned m = (unsigned)std::min(n - i0, 32768);
@@ -2524,10 +2486,25 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
                               {(char*)ctl.data(), (char*)L->batch_ctl.p, sizeof(TeamCtl) * ctl.size()},
                               {(char*)reports.data(), (char*)L->batch_reports.p, sizeof(double) * 27 * n}};
     HIPCHK_CTX(L, copy_parts(L, head, 3, true));
-    for (const TeamCtl& c : ctl)
-        if (c.failed) return fail(L, MDN_ERR_STATE, "a workgroup of the minimizer gave up waiting for the others");
+    std::vector<char> failed(n, 0);
+    for (size_t t = 0; t < plan.team.size(); t++) {
+        const int i = plan.team[t].sys;
+        if (!ctl[t].failed || i < 0) continue;   // (a workgroup that pulls systems waits for nobody)
+        failed[i] = 1;
+        again->push_back(i);
+        HIPCHK_CTX(L, hipMemsetAsync(ctxs[i]->defer_n.p, 0, sizeof(int), L->stream));
+        if (start[i])
+            HIPCHK_CTX(L, hipMemcpyAsync(ctxs[i]->x[0].p, ctxs[i]->ext.p, sizeof(double) * 3 * ctxs[i]->n_beads,
+                                         hipMemcpyDeviceToDevice, L->stream));
+    }
+    std::sort(again->begin(), again->end());
+    if (teams) {
+        L->last_team[0] = plan.teamed;
+        L->last_team[1] = (int)again->size();
+    }
     std::vector<HostCopy> out;
     for (int i = 0; i < n; i++) {
+        if (failed[i]) continue;
         mdn_ctx* c = ctxs[i];
         const CgState& S = states[i];
         const size_t bytes = sizeof(double) * 3 * c->n_beads;
@@ -2537,8 +2514,8 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
     }
     HIPCHK_CTX(L, copy_parts(L, out.data(), (int)out.size(), true));
     HIPCHK_CTX(L, hipStreamSynchronize(L->stream));
-    int first_err = MDN_OK;
     for (int i = 0; i < n; i++) {
+        if (failed[i]) continue;
         mdn_ctx* c = ctxs[i];
         const CgState& S = states[i];
         const double* rep = reports.data() + 27L * i;
@@ -2546,38 +2523,86 @@ int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p
         c->cur = S.parity;
         const bool ok = S.status == 0 && S.error_flags == 0;
         fill_result(S, rep, rep + 9, ok, &results[i]);
-        int code = MDN_OK;
         if (S.status != 0) {
-            code = (S.status == ST_NEED_FORCEN || S.status == 9) ? MDN_ERR_UNSUPPORTED : S.status;
-            fail(c, code, S.status == ST_NEED_FORCEN ? "an excluded-volume pair needed the numerical force fallback, "
+            code[i] = (S.status == ST_NEED_FORCEN || S.status == 9) ? MDN_ERR_UNSUPPORTED : S.status;
+            fail(c, code[i], S.status == ST_NEED_FORCEN ? "an excluded-volume pair needed the numerical force fallback, "
                                                        "which the batched minimizer does not run"
                           : S.status == 9 ? "more excluded-volume pairs need the Simpson energy than the capacity"
                                           : "minimization stopped with status %d", S.status);
         } else if (ok && rep[9 + 8] != 0.0) {
-            code = MDN_ERR_UNSUPPORTED;
-            fail(c, code, "excluded-volume pairs beyond the Simpson-energy capacity");
+            code[i] = MDN_ERR_UNSUPPORTED;
+            fail(c, code[i], "excluded-volume pairs beyond the Simpson-energy capacity");
         } else if (S.error_flags & MDN_MIN_ERR_LINESEARCH) {
-            code = MDN_ERR_LINESEARCH;
-            fail(c, code, "line search failed (recovery disabled)");
-        }
-        if (code != MDN_OK && first_err == MDN_OK) {
-            first_err = code;
-            if (c != L) fail(L, code, "system %d: %s", i, c->err.c_str());
+            code[i] = MDN_ERR_LINESEARCH;
+            fail(c, code[i], "line search failed (recovery disabled)");
         }
     }
-    return first_err;
+    return MDN_OK;
 }
 
-// The schedule of the last batched minimization on a lead context: [workgroup size,
-// largest-first order (1) or given order (0), tuned in that call (1) or reused (0)], and the
-// tuning times (ms) of the candidates (128, 256, 512, 1024 threads, each in given then sorted order).
+int mdn_minimize_batched(mdn_ctx* const* ctxs, int32_t n, const mdn_cg_params* p, double* const* coords,
+                         double* const* forces_out, mdn_min_result* results) {
+    if (!ctxs || n <= 0 || !ctxs[0]) return MDN_ERR_ARG;
+    mdn_ctx* L = ctxs[0];
+    if (!p || !coords || !results) return fail(L, MDN_ERR_ARG, "null argument");
+    if (p->precision != MDN_PREC_FP64 && p->precision != MDN_PREC_MIXED)
+        return fail(L, MDN_ERR_ARG, "unknown precision %d", p->precision);
+    if (p->method < 0 || p->method > 2) return fail(L, MDN_ERR_ARG, "unknown descent method %d", p->method);
+    if (p->line_search != MDN_LS_BACKTRACKING && p->line_search != MDN_LS_QUADRATIC)
+        return fail(L, MDN_ERR_ARG, "unknown line search %d", p->line_search);
+    for (int i = 0; i < n; i++) {
+        mdn_ctx* c = ctxs[i];
+        if (!c) return fail(L, MDN_ERR_ARG, "system %d: null context", i);
+        if (c->device != L->device) return fail(L, MDN_ERR_ARG, "system %d is on another device", i);
+        for (int j = 0; j < i; j++)
+            if (ctxs[j] == c) return fail(L, MDN_ERR_ARG, "system %d repeats context %d", i, j);
+        int st = need_system(c, true);
+        if (st) return fail(L, st, "system %d: %s", i, c->err.c_str());
+    }
+    HIPCHK_CTX(L, hipSetDevice(L->device));
+    std::vector<int> code(n, MDN_OK), again;
+    int st = batched_run(L, ctxs, n, p, coords, forces_out, results, code.data(), true, &again);
+    if (st) return st;
+    if (!again.empty()) {   // by single workgroups, which wait for nobody
+        const int m = (int)again.size();
+        std::vector<mdn_ctx*> sub(m);
+        std::vector<double*> x(m), f(m);
+        std::vector<mdn_min_result> res(m);
+        std::vector<int> sub_code(m, MDN_OK), none;
+        for (int j = 0; j < m; j++) {
+            sub[j] = ctxs[again[j]];
+            x[j] = coords[again[j]];
+            f[j] = forces_out ? forces_out[again[j]] : nullptr;
+        }
+        if ((st = batched_run(L, sub.data(), m, p, x.data(), f.data(), res.data(), sub_code.data(), false, &none))) return st;
+        for (int j = 0; j < m; j++) {
+            results[again[j]] = res[j];
+            code[again[j]] = sub_code[j];
+        }
+    }
+    for (int i = 0; i < n; i++)   // the first failing system's status
+        if (code[i] != MDN_OK) {
+            if (ctxs[i] != L) fail(L, code[i], "system %d: %s", i, ctxs[i]->err.c_str());
+            return code[i];
+        }
+    return MDN_OK;
+}
+
+// [workgroup size, largest-first order (1), tuned in that call (0)]: fixed, and no times.
 int mdn_last_batch_schedule(mdn_ctx* ctx, int32_t* out3, double* tune_ms) {
     if (!ctx || !out3) return MDN_ERR_ARG;
-    out3[0] = ctx->batch_nt;
+    out3[0] = TEAM_NT;
     out3[1] = 1;
     out3[2] = 0;
     if (tune_ms)
         for (int c = 0; c < MDN_BATCH_CANDIDATES; c++) tune_ms[c] = 0.0;
+    return MDN_OK;
+}
+
+int mdn_last_team(mdn_ctx* ctx, int32_t* out2) {
+    if (!ctx || !out2) return MDN_ERR_ARG;
+    out2[0] = ctx->last_team[0];
+    out2[1] = ctx->last_team[1];
     return MDN_OK;
 }
 

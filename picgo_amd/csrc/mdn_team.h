@@ -34,6 +34,7 @@
 #pragma once
 
 #include "mdn_kernels.h"
+#include "mdn_team_plan.h"
 
 namespace mdn {
 
@@ -45,14 +46,6 @@ struct BatchItem {
     double* wpart;    // wavefront partials (team_wpart_doubles)
 };
 
-// One team: its workgroups and the system it owns (sys < 0: a single workgroup that pulls systems
-// from the queue).
-struct TeamInfo {
-    int size, sys;
-};
-struct TeamSlot {   // per workgroup: its team (< 0: none) and its place in it
-    int team, member;
-};
 // Barrier counter and the mask of the XCDs its members run on, a cache line each; zero at launch.
 struct TeamCtl {
     unsigned count, pad0[31];
@@ -64,12 +57,15 @@ struct TeamCtl {
 constexpr int TEAM_NT = 512;
 constexpr int SUM_NT = 512;        // the threads whose order SUM_STRIDED keeps
 enum { SUM_SLOTS = 0, SUM_STRIDED = 1 };
-constexpr int TEAM_MAX = 32;       // workgroups of a team: the CUs of an XCD
 constexpr int TEAM_GB = 64;        // beads per gather column (k_cg_gather below GB_LARGE_BEADS beads)
-// a barrier gives up after this many ticks of the 100 MHz clock (2 s; a phase takes microseconds)
-// and raises TeamCtl::failed: the kernel then ends instead of waiting for a workgroup that never
-// arrives
-constexpr long long TEAM_TICKS = 200000000LL;
+// A barrier gives up after this many polls of its counter (97 ns each) and raises TeamCtl::failed, at
+// which the others give up too: the kernel then ends instead of waiting for a workgroup that never
+// arrives, and the host minimizes without a team. Polls, not time: a queue that is taken off the
+// device and put back has not waited meanwhile. The first barrier waits until all workgroups are
+// resident, for as long as other kernels hold the CUs: 25 ms, after which the slots, whose
+// workgroups fit beside those kernels, are the better way. Beyond it every workgroup is resident
+// and arrives after microseconds, or up to tens of milliseconds with deferred Simpson energies.
+constexpr int TEAM_START_POLLS = 1 << 18, TEAM_POLLS = 1 << 24;
 
 // Wavefront partials of one slot parity: energies [3][4 columns], bead kernel [2][4 nbb], gather [3][ngb]
 MDN_HD inline long team_wpart_half(const DevSys& s) {
@@ -99,6 +95,7 @@ struct Team {
     TeamCtl* c;
     unsigned target;
     int size, member, gw, nw;
+    int polls;   // a barrier's limit
     bool local;
 };
 
@@ -116,6 +113,10 @@ __device__ inline float team_load(const float* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ inline bool team_failed(TeamCtl* c) {
+    return __hip_atomic_load(&c->failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
 // All of the team's stores before it are visible after it, to team_load and, with INV, to every
 // load. False (in every thread) when it gave up.
 template <bool INV>
@@ -130,10 +131,11 @@ __device__ inline bool team_barrier(Team& t, TeamShared& sh) {
     if (threadIdx.x == 0) {
         if (!t.local) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __hip_atomic_fetch_add(&t.c->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const long long t0 = wall_clock64();
         int ok = 1;
-        while (__hip_atomic_load(&t.c->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < t.target)
-            if (wall_clock64() - t0 > TEAM_TICKS) {
+        // (the difference: the counter may pass 2^32)
+        for (int k = 0; t.polls < 0 ||
+                        (int)(__hip_atomic_load(&t.c->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - t.target) < 0; k++)
+            if (k >= t.polls || ((k & 63) == 63 && team_failed(t.c))) {
                 ok = 0;
                 __hip_atomic_store(&t.c->failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
@@ -653,8 +655,10 @@ __device__ inline void team_run(const DevSys& s, const CgBufs& B, CgState* st, d
     __syncthreads();   // the shared state is reused by the next system
 }
 
-__device__ inline Team team_start(TeamCtl* c, int size, int member, TeamShared& sh, int nwaves) {
+// polls: the first barrier's limit. size 0: the team gave up, nothing is written.
+__device__ inline Team team_start(TeamCtl* c, int size, int member, TeamShared& sh, int nwaves, int polls) {
     Team t;
+    t.polls = polls;
     t.c = c;
     t.target = 0;
     t.size = size;
@@ -666,6 +670,7 @@ __device__ inline Team team_start(TeamCtl* c, int size, int member, TeamShared& 
         if (threadIdx.x == 0)
             __hip_atomic_fetch_or(&c->xmask, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (!team_barrier<false>(t, sh)) t.size = 0;
+        t.polls = TEAM_POLLS;
         if (threadIdx.x == 0)
             sh.k = __popc(__hip_atomic_load(&c->xmask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         __syncthreads();
@@ -679,10 +684,10 @@ __device__ inline Team team_start(TeamCtl* c, int size, int member, TeamShared& 
 // others end at once (workgroups go round-robin over the XCDs, so a stride of 8 keeps the team on one).
 template <typename R, int NT>
 __global__ void __launch_bounds__(NT) k_cg_team_one(DevSys s, CgBufs B, CgState* st, TeamCtl* ctl, double* wpart,
-                                                    int size, int stride) {
+                                                    int size, int stride, int polls) {
     __shared__ TeamShared sh;
     if (blockIdx.x % stride) return;
-    Team t = team_start(ctl, size, blockIdx.x / stride, sh, NT / 64);
+    Team t = team_start(ctl, size, blockIdx.x / stride, sh, NT / 64, polls);
     if (t.size == 0) return;
     team_run<R, NT, SUM_SLOTS>(s, B, st, wpart, t, sh);
 }
@@ -692,12 +697,12 @@ __global__ void __launch_bounds__(NT) k_cg_team_one(DevSys s, CgBufs B, CgState*
 template <typename R, int NT>
 __global__ void __launch_bounds__(NT) k_cg_team(const BatchItem* __restrict__ items, const TeamSlot* __restrict__ slot,
                                                 const TeamInfo* __restrict__ team, TeamCtl* ctl,
-                                                const int* __restrict__ order, int n, int* queue) {
+                                                const int* __restrict__ order, int n, int* queue, int polls) {
     __shared__ TeamShared sh;
     const TeamSlot me = slot[blockIdx.x];
     if (me.team < 0) return;
     const TeamInfo ti = team[me.team];
-    Team t = team_start(ctl + me.team, ti.size, me.member, sh, NT / 64);
+    Team t = team_start(ctl + me.team, ti.size, me.member, sh, NT / 64, polls);
     if (t.size == 0) return;
     for (;;) {
         int i = ti.sys;
@@ -853,8 +858,8 @@ __global__ void __launch_bounds__(256) k_batch_collect(const BatchItem* __restri
 }
 
 // One launch for the start copies of a whole batch (each system's device coordinates into its
-// x[0], the start's backup for the schedule tuning and its restores): copy i moves c[i].n doubles
-// from c[i].src to c[i].dst. Grid (blocks per copy, systems), both strided.
+// x[0], and into a backup where a team that gives up would leave them overwritten): copy i moves
+// c[i].n doubles from c[i].src to c[i].dst. Grid (blocks per copy, copies), both strided.
 struct BatchCopy {
     const double* src;
     double* dst;

@@ -29,7 +29,7 @@ EXPORTED = [
     "mdn_system_counts", "mdn_nl_build", "mdn_nl_pairs", "mdn_boundary_list", "mdn_energy",
     "mdn_forces", "mdn_ff_forces", "mdn_crosslink_stretch_forces", "mdn_minimize",
     "mdn_bench_forces", "mdn_bench_energy", "mdn_set_coords", "mdn_get_coords", "mdn_forces_mixed",
-    "mdn_last_min_stats", "mdn_energy_mixed", "mdn_minimize_batched", "mdn_last_batch_schedule",
+    "mdn_last_min_stats", "mdn_last_team", "mdn_energy_mixed", "mdn_minimize_batched", "mdn_last_batch_schedule",
     "mdn_param_grad", "mdn_hvp", "mdn_set_params", "mdn_boundary_load_forces", "mdn_crosslinks_update",
     "mdn_forces_noalloc", "mdn_displace", "mdn_perturb", "mdn_param_grad_mixed", "mdn_hvp_mixed",
     "mdn_dof_serialize", "mdn_binding_pairs", "mdn_bench_adjoint", "mdn_hvp_batch",
@@ -89,6 +89,7 @@ def lib():
         L.mdn_param_grad_mixed.argtypes = [C.c_void_p, dp, dp, C.c_int64]
         L.mdn_set_params.argtypes = [C.c_void_p, dp, dp, dp]
         L.mdn_last_min_stats.argtypes = [C.c_void_p, i64p]
+        L.mdn_last_team.argtypes = [C.c_void_p, i32p]
         L.mdn_forces_noalloc.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_int32]
         L.mdn_displace.argtypes = [C.c_void_p, C.c_void_p, C.c_int32]
         L.mdn_perturb.argtypes = [C.c_void_p, C.c_uint64, C.c_uint64, C.c_double]
@@ -273,6 +274,13 @@ class ForceFieldManager:
                                                    nm.ctypes.data_as(i32p), stride, lp.ctypes.data_as(dp),
                                                    lm.ctypes.data_as(dp)))
         return lp.reshape(nf, stride), lm.reshape(nf, stride)
+
+    def last_team(self):
+        """(workgroups that minimized in teams in the last minimization, systems taken over from a
+        team that gave up)."""
+        out = (C.c_int32 * 2)()
+        self._chk(self._L.mdn_last_team(self._h, out))
+        return out[0], out[1]
 
     def last_min_stats(self):
         out = (C.c_int64 * 4)()
