@@ -250,6 +250,8 @@ struct StagePool {
     int made = 0, users = 0;
 };
 StagePool g_stage[64];   // per device
+TeamRoom g_team_room[64];   // likewise
+TeamRoom* team_room_of(int device) { return device >= 0 && device < 64 ? &g_team_room[device] : nullptr; }
 StagePool* stage_pool(int device) { return device >= 0 && device < 64 ? &g_stage[device] : nullptr; }
 
 // the current device's ring for this call, or null
@@ -2037,28 +2039,25 @@ static long team_one_work(const DevSys& s) {
 // Workgroups of the persistent minimizer for a single network; 0: the four-kernel slots.
 static int team_workgroups(const mdn_ctx* ctx) {
     if (!cg_bonded_sums(ctx, 0) || ctx->n_beads >= GB_LARGE_BEADS) return 0;
-    return ctx->team_size >= 0 ? ctx->team_size : team_size_one(team_one_work(ctx->sys));
+    const int room = team_room(ctx->n_cu);
+    return ctx->team_size >= 0 ? std::min(ctx->team_size, room) : team_size_one(team_one_work(ctx->sys), room);
 }
 
 // The persistent minimizer on one system from its device state until that is done. The barrier's
-// words at team_ctl(cg) are zero.
+// words at team_ctl(cg) are zero. A team of more than one has its share of the device's TeamRoom.
 static int launch_team(mdn_ctx* ctx, int prec, int size) {
-    DevSys s = cg_sys(ctx, prec);
-    CgBufs B = cg_bufs(ctx);
-    CgState* st = ctx->cg.p;
-    TeamCtl* ctl = team_ctl(st);
-    double* wp = ctx->team_part.p;
-    int stride = size > 1 ? ctx->team_stride : 1, polls = ctx->team_polls;
-    void* args[] = {&s, &B, &st, &ctl, &wp, &size, &stride, &polls};
+    const DevSys s = cg_sys(ctx, prec);
+    const CgBufs B = cg_bufs(ctx);
+    const int stride = size > 1 ? ctx->team_stride : 1;
     const dim3 g(stride * (size - 1) + 1), b(TEAM_NT);
-    auto launch = [&](auto k) {
-        // the workgroups of a team wait for each other: a cooperative launch has them all resident
-        if (size > 1) return hipLaunchCooperativeKernel(k, g, b, args, 0, ctx->stream);
-        hipLaunchKernelGGL(k, g, b, 0, ctx->stream, s, B, st, ctl, wp, size, stride, polls);
-        return hipGetLastError();
-    };
-    if (prec == MDN_PREC_MIXED) HIPCHK(launch(k_cg_team_one<float, TEAM_NT>));
-    else HIPCHK(launch(k_cg_team_one<double, TEAM_NT>));
+    TeamCtl* ctl = team_ctl(ctx->cg.p);
+    if (prec == MDN_PREC_MIXED)
+        hipLaunchKernelGGL((k_cg_team_one<float, TEAM_NT>), g, b, 0, ctx->stream, s, B, ctx->cg.p, ctl, ctx->team_part.p, size,
+                           stride, ctx->team_polls);
+    else
+        hipLaunchKernelGGL((k_cg_team_one<double, TEAM_NT>), g, b, 0, ctx->stream, s, B, ctx->cg.p, ctl, ctx->team_part.p, size,
+                           stride, ctx->team_polls);
+    HIPCHK(hipGetLastError());
     return MDN_OK;
 }
 
@@ -2152,7 +2151,10 @@ static int minimize_run(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, dou
     HIPCHK(hipMemsetAsync(ctx->d[0].p, 0, sizeof(double) * nv, ctx->stream));   // searchDir.assign(numDof, 0)
     HIPCHK(hipMemcpyAsync(ctx->cg.p, &S, CG_BYTES, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->bad_count.p, 0, sizeof(int), ctx->stream));
-    const int team = teams ? team_workgroups(ctx) : 0;
+    // a team of several needs its share of the device's room for teams (none left: the slots)
+    TeamHold hold(team_room_of(ctx->device));
+    int team = teams ? team_workgroups(ctx) : 0;
+    if (team > 1 && !S.done && !hold.take(team, team_room(ctx->n_cu))) team = 0;
     if (!S.done) ctx->last_team[0] = team;
     if (team > 1 && !S.done && !coord)   // the start, should the team give up
         HIPCHK(hipMemcpyAsync(ctx->ext.p, ctx->x[0].p, sizeof(double) * nv, hipMemcpyDeviceToDevice, ctx->stream));
@@ -2240,6 +2242,7 @@ static int minimize_run(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, dou
         // before the pinned copy is overwritten
         HIPCHK(d2h(ctx, &S, ctx->cg.p, sizeof(CgState)));
     }
+    hold.give();
     ctx->last_cg = S;
     if (!S.done) return fail(ctx, MDN_ERR_STATE, "minimizer did not terminate within %ld batches", launched);
     ctx->cur = S.parity;
@@ -2333,18 +2336,11 @@ static hipError_t batch_copy(mdn_ctx* L, std::vector<HostCopy>& parts, double* h
 
 // The persistent kernel of a planned batch.
 static int launch_batch(mdn_ctx* L, const TeamPlan& P, int prec) {
-    const BatchItem* items = L->batch_items.p;
-    const TeamSlot* slot = L->batch_slot.p;
-    const TeamInfo* team = L->batch_team.p;
-    TeamCtl* ctl = L->batch_ctl.p;
-    const int* order = L->batch_order.p;
-    int n = (int)P.order.size(), polls = L->team_polls;
-    int* queue = L->batch_queue.p;
-    void* args[] = {&items, &slot, &team, &ctl, &order, &n, &queue, &polls};
     const dim3 g(P.slot.size()), b(TEAM_NT);
     auto launch = [&](auto k) {
-        if (P.teamed > 0) return hipLaunchCooperativeKernel(k, g, b, args, 0, L->stream);
-        hipLaunchKernelGGL(k, g, b, 0, L->stream, items, slot, team, ctl, order, n, queue, polls);
+        hipLaunchKernelGGL(k, g, b, 0, L->stream, (const BatchItem*)L->batch_items.p, (const TeamSlot*)L->batch_slot.p,
+                           (const TeamInfo*)L->batch_team.p, L->batch_ctl.p, (const int*)L->batch_order.p, (int)P.order.size(),
+                           L->batch_queue.p, L->team_polls);
         return hipGetLastError();
     };
     if (prec == MDN_PREC_MIXED) HIPCHK_CTX(L, launch(k_cg_team<float, TEAM_NT>));
@@ -2411,7 +2407,11 @@ static int batched_run(mdn_ctx* L, mdn_ctx* const* ctxs, int n, const mdn_cg_par
     int groups = std::max(1, L->n_cu);
     if (const char* env = getenv("MDN_BATCH_MAX_WORKGROUPS"))
         if (atoi(env) > 0) groups = std::min(groups, atoi(env));
-    const TeamPlan plan = plan_teams(cost, groups, teams ? TEAM_MAX : 1);
+    // a batch's teams may fill every XCD: they need the whole room for teams (taken: single workgroups)
+    TeamHold hold(team_room_of(L->device));
+    TeamPlan plan = plan_teams(cost, groups, teams ? TEAM_MAX : 1);
+    const int room = team_room(L->n_cu);
+    if (plan.teamed > 0 && !hold.take(room, room)) plan = plan_teams(cost, groups, 1);
     for (const TeamInfo& t : plan.team)
         if (t.size > 1 && start[t.sys])
             copies.push_back(BatchCopy{start[t.sys], ctxs[t.sys]->ext.p, 3L * ctxs[t.sys]->n_beads});
@@ -2486,6 +2486,7 @@ static int batched_run(mdn_ctx* L, mdn_ctx* const* ctxs, int n, const mdn_cg_par
                               {(char*)ctl.data(), (char*)L->batch_ctl.p, sizeof(TeamCtl) * ctl.size()},
                               {(char*)reports.data(), (char*)L->batch_reports.p, sizeof(double) * 27 * n}};
     HIPCHK_CTX(L, copy_parts(L, head, 3, true));
+    hold.give();
     std::vector<char> failed(n, 0);
     for (size_t t = 0; t < plan.team.size(); t++) {
         const int i = plan.team[t].sys;

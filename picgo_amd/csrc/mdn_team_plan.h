@@ -1,9 +1,20 @@
 // mdn_team_plan.h -- the host side of the persistent minimizer's teams (mdn_team.h): how many
-// workgroups a network gets and how a batch's workgroups are shared out. No HIP.
+// workgroups a network gets, how a batch's workgroups are shared out, and how many workgroups that
+// wait for each other may be in flight on a device. No HIP: also compiled into a CPU check.
+//
+// Workgroups of a team wait for each other, and each of them fills a CU, so a team only gets on once
+// all of it is resident. A cooperative launch guarantees that, but it goes through a queue of its own:
+// teams of several contexts then run one after the other, and once that queue exists everything else
+// that a process runs on four streams is slowed down (7,500 beads by four threads, no team among
+// them: 1,270 us per minimization without the queue, 3,660 with it; 550 beads by teams: 1,195).
+// Teams are therefore launched like any other kernel, and TeamRoom keeps those in flight to what
+// fits: whoever finds no room left takes the form that waits for nobody (the four-kernel slots, a
+// batch of single workgroups), with the same result.
 #pragma once
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 namespace mdn {
@@ -17,6 +28,45 @@ struct TeamInfo {
 };
 struct TeamSlot {   // per workgroup: its team (< 0: none) and its place in it
     int team, member;
+};
+
+// Workgroups of teams that are resident together for certain: those of one XCD. Which XCD a launch's
+// first workgroup runs on depends on its hardware queue, so any two teams may meet on the same one.
+// A partition holds whole XCDs; a device that shows fewer CUs than one has the CUs it shows.
+inline int team_room(int n_cu) { return std::max(1, std::min(TEAM_MAX, n_cu)); }
+
+// The workgroups of teams in flight on one device.
+struct TeamRoom {
+    std::mutex mu;
+    int used = 0;
+    bool take(int n, int room) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (n > room - used) return false;
+        used += n;
+        return true;
+    }
+    void give(int n) {
+        std::lock_guard<std::mutex> lk(mu);
+        used -= n;
+    }
+};
+// A call's share of a room (null: none), given back by give() or at the end of the scope.
+struct TeamHold {
+    TeamRoom* room;
+    int n = 0;
+    explicit TeamHold(TeamRoom* r) : room(r) {}
+    TeamHold(const TeamHold&) = delete;
+    TeamHold& operator=(const TeamHold&) = delete;
+    ~TeamHold() { give(); }
+    bool take(int k, int size) {
+        if (!room || !room->take(k, size)) return false;
+        n = k;
+        return true;
+    }
+    void give() {
+        if (n) room->give(n);
+        n = 0;
+    }
 };
 
 // Work per workgroup below which another workgroup does not pay: batches of 8, 16 and 48 networks
@@ -37,9 +87,10 @@ constexpr long TEAM_SHARE = 256;
 // TEAM_ONE_MAX and a work of about 21,000, and 3 % from 32 workgroups at 13,900.
 constexpr long TEAM_ONE_SHARE = 160, TEAM_WIDE = 9000, TEAM_ONE_MAX = 17500;
 // Workgroups of the persistent minimizer for a single network; 0: the four-kernel slots.
-inline int team_size_one(long work) {
+inline int team_size_one(long work, int room) {
     if (work > TEAM_ONE_MAX) return 0;
-    return work > TEAM_WIDE ? 24 : (int)std::min<long>(16, (work + TEAM_ONE_SHARE - 1) / TEAM_ONE_SHARE);
+    const long k = work > TEAM_WIDE ? 24 : std::min<long>(16, (work + TEAM_ONE_SHARE - 1) / TEAM_ONE_SHARE);
+    return (int)std::min<long>(k, room);
 }
 
 // A batch's workgroups: which team each is in, and which system each team has. Large systems get
