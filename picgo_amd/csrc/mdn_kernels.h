@@ -1999,8 +1999,9 @@ __device__ inline bool nl_keep_at(const NLDev& n, const NlRec& c, const NlRec& c
 // A halo with more than NL_CAP members is read from global memory instead (the same 27 bins). The
 // bins are wider than the range, so the pair set is the predicate's whatever the bin size.
 // PASS 0: count per cylinder, the largest count, and the first NL_HITS neighbours into
-// found[NL_HITS c ...] (in order if there are no more): k_nl_emit then copies them into the list.
-// PASS 1, if a cylinder has more: emit into [off[c], off[c + 1]), sorted there.
+// found[NL_HITS c ...] (in order, if there are no more): k_nl_emit then copies them into the list.
+// PASS 1, if a cylinder has more: every neighbour into list[off[c] .. off[c + 1]), in any order, and c
+// into the pairs; k_nl_place then orders them.
 // Latency bound. With one lane per cylinder (36 of 256 lanes busy at 42,000 beads), the predicate's
 // records read from global memory and a second search that sorted in global memory, count and
 // emission took 105 us there, 205 us at 420,000 and 308 us for a binder's wider list at 42,000;
@@ -2015,7 +2016,8 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
                                                    const NlRec* __restrict__ members, const int* __restrict__ mbin,
                                                    const double* __restrict__ mmid, int* __restrict__ count,
                                                    int* __restrict__ most, int* __restrict__ found,
-                                                   const int* __restrict__ off, int* __restrict__ pairs) {
+                                                   const int* __restrict__ off, int* __restrict__ list,
+                                                   int* __restrict__ pairs) {
     __shared__ int s_ah[NL_GROUPS * NL_HITS > NL_HMAX ? NL_GROUPS * NL_HITS : NL_HMAX];
     __shared__ int s_start[NL_HMAX + 1], s_part[BLOCK / 64], s_cnt[NL_GROUPS];
     __shared__ NlRec s_rec[NL_CAP];
@@ -2108,8 +2110,12 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
             const int lx = (loc & (T - 1)) + 1, ly = ((loc >> lt) & (T - 1)) + 1, lz = (loc >> (2 * lt)) + 1;   // halo coords
             auto hit = [&](int cn) {
                 const int k = atomicAdd(&s_cnt[grp], 1);
-                if (k < NL_HITS) s_hit[k] = cn;
-                else if (PASS) pairs[2 * (base + k) + 1] = cn;
+                if (PASS) {
+                    list[base + k] = cn;
+                    pairs[2 * (base + k)] = c.c;
+                } else if (k < NL_HITS) {
+                    s_hit[k] = cn;
+                }
             };
             if (staged) {
                 int first[9], before[10];   // the rows' first members in LDS, the candidates before each
@@ -2128,53 +2134,60 @@ __global__ void __launch_bounds__(BLOCK) k_nl_tile(NLDev n, const int* __restric
                     if (nl_keep_at(n, c, cn, mc, &s_mid[3 * k])) hit(cn.c);
                 }
             } else {
-                for (int r = lane; r < 9; r += NL_LANES)
-                    for (int dx = -1; dx <= 1; dx++) {
-                        const int X = hx0 + lx + dx, Y = hy0 + ly + r % 3 - 1, Z = hz0 + lz + r / 3 - 1;
-                        if (X < 0 || Y < 0 || Z < 0 || X >= n.nb[0] || Y >= n.nb[1] || Z >= n.nb[2]) continue;
-                        const int nbin = nl_bin_id(n, X, Y, Z);
-                        const int m1 = bin_start[nbin + 1];
-                        for (int m = bin_start[nbin]; m < m1; m++)
-                            if (nl_keep_at(n, c, members[m], mc, &mmid[3 * (long)m])) hit(members[m].c);
+                int a[4], z[4];   // the member ranges of the 27 bins, four per lane, in flight together
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int b = NL_LANES * j + lane;
+                    const int X = hx0 + lx + b % 3 - 1, Y = hy0 + ly + b / 3 % 3 - 1, Z = hz0 + lz + b / 9 - 1;
+                    a[j] = z[j] = 0;
+                    if (b < 27 && X >= 0 && Y >= 0 && Z >= 0 && X < n.nb[0] && Y < n.nb[1] && Z < n.nb[2]) {
+                        const int g = nl_bin_id(n, X, Y, Z);
+                        a[j] = bin_start[g];
+                        z[j] = bin_start[g + 1];
                     }
+                }
+#pragma unroll
+                for (int b = 0; b < 27; b++) {
+                    const int m1 = __shfl(z[b / NL_LANES], b % NL_LANES, NL_LANES);
+                    for (int m = __shfl(a[b / NL_LANES], b % NL_LANES, NL_LANES) + lane; m < m1; m += NL_LANES) {
+                        const NlRec cn = members[m];
+                        if (nl_keep_at(n, c, cn, mc, &mmid[3 * (long)m])) hit(cn.c);
+                    }
+                }
             }
         }
         __syncthreads();
         // 3. in ascending order
-        const int cnt = mine ? s_cnt[grp] : 0;
-        const bool small = cnt <= NL_HITS;
-        for (int a = lane; a < min(cnt, NL_HITS); a += NL_LANES) {
-            const int v = s_hit[a];
-            int to = a;
-            if (small) {
-                to = 0;
-                for (int b = 0; b < cnt; b++) to += s_hit[b] < v;
-            }
-            if (PASS) {
-                pairs[2 * (base + to)] = c.c;
-                pairs[2 * (base + to) + 1] = v;
-            } else {
-                found[(long)NL_HITS * c.c + to] = v;
-            }
-        }
-        if (!PASS && mine && lane == 0) {
-            count[c.c] = cnt;
-            if (!small) atomicMax(most, cnt);
-        }
-        if (PASS && __syncthreads_or(!small) && !small && lane == 0) {
-            for (int a = 1; a < cnt; a++) {   // insertion sort in global memory
-                const int v = pairs[2 * (base + a) + 1];
-                int j = a - 1;
-                while (j >= 0 && pairs[2 * (base + j) + 1] > v) {
-                    pairs[2 * (base + j + 1) + 1] = pairs[2 * (base + j) + 1];
-                    j--;
+        if (!PASS && mine) {
+            const int cnt = s_cnt[grp];
+            if (cnt <= NL_HITS) {
+                for (int q = lane; q < cnt; q += NL_LANES) {
+                    const int v = s_hit[q];
+                    int to = 0;
+                    for (int b = 0; b < cnt; b++) to += s_hit[b] < v;
+                    found[(long)NL_HITS * c.c + to] = v;
                 }
-                pairs[2 * (base + j + 1) + 1] = v;
-                pairs[2 * (base + a)] = c.c;
+            }
+            if (lane == 0) {
+                count[c.c] = cnt;
+                if (cnt > NL_HITS) atomicMax(most, cnt);
             }
         }
         __syncthreads();   // the group's counter and list are used again
     }
+}
+
+// the neighbours of k_nl_tile<1> into the pairs, ascending, by rank: a thread per entry, whose reads of
+// its cylinder's other entries its neighbours in the wavefront share. An insertion sort in global memory
+// by one lane in eight took 1,170 ms of a binder's list with up to 1,000 neighbours (7,800 beads), by one
+// lane per cylinder 270 ms.
+__global__ void k_nl_place(long n_pairs, const int* __restrict__ off, const int* __restrict__ list, int* __restrict__ pairs) {
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n_pairs) return;
+    const int c = pairs[2 * e], lo = off[c], hi = off[c + 1], v = list[e];
+    int to = lo;
+    for (int q = lo; q < hi; q++) to += list[q] < v;
+    pairs[2 * (long)to + 1] = v;
 }
 
 // the pairs of every cylinder from the neighbours that k_nl_tile<0> found (none has more than NL_HITS)

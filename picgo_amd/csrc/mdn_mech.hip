@@ -129,7 +129,7 @@ struct mdn_ctx {
     DBuf<double> d_cyl_kexvol, d_cyl_eql, d_krep_e, d_slen_e;
     // NL workspace
     DBuf<double> mid;
-    DBuf<int> bin, bin_count, bin_start, place, nl_found, nl_count, nl_off, pairs, bnd_cnt, bnd_off;
+    DBuf<int> bin, bin_count, bin_start, place, nl_found, nl_list, nl_count, nl_off, pairs, bnd_cnt, bnd_off;
     // the binding-site search's own list (mdn_binding_pairs) and its per-pair counts
     DBuf<double> b_mid, mmid, b_mmid;
     DBuf<NlRec> members, b_members;
@@ -815,7 +815,7 @@ int mdn_ctx_destroy(mdn_ctx* ctx) {
                        &ctx->inc_s_start, &ctx->inc_s, &ctx->inc_cnt, &ctx->inc_list,
                        &ctx->d_cyl_b1, &ctx->d_cyl_b2, &ctx->d_cyl_fil, &ctx->d_cyl_pos,
                        &ctx->d_cyl_type, &ctx->bin, &ctx->bin_count, &ctx->bin_start, &ctx->place,
-                       &ctx->nl_found, &ctx->nl_count, &ctx->nl_off, &ctx->pairs, &ctx->bnd_cnt, &ctx->bnd_off,
+                       &ctx->nl_found, &ctx->nl_list, &ctx->nl_count, &ctx->nl_off, &ctx->pairs, &ctx->bnd_cnt, &ctx->bnd_off,
                        &ctx->bad_count, &ctx->bad_list, &ctx->fallback_ok, &ctx->bstart,
                        &ctx->sorted_id, &ctx->pos, &ctx->dof_src, &ctx->b_bin, &ctx->b_bin_count,
                        &ctx->b_bin_start, &ctx->b_place, &ctx->b_count, &ctx->b_off,
@@ -1339,7 +1339,7 @@ static int count_pairs(mdn_ctx* ctx, const NLDev& n, const double* x, NlBufs& B)
                        (const int*)B.place.p, (const double*)B.mid.p, B.members.p, B.mbin.p, B.mmid.p);
     hipLaunchKernelGGL(k_nl_tile<0>, dim3(nl_tile_count(n)), dim3(BLOCK), 0, ctx->stream, n, (const int*)B.bin_start.p,
                        (const NlRec*)B.members.p, (const int*)B.mbin.p, (const double*)B.mmid.p, B.count.p, flags + 1,
-                       ctx->nl_found.p, (const int*)nullptr, (int*)nullptr);
+                       ctx->nl_found.p, (const int*)nullptr, (int*)nullptr, (int*)nullptr);
     HIPCHK(hipGetLastError());
     return exclusive_scan(ctx, B.count.p, B.off.p, nc + 1);
 }
@@ -1363,11 +1363,15 @@ static int emit_pairs(mdn_ctx* ctx, const NLDev& n, NlBufs& B, int ne, const int
     if (ctx->h_int[2] == 0)
         hipLaunchKernelGGL(k_nl_emit, dim3(std::max(1, ceil_div(nc, BLOCK))), dim3(BLOCK), 0, ctx->stream, nc,
                            (const int*)B.off.p, (const int*)ctx->nl_found.p, (int2*)B.pairs.p);
-    else
+    else {
+        HIPCHK(ctx->nl_list.ensure((size_t)*np));
         hipLaunchKernelGGL(k_nl_tile<1>, dim3(nl_tile_count(n)), dim3(BLOCK), 0, ctx->stream, n,
                            (const int*)B.bin_start.p, (const NlRec*)B.members.p, (const int*)B.mbin.p,
                            (const double*)B.mmid.p, B.count.p, flags + 1, ctx->nl_found.p, (const int*)B.off.p,
-                           B.pairs.p);
+                           ctx->nl_list.p, B.pairs.p);
+        hipLaunchKernelGGL(k_nl_place, dim3(ceil_div(*np, BLOCK)), dim3(BLOCK), 0, ctx->stream, *np, (const int*)B.off.p,
+                           (const int*)ctx->nl_list.p, B.pairs.p);
+    }
     HIPCHK(hipGetLastError());
     return MDN_OK;
 }
