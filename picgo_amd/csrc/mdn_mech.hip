@@ -1986,8 +1986,14 @@ extern "C++" {
 // FP64 excluded-volume force blocks of their own pay while the chip is not full without them (80
 // iterations without the rebuild, one thread per pair -> two: 14,700 beads in a cube 2.22 -> 2.07 ms,
 // 42,000 2.53 -> 2.48, 84,000 3.04 -> 3.02, 126,000 3.31 -> 3.42; in a sphere 42,000 2.26 -> 2.08,
-// 84,000 2.47 -> 2.42, 126,000 2.62 -> 2.69, 420,000 4.84 -> 4.93).
-static const int EV_SPLIT_BEADS = 100000;
+// 84,000 2.47 -> 2.42, 126,000 2.62 -> 2.69, 420,000 4.84 -> 4.93). Denser networks fill it with fewer
+// beads (40 iterations): 42,000 beads with 153,000 pairs 2.76 -> 2.73, 228,000 2.54 -> 2.56, 507,000
+// 5.61 -> 5.73; 94,500 with 186,000 2.75 -> 2.77, 366,000 4.05 -> 4.12; 21,000 with 127,000 3.10 -> 3.07,
+// 287,000 5.16 -> 5.13.
+static const long EV_SPLIT_BEADS = 100000, EV_SPLIT_WORK = 140000;
+static bool ev_split(const DevSys& s) {
+    return s.n_beads < EV_SPLIT_BEADS && s.n_beads + s.n[FF_EXVOL] / 2L < EV_SPLIT_WORK;
+}
 template <typename R>
 static void launch_slot(mdn_ctx* ctx, const DevSys& s, const CgBufs& B) {
     const int gbk = gather_blocks(ctx);
@@ -1996,7 +2002,7 @@ static void launch_slot(mdn_ctx* ctx, const DevSys& s, const CgBufs& B) {
     // with bead_energy the filament terms' blocks are left out
     const int lsg = s.bonded_gather ? (s.bead_energy ? s.blk_nb : s.blk[NFF]) + s.nbb : s.blk[NFF];
     bool split = false;
-    if constexpr (sizeof(R) == 8) split = s.n_beads < EV_SPLIT_BEADS;
+    if constexpr (sizeof(R) == 8) split = ev_split(s);
     if constexpr (sizeof(R) == 8)
         if (split)
             hipLaunchKernelGGL((k_cg_ls<R, true>), dim3(std::max(1, ev_force_blocks<R, true>(s) + lsg)), dim3(BLOCK), 0,
