@@ -2421,7 +2421,7 @@ static int batched_run(mdn_ctx* L, mdn_ctx* const* ctxs, int n, const mdn_cg_par
     TeamHold hold(team_room_of(L->device));
     TeamPlan plan = plan_teams(cost, groups, teams ? TEAM_MAX : 1);
     const int room = team_room(L->n_cu);
-    if (plan.teamed > 0 && !hold.take(room, room)) plan = plan_teams(cost, groups, 1);
+    if (plan.teamed > 0 && !hold.take(room, room, TEAM_ROOM_WAIT)) plan = plan_teams(cost, groups, 1);
     for (const TeamInfo& t : plan.team)
         if (t.size > 1 && start[t.sys])
             copies.push_back(BatchCopy{start[t.sys], ctxs[t.sys]->ext.p, 3L * ctxs[t.sys]->n_beads});

@@ -62,7 +62,7 @@ int main() {
             for (int i = 0; i < 20000; i++) {
                 const int want = 1 + (k * 7 + i) % 32;
                 TeamHold h(&room);
-                if (!h.take(want, 32)) continue;
+                if (!h.take(want, 32, std::chrono::microseconds(k < 2 ? 2000 : 0))) continue;
                 got++;
                 const int in = now += want;
                 int m = most;
@@ -77,6 +77,23 @@ int main() {
     EXPECT(!none.take(1, 32) && all.take(32, 32) && !late.take(1, 32));
     all.give();
     EXPECT(late.take(1, 32) && room.used == 1);
+    // whoever waits gets the room when it is given back, and not before; others don't pass it
+    late.give();
+    EXPECT(all.take(32, 32));
+    const auto t0 = std::chrono::steady_clock::now();
+    EXPECT(!late.take(32, 32, std::chrono::microseconds(3000)));
+    EXPECT(std::chrono::steady_clock::now() - t0 >= std::chrono::microseconds(3000) && room.waiting == 0);
+    std::thread w([&] { TeamHold h(&room); EXPECT(h.take(32, 32, std::chrono::seconds(20))); });
+    for (bool seen = false; !seen;) {
+        std::lock_guard<std::mutex> lk(room.mu);
+        seen = room.waiting == 1;
+    }
+    all.n = 31;
+    all.give();
+    EXPECT(!late.take(1, 32));
+    room.give(1);
+    w.join();
+    EXPECT(room.used == 0 && late.take(1, 32));
     std::printf("%d wrong\n", bad);
     return bad != 0;
 }
