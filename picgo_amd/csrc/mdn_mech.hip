@@ -336,8 +336,12 @@ struct HostCopy { char* host; char* dev; size_t bytes; };
 hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host) {
     size_t total = 0;
     for (int i = 0; i < np; i++) total += parts[i].bytes;
-    char* r = total ? stage_acquire(ctx->device) : nullptr;
-    hipError_t e = hipSuccess;
+    // the ring's kernels and events belong to the calling thread's current device: on another one than
+    // the context's (entry points that only read leave it as it is) the runtime copies
+    int current = -1;
+    hipError_t e = hipGetDevice(&current);
+    char* r = total && e == hipSuccess && current == ctx->device ? stage_acquire(ctx->device) : nullptr;
+    e = hipSuccess;
     if (!r) {
         for (int i = 0; i < np && e == hipSuccess; i++)
             e = to_host ? hipMemcpyAsync(parts[i].host, parts[i].dev, parts[i].bytes, hipMemcpyDeviceToHost, ctx->stream)
