@@ -1,6 +1,7 @@
 """GPU: results to the host where the way they are copied changes, bit for bit: just below and above
-16 KB, 96 KB and 2 MB, into memory that is mapped and into fresh pages, aligned to pages and not; and
-parameters uploaded one after another from buffers that are overwritten as soon as the call returns."""
+16 KB, 96 KB, 256 KB, 768 KB and 2 MB, from an idle stream and behind queued kernels, into memory that
+is mapped and into fresh pages, aligned to pages and not; and parameters uploaded one after another
+from buffers that are overwritten as soon as the call returns."""
 import ctypes
 import mmap
 
@@ -12,10 +13,10 @@ from picgo_amd import autograd, mech, synth
 pytestmark = pytest.mark.gpu
 
 
-def _ctx(fil, cyl):
+def _ctx(fil, cyl, wide=1.0):
     p = synth.preset(1)
     p.n_fil, p.n_cyl_min, p.n_cyl_max, p.seed = fil, cyl, cyl, 7
-    p.box = max(3000.0, 1000.0 * (fil * cyl / 95.0) ** (1 / 3))
+    p.box = wide * max(3000.0, 1000.0 * (fil * cyl / 95.0) ** (1 / 3))
     p.n_linkers = p.n_motors = 0
     net = synth.Network(p)
     g = mech.ForceFieldManager(0)
@@ -29,7 +30,31 @@ def _get(g, a):
     return a
 
 
-@pytest.mark.parametrize("fil", [32, 33, 195, 196, 4161, 4162])   # 21 beads, 504 bytes, each
+SIZES = [32, 33, 195, 196, 520, 521, 1560, 1561, 4161, 4162]   # filaments of 21 beads, 504 bytes, each
+
+
+@pytest.mark.parametrize("fil", SIZES)
+def test_product_into_mapped_and_fresh_pages(fil):
+    """Behind the product's kernels: H v, the same whatever memory receives it (in a wide box: a pair of
+    crossing filaments may have no tangent)."""
+    net, g = _ctx(fil, 20, 10.0)
+    x = net.coord + np.random.default_rng(fil).normal(0.0, 1.0, net.coord.size)
+    v = np.random.default_rng(1).normal(size=x.size)
+    g.reset_neighbor_lists(x)
+    p = [a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in (x, v)]
+    want = None
+    for at in (None, None, 0, 8):
+        if at is None:
+            a = np.full(x.size, 7.0)
+        else:
+            m = mmap.mmap(-1, x.nbytes + 8192)
+            a = np.frombuffer(m, np.float64, x.size, at)
+        assert mech.lib().mdn_hvp(g._h, *p, a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), x.size) == 0
+        want = a.copy() if want is None else want
+        assert want.any() and np.array_equal(a, want)
+
+
+@pytest.mark.parametrize("fil", SIZES)
 def test_result_into_mapped_and_fresh_pages(fil):
     net, g = _ctx(fil, 20)
     x = np.random.default_rng(fil).normal(500.0, 100.0, net.coord.size)
