@@ -225,29 +225,32 @@ hipError_t d2h(mdn_ctx* ctx, void* dst, const void* src, size_t bytes) {
 }
 
 // ---- host copies through pinned memory ------------------------------------------------------
-// Results go through a pinned ring where that is the faster way: a kernel moves the pieces between
+// Copies go through a pinned ring where that is the faster way: a kernel moves the pieces between
 // device and ring (k_copy_pieces), the CPU between ring and caller, chunk by chunk side by side, and
-// pages that the caller has not touched yet are mapped in one call per chunk ahead of the copy. The
-// runtime's copy and the ring, us:
-//     behind queued kernels    7 KB 52, 42;  18 KB 57, 51;  76 KB 64, 58;  94 KB 67, 62;  211 KB 78, 72;
-//       (mdn_hvp, whole call)  into fresh pages 76 KB 76, 66;  211 KB 114, 95;  with more than one chunk
-//                              it depends: 374 KB 100, 119;  456 KB 108, 127 (103, 98 if the program does
-//                              not wait for the device between the calls)
-//     idle stream,             16 KB 21, 13;  17 KB 9, 13;  64 KB 11, 15;  256 KB 19, 23;
-//       touched pages          1 MB 62, 78;  2 MB 122, 129;  3 MB 182, 135;  8 MB 485, 385
-//     idle stream, fresh       16 KB 23, 16;  24 KB 14, 18;  64 KB 22, 22;  96 KB 29, 26;
-//       pages                  256 KB 63, 49;  768 KB 170, 121;  1 MB 280, 180;  8 MB 2240, 1490
-//     input                    16 KB 13, 14;  64 KB 11, 15;  256 KB 16, 21;  1 MB 55, 78;  8 MB 250, 280
-// So results of one chunk take the ring behind queued kernels, from an idle stream up to STAGE_TINY and
-// from STAGE_FRESH on into fresh pages; larger ones beyond STAGE_LARGE, and from STAGE_FRESH_LARGE on
-// into fresh pages. Inputs never do: the runtime queues them, while each one through the ring is a wait
-// (four parameter uploads of 144 KB: 61 us, through the ring 111). A batch's many tables and
-// coordinates take the ring together in both directions.
+// pages of a result that the caller has not touched yet are mapped in one call per chunk ahead of the
+// copy. The runtime's copy of more than 16 KB is a copy engine's: fast when the same stream used that
+// engine last, 17 to 35 us more when a program goes through more than some 8 contexts, and a wait for
+// the kernels queued before it. The ring's costs are the same always. Runtime and ring, us:
+//     result, idle stream         13 KB 23, 14;  94 KB 13, 17;  256 KB 20, 23;  1 MB 62, 78;
+//                                 2 MB 122, 129;  3 MB 182, 135;  8 MB 485, 385
+//       one of 32 contexts        91 KB 51, 19
+//       into fresh pages          24 KB 14, 18;  96 KB 29, 26;  256 KB 63, 49;  768 KB 170, 121;
+//                                 1 MB 280, 180;  8 MB 2240, 1490
+//     result behind kernels       7 KB 52, 42;  18 KB 57, 51;  76 KB 64, 58;  211 KB 78, 72;  with more
+//       (mdn_hvp, whole call)     than one chunk it depends: 374 KB 100, 119;  456 KB 108, 127
+//     input                       16 KB 13, 14;  64 KB 11, 15;  256 KB 16, 21;  1 MB 55, 78;  8 MB 250, 280
+//       of mdn_forces             91 KB 53, 58;  one of 32 contexts 87, 59
+//       of mdn_minimize           91 KB 832, 839;  96 contexts in turn 566, 533
+//       four 144 KB parameters    61, 111
+// So results of one chunk take the ring, larger ones beyond STAGE_LARGE and from STAGE_FRESH on into
+// fresh pages. The runtime queues inputs, while each one through the ring is a wait: only a
+// minimization's coordinates take it, for which that is little. A batch's many tables and coordinates
+// take the ring together in both directions.
 // Rings belong to the process, at most STAGE_RINGS per device: a call holds one while it copies
 // and gives it back; a call that finds none free takes the runtime's copy. They are freed with
 // the device's last context.
-constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_TINY = 16u << 10, STAGE_FRESH = 96u << 10;
-constexpr size_t STAGE_ONE = 256u << 10, STAGE_FRESH_LARGE = 768u << 10, STAGE_LARGE = 2u << 20;
+constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MIN = 2048, STAGE_IN_MIN = 32u << 10, STAGE_ONE = 256u << 10;
+constexpr size_t STAGE_FRESH = 768u << 10, STAGE_LARGE = 2u << 20;
 constexpr int STAGE_RINGS = 4;
 struct StagePool {
     std::mutex mu;
@@ -406,16 +409,17 @@ hipError_t copy_parts(mdn_ctx* ctx, const HostCopy* parts, int np, bool to_host)
     return e;
 }
 
-// Host data onto the device, queued.
-hipError_t copy_in(mdn_ctx* ctx, void* dev, const void* host, size_t bytes) {
-    return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+// Host data onto the device: queued, or (ring) complete on return.
+hipError_t copy_in(mdn_ctx* ctx, void* dev, const void* host, size_t bytes, bool ring = false) {
+    if (!ring || bytes < STAGE_IN_MIN || bytes > STAGE_ONE || !pageable(host))
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+    const HostCopy c{const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes};
+    return copy_parts(ctx, &c, 1, false);
 }
-// Device data to the host after everything queued on the stream; complete on return. idle: the caller
-// has waited for the stream.
-hipError_t copy_out(mdn_ctx* ctx, void* host, const void* dev, size_t bytes, bool idle) {
-    const bool ring = bytes <= STAGE_ONE ? bytes >= STAGE_MIN && (!idle || bytes <= STAGE_TINY ||
-                                                                  (bytes >= STAGE_FRESH && fresh_pages(host, bytes)))
-                                         : bytes > STAGE_LARGE || (bytes >= STAGE_FRESH_LARGE && fresh_pages(host, bytes));
+// Device data to the host after everything queued on the stream; complete on return.
+hipError_t copy_out(mdn_ctx* ctx, void* host, const void* dev, size_t bytes) {
+    const bool ring = bytes <= STAGE_ONE ? bytes >= STAGE_MIN
+                                         : bytes > STAGE_LARGE || (bytes >= STAGE_FRESH && fresh_pages(host, bytes));
     if (!ring || !pageable(host)) return d2h(ctx, host, dev, bytes);
     const HostCopy c{static_cast<char*>(host), const_cast<char*>(static_cast<const char*>(dev)), bytes};
     return copy_parts(ctx, &c, 1, true);
@@ -1271,7 +1275,7 @@ int mdn_perturb(mdn_ctx* ctx, uint64_t seed, uint64_t stream, double sigma) {
 int mdn_get_coords(mdn_ctx* ctx, double* coord) {
     int st = need_system(ctx, false);
     if (st) return st;
-    HIPCHK(copy_out(ctx, coord, ctx->x[ctx->cur].p, sizeof(double) * 3 * ctx->n_beads, true));
+    HIPCHK(copy_out(ctx, coord, ctx->x[ctx->cur].p, sizeof(double) * 3 * ctx->n_beads));
     return MDN_OK;
 }
 
@@ -1561,7 +1565,7 @@ int mdn_binding_pairs(mdn_ctx* ctx, const mdn_binding_params* p, const double* c
     hipLaunchKernelGGL(k_bind_sites<1>, dim3(G), dim3(BLOCK), 0, ctx->stream, n, b, x, np, (const int*)ctx->b_pairs.p,
                        ctx->b_scount.p, (const int*)ctx->b_soff.p, ctx->b_out.p);
     HIPCHK(hipGetLastError());
-    HIPCHK(copy_out(ctx, out, ctx->b_out.p, sizeof(uint32_t) * 2 * total, false));
+    HIPCHK(copy_out(ctx, out, ctx->b_out.p, sizeof(uint32_t) * 2 * total));
     return MDN_OK;
 }
 
@@ -1571,7 +1575,7 @@ int mdn_nl_pairs(mdn_ctx* ctx, int32_t* out, int64_t cap, int64_t* n_pairs) {
     if (n_pairs) *n_pairs = ctx->n_pairs;
     if (cap < ctx->n_pairs) return fail(ctx, MDN_ERR_CAPACITY, "need room for %ld pairs", ctx->n_pairs);
     if (ctx->n_pairs > 0)
-        HIPCHK(copy_out(ctx, out, ctx->pairs.p, sizeof(int) * 2 * ctx->n_pairs, true));
+        HIPCHK(copy_out(ctx, out, ctx->pairs.p, sizeof(int) * 2 * ctx->n_pairs));
     return MDN_OK;
 }
 
@@ -1582,7 +1586,7 @@ int mdn_boundary_list(mdn_ctx* ctx, int32_t* out_beads, int64_t cap, int32_t* ou
     if (n_interactions) *n_interactions = ctx->n_bint;
     if (cap < ctx->n_bint) return fail(ctx, MDN_ERR_CAPACITY, "need room for %d interactions", ctx->n_bint);
     if (ctx->n_bint > 0 && out_beads)
-        HIPCHK(copy_out(ctx, out_beads, ctx->bnd_b.p, sizeof(int) * ctx->n_bint, true));
+        HIPCHK(copy_out(ctx, out_beads, ctx->bnd_b.p, sizeof(int) * ctx->n_bint));
     if (out_nneighbors)
         for (size_t e = 0; e < ctx->bnd_nneighbors.size(); e++) out_nneighbors[e] = ctx->bnd_nneighbors[e];
     return MDN_OK;
@@ -1635,7 +1639,7 @@ static int forces_impl(mdn_ctx* ctx, int ff, const double* coord, double* force,
     HIPCHK(hipStreamSynchronize(ctx->stream));
     bool redone;
     if ((st = ev.finish(&redone))) return st;
-    HIPCHK(copy_out(ctx, force, ctx->f.p, sizeof(double) * n_var, true));
+    HIPCHK(copy_out(ctx, force, ctx->f.p, sizeof(double) * n_var));
     return MDN_OK;
 }
 
@@ -1725,7 +1729,7 @@ static int param_grad_impl(mdn_ctx* ctx, const double* coord, double* out, int64
     HIPCHK(ctx->ev_U.ensure(std::max(1, ctx->sys.n[FF_EXVOL])));
     HIPCHK(ctx->grad_out.ensure(3 * (size_t)std::max(1, ctx->n_cyl)));
     if ((st = param_grad_launch(ctx, x, prec, true))) return st;
-    HIPCHK(copy_out(ctx, out, ctx->grad_out.p, sizeof(double) * 3 * ctx->n_cyl, false));
+    HIPCHK(copy_out(ctx, out, ctx->grad_out.p, sizeof(double) * 3 * ctx->n_cyl));
     return MDN_OK;
 }
 
@@ -1794,7 +1798,7 @@ static int hvp_impl(mdn_ctx* ctx, const double* coord, const double* v, double* 
     HIPCHK(ctx->tan_v.ensure(n_var));
     HIPCHK(copy_in(ctx, ctx->tan_v.p, v, sizeof(double) * n_var));
     if ((st = hvp_launch(ctx, x, prec))) return st;
-    HIPCHK(copy_out(ctx, out, ctx->scratch_f.p, sizeof(double) * n_var, false));
+    HIPCHK(copy_out(ctx, out, ctx->scratch_f.p, sizeof(double) * n_var));
     if (ctx->h_int[0] != 0)
         return fail(ctx, MDN_ERR_UNSUPPORTED, "%d excluded-volume pairs need the numerical force fallback (no tangent)",
                     ctx->h_int[0]);
@@ -1840,7 +1844,7 @@ int mdn_hvp_batch(mdn_ctx* ctx, int32_t precision, const double* coord, const do
         HIPCHK(hipGetLastError());
         gather_tangents(ctx, nv, ctx->hb_slots.p, slot_stride, ctx->hb_piece.p, piece_stride, ctx->hb_out.p);
         HIPCHK(hipGetLastError());
-        HIPCHK(copy_out(ctx, out + (size_t)k0 * n_var, ctx->hb_out.p, sizeof(double) * nv * n_var, false));
+        HIPCHK(copy_out(ctx, out + (size_t)k0 * n_var, ctx->hb_out.p, sizeof(double) * nv * n_var));
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->h_int[0] != 0)
@@ -2108,7 +2112,7 @@ static int minimize_run(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, dou
     const int nv = 3 * ctx->n_beads;
     // startMinimization + initial energy / forces (CGMethod.hpp:876-896); the start is in x[0]
     if (coord)
-        HIPCHK(copy_in(ctx, ctx->x[0].p, coord, sizeof(double) * nv));
+        HIPCHK(copy_in(ctx, ctx->x[0].p, coord, sizeof(double) * nv, true));
     else if (ctx->cur != 0)   // the context's device coordinates
         HIPCHK(hipMemcpyAsync(ctx->x[0].p, ctx->x[ctx->cur].p, sizeof(double) * nv, hipMemcpyDeviceToDevice,
                               ctx->stream));
@@ -2295,8 +2299,8 @@ static int minimize_run(mdn_ctx* ctx, const mdn_cg_params* p, double* coord, dou
         fill_report(ctx->h_eout, &res->energies_after);
         res->num_energy_call += 1;
     }
-    if (coord) HIPCHK(copy_out(ctx, coord, xres, sizeof(double) * nv, true));
-    if (force_out) HIPCHK(copy_out(ctx, force_out, (S.fpar ? ctx->f2 : ctx->f).p, sizeof(double) * nv, true));
+    if (coord) HIPCHK(copy_out(ctx, coord, xres, sizeof(double) * nv));
+    if (force_out) HIPCHK(copy_out(ctx, force_out, (S.fpar ? ctx->f2 : ctx->f).p, sizeof(double) * nv));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (S.error_flags & MDN_MIN_ERR_LINESEARCH) return fail(ctx, MDN_ERR_LINESEARCH, "line search failed (recovery disabled)");
     return MDN_OK;

@@ -1,7 +1,7 @@
-"""GPU: results to the host where the way they are copied changes, bit for bit: just below and above
-16 KB, 96 KB, 256 KB, 768 KB and 2 MB, from an idle stream and behind queued kernels, into memory that
-is mapped and into fresh pages, aligned to pages and not; and parameters uploaded one after another
-from buffers that are overwritten as soon as the call returns."""
+"""GPU: results to the host at sizes around those where the way they are copied changes (256 KB, 768 KB
+and 2 MB) and below, bit for bit, from an idle stream and behind queued kernels, into memory that is
+mapped and into fresh pages, aligned to pages and not; and parameters uploaded one after another from
+buffers that are overwritten as soon as the call returns."""
 import ctypes
 import mmap
 
