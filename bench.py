@@ -336,14 +336,14 @@ def batch_256(args):
                                                "over": "networks whose start state holds max|F| < 1 pN"}
     for name, prec in (("fp64", abi.MDN_PREC_FP64), ("mixed", abi.MDN_PREC_MIXED)):
         p = abi.default_cg_params(precision=prec)
-        mech.minimize_batched(ffms, p, coords)   # schedule tuning + warm-up
+        mech.minimize_batched(ffms, p, coords)   # warm-up
         for g, c in zip(ffms, coords):   # the start coordinates resident in HBM before the timed call
             g.set_coords(c)
         t0 = time.perf_counter()
         _, _, res = mech.minimize_batched(ffms, p, None, want_forces=False)
         dt = time.perf_counter() - t0
         nt, srt, _, tune = mech.last_batch_schedule(ffms[0])
-        # the network with the most work (CG iterations x beads) alone, after its own schedule tuning
+        # the network with the most work (CG iterations x beads) alone, after a warm-up
         heavy = int(np.argmax([r.num_iter * n.n_beads for r, n in zip(res, nets)]))
         mech.minimize_batched([ffms[heavy]], p, [coords[heavy]], want_forces=False)
         ffms[heavy].set_coords(coords[heavy])

@@ -1,5 +1,8 @@
 // mdn_team.h -- persistent minimizer: whole minimizations in one kernel launch, each system by a
-// team of 1 to 32 workgroups that share an XCD. Used for small single networks and for batches.
+// team of 1 to 32 workgroups that share an XCD. Used for small single networks and for batches. The
+// launch is an ordinary one; mdn_team_plan.h says which teams may be in flight together, and a team
+// whose workgroups are not resident in time gives up before it has done anything that matters (the
+// host then minimizes from the start again, without a team).
 //
 // A slot of the multi-kernel minimizer is four dependent launches (k_cg_pos, k_cg_ls, k_cg_gather,
 // k_cg_fin), 6 to 7 us of launch and drain around a few us of work on a small network. Here the

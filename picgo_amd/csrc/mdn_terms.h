@@ -437,7 +437,9 @@ MDN_HD inline bool exvol_forces(P c1, P c2in, P c3, P c4, double kRepScaled, O* 
 
 // Energy and forces of one pair: the invariants are shared when the coplanar shift does not
 // apply (the energy never shifts, CylinderExclVolRepulsion.cpp:353-435 vs :610-630).
-// *deferred: the closed-form energy needs the Simpson fallback.
+// *deferred: the closed-form energy needs the Simpson fallback. The kernels evaluate energy and forces
+// by separate calls; the host check measures both forms' rounding with these two combined ones, whose
+// values are the separate calls' (FP64: bit for bit).
 template <typename R>
 MDN_HD inline double exvol_energy_forces(D3 c1, D3 c2, D3 c3, D3 c4, double kRepScaled, int* deferred,
                                              bool* fok, D3* out) {
